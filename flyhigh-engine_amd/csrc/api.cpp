@@ -207,6 +207,12 @@ bool direct_fits(const fhc_conv_desc& d, int idx) {
     return c.ks == (int)d.kh && c.stride == (int)d.stride && (uint32_t)c.cin32 == div_ceil(d.cin, 32) * 32;
 }
 
+// Whether the deep-layer kernel can read this input view by channel pairs (gemm_path_ok; the base pointer's alignment
+// is the launch's to check)
+bool pairs_view(const fhc_conv_desc& d) {
+    return d.x_cstride % 2 == 0 && d.x_c0 % 2 == 0 && d.cin % 2 == 0 && d.cin >= 8;
+}
+
 // The direct kernel's launch geometry for configuration `idx`: input channels padded to 32 in one pass, weights
 // resident; one workgroup per spatial tile (grid x) and channel tile (grid y). False if it does not serve the conv.
 bool configure_direct(fhc_conv_plan& p, int idx, std::string* why) {
@@ -341,8 +347,8 @@ bool configure_igemm(fhc_conv_plan& p, int cfg, uint32_t ks, std::string* why) {
 // The deep-layer kernel's launch geometry for configuration `idx` and global split `ks`: chunks of CK input
 // channels (the packed weights of the chunked layout with cc = CK), one workgroup per spatial tile (grid x), channel
 // tile (grid y) and split (grid z). False if it does not serve the conv: 3x3 of its stride, an input view of
-// 16-byte groups below 2^31 bytes, at least `ks` chunks.
-bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why) {
+// 16-byte groups (with `pairs` also of channel pairs) below 2^31 bytes, at least `ks` chunks.
+bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why, bool pairs = false) {
     const fhc_conv_desc& d = p.d;
     if (idx < 0 || idx >= kNumGemm) {
         *why = "unknown deep-layer configuration";
@@ -353,7 +359,7 @@ bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why) {
         *why = "the deep-layer configuration serves 3x3 convs of stride " + std::to_string(c.s) + " only";
         return false;
     }
-    if (d.x_cstride % 8 || d.x_c0 % 8 || (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 >= (1ull << 31)) {
+    if (((d.x_cstride % 8 || d.x_c0 % 8) && !(pairs && pairs_view(d))) || (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 >= (1ull << 31)) {
         *why = "the deep-layer kernel needs an input view of 16-byte channel groups below 2^31 bytes";
         return false;
     }
@@ -403,7 +409,9 @@ bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why) {
 int heuristic_cfg(const fhc_conv_desc& d, const Geometry& g);
 void* static_scratch(int dev);
 
-bool configure(fhc_conv_plan& p, const Variant& v, std::string* why) {
+// pairs: the deep-layer kernel may read a view of channel pairs (the planner's own choice; a variant that the caller
+// or the table names is held to views of 16-byte groups)
+bool configure(fhc_conv_plan& p, const Variant& v, std::string* why, bool pairs = false) {
     if (v.family == 1) {
         if (v.ks > 1) {
             *why = "the direct kernel has no split-K";
@@ -411,7 +419,7 @@ bool configure(fhc_conv_plan& p, const Variant& v, std::string* why) {
         }
         return configure_direct(p, v.cfg, why);
     }
-    if (v.family == 3) return configure_gemm(p, v.cfg, v.ks, why);
+    if (v.family == 3) return configure_gemm(p, v.cfg, v.ks, why, pairs);
     return configure_igemm(p, v.cfg, v.ks, why);
 }
 
@@ -462,7 +470,14 @@ constexpr int kGemmDefault = 11;
 uint32_t heuristic_code(const fhc_conv_desc& d, const Geometry& g) {
     const bool gemm_ok = d.kh == 3 && d.stride == 1 && d.cin >= 64 && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0 &&
                          (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31);
-    if (gemm_ok && d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096) return make_code(kGemmDefault, 1, 3);
+    const bool big = d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096;
+    if (gemm_ok && big) return make_code(kGemmDefault, 1, 3);
+    // the same layers in a view of channel pairs, unless the caller splits K: 100 -> 100 at 3 x 135 x 241 in a dense
+    // view 76 us (73 in a padded stride) where the direct kernel took 163 with 2-byte loads
+    const bool unsplit = d.ksplit == 0 && (d.ref_cand == 0xFFu || (d.ref_cand >> 4) == 0);
+    if (big && unsplit && d.kh == 3 && d.stride == 1 && pairs_view(d) &&
+        (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31))
+        return make_code(kGemmDefault, 1, 3);
     const int idx = direct_default(d, g);
     if (idx >= 0) return kDirectBase + (uint32_t)idx;
     if (gemm_ok) return make_code(kGemmDefault, 1, 3);
@@ -617,6 +632,7 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
     p.g.cin8 = div_ceil(d.cin, 8) * 8;
     // the choice: forced variant, then the table, then the heuristic (conv_pick, autotune.rs:186-233)
     Variant v{};
+    bool own = false;  // the planner's own choice
     if (d.variant != 0) {
         if (!decode_code(d.variant, &v)) {
             *why = "unknown variant " + std::to_string(d.variant);
@@ -624,7 +640,7 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
         }
     } else {
         const int hit = fhc_tune_get_ex(d.cin, d.cout, d.h, d.w, d.stride, d.n, d.kh);
-        if (hit < 0 || !decode_code((uint32_t)hit, &v)) decode_code(heuristic_code(d, p.g), &v);
+        if (hit < 0 || !decode_code((uint32_t)hit, &v)) own = decode_code(heuristic_code(d, p.g), &v);
     }
     // a forced split (or the reference code's split nibble, candidates.rs:4) moves to the chunked kernel
     uint32_t ks = 0;
@@ -645,7 +661,7 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
             v.ks = ks;
         }
     }
-    if (!configure(p, v, why)) {
+    if (!configure(p, v, why, own)) {
         // a table entry or heuristic that does not fit this shape falls back to the chunked 4-row tile
         const uint32_t code = variant_code(v);
         if (d.variant != 0 || !configure(p, Variant{0, d.cout <= 32 ? 5 : 4, v.family == 1 ? 1u : v.ks}, why)) {

@@ -121,8 +121,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void conv_igemm(ConvKArgs a) {
             uint4 v = {0u, 0u, 0u, 0u};
             if (gy >= 0 && gy < a.h && gx >= 0 && gx < a.w && ch < a.cin) {
                 const uint16_t* p = a.x + ((img_base + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch;
-                if (a.xvec && ch + 8 <= a.cin) {
-                    v = *reinterpret_cast<const uint4*>(p);
+                if (ch + 8 <= a.cin) {  // one 16-byte load at any alignment of the view
+                    const u32x4_a2 q = *reinterpret_cast<const u32x4_a2*>(p);
+                    v = uint4{q.x, q.y, q.z, q.w};
                 } else {
                     uint32_t t[4] = {0u, 0u, 0u, 0u};
 #pragma unroll

@@ -83,15 +83,23 @@ __device__ __forceinline__ uint2 load_res4(const ConvKArgs& a, size_t pix, int c
     return uint2{r[0] | (r[1] << 16), r[2] | (r[3] << 16)};
 }
 
-// 8 consecutive input channels ch..ch+7 of one pixel (p points at channel ch), zeros at and past cin. VEC: the
-// view is 16-byte aligned (cstride, c0 multiples of 8), so a full group is one 16-byte load, and so is a partial
-// group when the view's channel stride holds the whole group (`whole`: c0 + cin rounded up to 8 <= cstride); its
-// channels past cin are then zeroed by the caller (mask_group) where the value is next used. Any other group is 8
-// independent 2-byte loads at clamped in-bounds addresses, selected without branches.
+// 8 consecutive input channels ch..ch+7 of one pixel (p points at channel ch < cin), as one 16-byte load wherever the
+// pixel has 8 channels; settle_group then gives zeros at and past cin, where the value is next used (after the wait
+// for a whole tile's loads). VEC: the view is 16-byte aligned (cstride, c0 multiples of 8), so the stride holds every
+// whole group and a partial group arrives with the channels next to it in the tensor. Other views take the load at
+// its 2-byte alignment (global loads need none), a partial last group as the pixel's last 8 channels. Pixels of
+// fewer than 8 channels: independent 2-byte loads at clamped in-bounds addresses, selected without branches (as a
+// group's 8 loads in every unaligned view, 36 -> 48 at 2 x 200 x 320 took 36.0 us, with the 16-byte loads 29.0 (28.9 in
+// a padded stride); 279 -> 96 at 68 x 120 33.1 -> 24.1)
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 template <bool VEC>
-__device__ __forceinline__ uint4 load_group(const uint16_t* p, int ch, int cin, bool whole = false) {
+__device__ __forceinline__ uint4 load_group(const uint16_t* p, int ch, int cin) {
     const int rem = cin - ch;
-    if (VEC && (rem >= 8 || whole)) return *reinterpret_cast<const uint4*>(p);
+    if constexpr (VEC) return *reinterpret_cast<const uint4*>(p);
+    if (cin >= 8) {
+        const u32x4_a2 q = *reinterpret_cast<const u32x4_a2*>(p - max(0, 8 - rem));
+        return uint4{q.x, q.y, q.z, q.w};
+    }
     uint32_t q[4];
 #pragma unroll
     for (int k = 0; k < 8; k += 2) {
@@ -105,6 +113,23 @@ __device__ __forceinline__ uint4 load_group(const uint16_t* p, int ch, int cin, 
 __device__ __forceinline__ uint4 mask_group(uint4 v, int rem) {
     auto keep = [&](int h) { return (2 * h < rem ? 0xffffu : 0u) | (2 * h + 1 < rem ? 0xffff0000u : 0u); };
     return uint4{v.x & keep(0), v.y & keep(1), v.z & keep(2), v.w & keep(3)};
+}
+
+// the 8 halves moved down by k (0 .. 7) places, zeros behind
+__device__ __forceinline__ uint4 shift_group(uint4 v, int k) {
+    uint64_t lo = (uint64_t)v.y << 32 | v.x, hi = (uint64_t)v.w << 32 | v.z;
+    lo = k & 4 ? hi : lo, hi = k & 4 ? 0 : hi;
+    const int s = (k & 3) * 16;
+    lo = lo >> s | (hi << 1) << (63 - s), hi >>= s;
+    return uint4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
+// load_group's value v with zeros past its rem valid channels (v is zero where rem <= 0: nothing was loaded)
+template <bool VEC>
+__device__ __forceinline__ uint4 settle_group(uint4 v, int rem, int cin) {
+    if constexpr (VEC) return mask_group(v, rem);
+    if (cin >= 8 && (cin & 7)) return shift_group(v, rem >= 8 ? 0 : min(8 - rem, 7));  // uniform
+    return v;
 }
 
 // The MFMA schedule of one tile (WK == 1). The distinct B operands of a wave are the halo rows r = 0 .. R-1 it
@@ -248,7 +273,7 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
         for (int i = 0; i < NLD; i++) {
             const int e = tid + i * NT;
             const int pix = e / GPT, g = e - pix * GPT;
-            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = pre[i];
+            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
         }
     };
 
@@ -590,7 +615,6 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
         for (int s = 0; s < KW; s++) wr[s] = wp[s * 64];
     }
     uint4 pre[NLD];
-    const bool whole = VEC && a.xc0 + ((a.cin + 7) & ~7) <= a.xcs;  // partial groups load as one 16-byte group
     {
         const int iy0 = oy0 * S - a.pad, ix0 = ox0 * S - a.pad;
 #pragma unroll
@@ -603,7 +627,7 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
             if ((i + 1) * NT <= HALO || e < HALO)
                 if (gy >= 0 && gy < a.h && gx >= 0 && gx < a.w && ch < a.cin)
                     pre[i] = load_group<VEC>(
-                        a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin, whole);
+                        a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin);
         }
     }
     uint2 rres[FM];
@@ -637,7 +661,7 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
         const int e = tid + i * NT;
         if ((i + 1) * NT <= HALO || e < HALO) {
             const int pix = e / GPT, g = e - pix * GPT;
-            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = whole ? mask_group(pre[i], a.cin - g * 8) : pre[i];
+            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
         }
     }
     __syncthreads();

@@ -20,12 +20,15 @@
 //   (k = tap * CK + ci within a chunk; api.cpp, pack_weights).
 // - A partial last 8-channel group (cin not a multiple of 8) arrives whole with the channels next to it in the
 //   tensor; its channels past cin are zeroed in LDS before the chunk computes (they may hold anything, NaN
-//   included, and zero weights do not cancel NaN).
+//   included, and zero weights do not cancel NaN). In a view of 4-byte channel pairs that group arrives as the
+//   pixel's last 8 channels (the channels next to it may be another pixel's, or past the tensor's end) and is moved
+//   down to its place in LDS.
 // - Global split-K (grid.z = z splits of chunks_per_split chunks): f32 partials [z][pixel][np], summed in z order
 //   by splitk_reduce, which then runs the epilogue; without a split the epilogue (bias, activation, f16, residual)
 //   runs straight from the accumulators.
-// - The input view must be 16-byte aligned (channel stride and offset multiples of 8, the base pointer aligned) and
-//   below 2^31 bytes; the launcher runs the chunked kernel (the same packed weights) on any other view.
+// - The input view must be 16-byte aligned (channel stride and offset multiples of 8, the base pointer aligned), or
+//   4-byte aligned with an even cin of at least 8 (a DMA lane's 16 bytes need dword alignment), and below 2^31 bytes;
+//   the launcher runs the chunked kernel (the same packed weights) on any other view.
 #pragma once
 #include "wave_impl.h"
 
@@ -80,7 +83,8 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_gemm(ConvKArgs a) {
     const auto rw = buffer_rsrc(a.wpk, (uint32_t)((uint64_t)(a.np / 16) * nch * KSC * 1024));
 
     // the lane's slot of each of this wave's halo DMA instructions (instruction k = wave + NW * i), the same for
-    // every chunk: its byte offset in chunk 0 (kOOB: padding, a pad slot or past the halo) and its first channel
+    // every chunk: its pixel's byte offset (kOOB: padding, a pad slot or past the halo) and its first channel in a
+    // chunk
     uint32_t hoff[DHW];
     int hch[DHW];
 #pragma unroll
@@ -89,17 +93,20 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_gemm(ConvKArgs a) {
         const int iy = p / IW, ix = p - iy * IW, gy = iy0 + iy, gx = ix0 + ix;
         const bool ok = (s < IH * IW * SLOTS) & (g < GPC) & (gy >= 0) & (gy < a.h) & (gx >= 0) & (gx < a.w);
         hoff[i] = ok ? ((((uint32_t)(img * a.h + gy) * (uint32_t)a.w + (uint32_t)gx) * (uint32_t)a.xcs) +
-                        (uint32_t)(a.xc0 + g * 8)) * 2u
+                        (uint32_t)a.xc0) * 2u
                      : kOOB;
         hch[i] = g * 8;
     }
+    // the last first channel of a group: a 4-byte aligned view's partial group is the pixel's last 8 channels
+    const int ch_max = a.xvec ? a.cin : a.cin - 8;
     // chunk c into buffer b: every wave issues DHW halo and DWW weight instructions (the padding ones write zeros)
     auto dma_chunk = [&](int b, int c) {
         const int c0 = c * CK;
 #pragma unroll
         for (int i = 0; i < DHW; i++)
             lds_dma16(rx, hbuf(b) + (wave + NW * i) * 64,
-                      ((hoff[i] != kOOB) & (c0 + hch[i] < a.cin)) ? hoff[i] + (uint32_t)c0 * 2u : kOOB);
+                      ((hoff[i] != kOOB) & (c0 + hch[i] < a.cin)) ? hoff[i] + (uint32_t)min(c0 + hch[i], ch_max) * 2u
+                                                                  : kOOB);
 #pragma unroll
         for (int i = 0; i < DWW; i++) {
             const int k = wave + NW * i;  // weight instruction k: block k / KSC of the tile, k-step k % KSC
@@ -115,7 +122,10 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_gemm(ConvKArgs a) {
         if ((rem_last & 7) == 0) return;  // uniform
         const int g = rem_last >> 3, keep = rem_last & 7;
         uint4* hb = hbuf(b);
-        for (int p = tid; p < IH * IW; p += 64 * NW) hb[p * SLOTS + g] = mask_group(hb[p * SLOTS + g], keep);
+        for (int p = tid; p < IH * IW; p += 64 * NW) {
+            const uint4 v = hb[p * SLOTS + g];
+            hb[p * SLOTS + g] = a.xvec ? mask_group(v, keep) : shift_group(v, 8 - keep);
+        }
     };
 
     // the first chunks' DMA goes out first; the residual and parameter loads queue behind it
@@ -232,9 +242,11 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_gemm(ConvKArgs a) {
     }
 }
 
-// Whether the kernel's input path serves these views: 16-byte aligned groups, offsets below 2^31.
+// Whether the kernel's input path serves these views: 16-byte aligned groups, or channel pairs aligned to 4 bytes and
+// an even cin of at least 8, offsets below 2^31.
 inline bool gemm_path_ok(const ConvKArgs& a) {
-    return a.xvec && (uint64_t)a.n * a.h * a.w * a.xcs * 2 < (1ull << 31);
+    const bool pairs = (uintptr_t)a.x % 4 == 0 && a.xcs % 2 == 0 && a.xc0 % 2 == 0 && a.cin % 2 == 0 && a.cin >= 8;
+    return (a.xvec || pairs) && (uint64_t)a.n * a.h * a.w * a.xcs * 2 < (1ull << 31);
 }
 
 // The chunked kernel's configuration that stands in on views the DMA path cannot read: 8 rows x 16 channels, which

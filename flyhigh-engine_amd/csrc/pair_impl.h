@@ -160,7 +160,6 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
     uint4 pre[NLD];
     uint32_t inside = 0;  // bit i: pre[i] holds input values (not the zero padding)
     static_assert(NLD <= 32 && NT % GPA == 0, "a lane stages the same channel group in every round");
-    const bool whole = VEC && a.xc0 + ((a.cin + 7) & ~7) <= a.xcs;  // partial groups load as one 16-byte group
     {
         const int iy0 = (oy0 - 1) * SA - a.pad, ix0 = (ox0 - 1) * SA - a.pad;
 #pragma unroll
@@ -173,7 +172,7 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
             if ((i + 1) * NT <= HALO || e < HALO)
                 if (gy >= 0 && gy < a.h && gx >= 0 && gx < a.w && ch < a.cin) {
                     pre[i] = load_group<VEC>(
-                        a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin, whole);
+                        a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin);
                     if constexpr (FILM) inside |= 1u << i;
                 }
         }
@@ -224,7 +223,7 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
         const int e = tid + i * NT;
         if ((i + 1) * NT <= HALO || e < HALO) {
             const int pix = e / GPA, g = e - pix * GPA;
-            uint4 q = whole ? mask_group(pre[i], a.cin - g * 8) : pre[i];
+            uint4 q = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
             if constexpr (FILM)
                 if ((inside >> i) & 1u) q = film_group(q, fgm, fbt, a.cin - g * 8);
             *reinterpret_cast<uint4*>(hin + pix * PSA + g * 8) = q;

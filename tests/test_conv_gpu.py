@@ -166,6 +166,30 @@ def test_padded_channel_stride_views(shape):
         assert np.array_equal(got[..., cout:], c.y0[..., cout:])
 
 
+# (shape, input view): channel pairs (4-byte aligned) on the deep-layer kernel with a partial last group of 2, 4 and 6
+# channels and with none, the view ending with the tensor and inside a wider one; odd strides, offsets and channel
+# counts (2-byte aligned) on the direct kernel's one-tile forms and the chunked kernel (stride 2 over 64 channels)
+UNALIGNED = [((2, 47, 51, 66, 40, 1), (66, 0)), ((1, 65, 67, 100, 52, 1), (100, 0)), ((1, 64, 64, 78, 20, 1), (86, 6)),
+             ((1, 64, 65, 80, 36, 1), (82, 2)), ((1, 65, 64, 99, 24, 1), (99, 0)), ((1, 19, 37, 9, 24, 1), (9, 0)),
+             ((2, 18, 33, 15, 20, 2), (17, 1)), ((1, 17, 35, 36, 48, 1), (37, 1)), ((1, 30, 54, 155, 48, 1), (155, 0)),
+             ((1, 17, 20, 71, 33, 2), (73, 2)), ((1, 17, 18, 7, 5, 1), (7, 0))]
+
+
+@pytest.mark.parametrize("shape,xv", UNALIGNED, ids=lambda s: "x".join(map(str, s)))
+def test_unaligned_dense_views(shape, xv):
+    # 16-byte input loads at 2- and 4-byte alignment: a partial last group arrives as the pixel's last 8 channels, so
+    # nothing past the view's last channel is read, and the channels before it (its own, or NaN outside the view)
+    # never reach another channel's place
+    n, h, w, cin, cout, s = shape
+    c = Case(n, h, w, cin, cout, stride=s, act=1, xv=xv, poison=xv[0] > cin, seed=cin)
+    got, plan = c.run_gpu(return_plan=True)
+    say("unaligned", shape, xv, plan.describe()["name"])
+    if cin % 2 == 0 and cin > 64:
+        assert plan.describe()["family"] == "gemm"
+    ok, md, mref = parity(got, c.run_oracle(threads=8))
+    assert ok, (plan.describe()["name"], md, mref)
+
+
 def test_batch_images_are_independent():
     c = Case(3, 22, 35, 24, 40, act=1, residual=True, seed=12)
     batched = c.run_gpu()
