@@ -423,6 +423,101 @@ bool configure(fhc_conv_plan& p, const Variant& v, std::string* why, bool pairs 
     return configure_igemm(p, v.cfg, v.ks, why);
 }
 
+// The direct configuration of these parameters that serves the conv, or -1
+int direct_index(const fhc_conv_desc& d, int fm, int wm, int wn, int wk, int persist) {
+    for (int i = 0; i < kNumDirect; i++) {
+        const DirectCfg& c = kDirectCfgs[i];
+        if (direct_fits(d, i) && c.fm == fm && c.wm == wm && c.wn == wn && c.na == 1 && c.wk == wk && c.persist == persist)
+            return i;
+    }
+    return -1;
+}
+
+// The 3x3 configurations measured faster than the general choices below, by the input channels padded to 32 (c), the
+// output channel blocks of 16 (b) and the output pixels (px); 0 where none is. The lines come from every variant's
+// time over some 400 shapes of the layers' ranges (17 to 544 rows, batches to 24), each lying where one family's times
+// cross the other's; over all of them the chosen variant is within 5% of the fastest on average, where the general
+// choices alone were 30% off (each line: an example with both sides' times, us).
+uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
+    if (d.kh != 3) return 0;
+    const uint32_t c = div_ceil(d.cin, 32) * 32, b = div_ceil(d.cout, 16);
+    const uint64_t px = (uint64_t)d.n * g.hout * g.wout, work = px * b;
+    auto dir = [&](int fm, int wm, int wn, int wk = 1, int persist = 0) -> uint32_t {
+        const int i = direct_index(d, fm, wm, wn, wk, persist);
+        return i < 0 ? 0 : kDirectBase + (uint32_t)i;
+    };
+    auto gemm = [&](int i) -> uint32_t { return make_code(i, 1, 3); };
+    // large tensors: the resident grid, whose weights load once, where the views allow its buffer loop
+    const bool in16 = d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0;
+    const bool loop = (in16 || pairs_view(d)) && d.cout % 4 == 0 && d.y_cstride % 4 == 0 && d.y_c0 % 4 == 0 &&
+                      (!d.residual || (d.r_cstride % 4 == 0 && d.r_c0 % 4 == 0)) &&
+                      (uint64_t)d.n * d.h * d.w * std::max({d.x_cstride, d.y_cstride, d.r_cstride}) * 2 < (1ull << 31);
+    if (loop && b >= 2 && d.stride == 1) {
+        // 14 -> 24 at 622,080 px: 18.3 against 23.5; 32 -> 48 at 264,322: 15.5 against 28.8
+        if (c == 32 && (b == 2 ? px >= 150000 : px >= 60000)) return dir(8, 1, b == 2 ? 2 : 4, 1, 1);
+        // 48 -> 128 at 309,190 px: 45 against 257; 64 -> 128 at 32,144: 11.5 against 37.7
+        if (c == 64 && (px >= 60000 || (b >= 5 && work >= 80000))) return dir(4, 1, b == 2 ? 2 : 4, 1, 1);
+        // 128 -> 128 at 275,940 px: 78 against the deep-layer kernel's 185, at 8,160: 9.6 against 8.8;
+        // 96 -> 96 at 65,280: 16.6 against 28.2; the fewest channel tiles that cover cout, then the narrowest
+        if ((c == 96 && work >= 80000) || (c == 128 && work >= (b >= 4 ? 80000u : 110000u))) {
+            const int widths[] = {2, 3, 4, 6, 8};
+            int wn = 8;
+            for (int w : widths)
+                if (div_ceil(b, (uint32_t)w) < div_ceil(b, (uint32_t)wn) ||
+                    (div_ceil(b, (uint32_t)w) == div_ceil(b, (uint32_t)wn) && w < wn))
+                    wn = w;
+            return dir(4, 1, wn, 1, 1);
+        }
+    }
+    if (loop && b >= 2 && d.stride == 2) {
+        if (c == 32 && b >= 3 && px >= 60000) return dir(2, 2, 4, 1, 1);  // 32 -> 64 at 130,560 px: 15.1 against 19
+        if (c == 64 && (b == 2 ? px >= 60000 : work >= 120000))            // 64 -> 96 at 113,430 px: 27.4 against 47.3
+            return dir(2, 2, b == 2 ? 2 : 4, 1, 1);
+    }
+    if (d.stride == 2) {  // two rows a wave: half the weight loads. 64 -> 72 at 14,400 px: 6.9 against 10.1
+        if (c == 32 && b >= 3 && px >= 16000 && px < 60000) return dir(2, 1, b == 4 || b > 6 ? 4 : 3);
+        if (c == 64 && b >= 5 && px >= 5000) return dir(2, 1, 3);
+        return 0;
+    }
+    if (c == 64 || c == 96) {  // small tensors: a third of the chain a wave. 96 -> 96 at 960 px: 3.7 against 5.1
+        if (b == 1 && px < (c == 64 ? 16000u : 7000u)) return dir(1, 1, 1, 3);
+        if (b == 2 && px < 4096) return dir(1, 1, 2, 3);
+        if (b == 3 && px < 7000) return dir(1, 1, 3, 3);
+        if (b >= 4 && px < (c == 64 ? 2500u : 4096u)) return dir(1, 1, 3, 3);
+    }
+    if (c == 32) {
+        if (b == 2 && px >= 24000 && px < 60000) return dir(4, 2, 2);  // 14 -> 24 at 58,880 px: 5.0 against 6.0
+        if (b == 3 && px >= 10000) return dir(2, 1, 3);                // 32 -> 48 at 12,480 px: 3.8 against 4.0
+        if (b >= 5 && px >= 7000) return px < 16000 ? dir(2, 1, 2) : dir(4, 2, 2);  // 32 -> 128 at 40,000: 1.0 to 1.7
+    }
+    if (c == 64) {
+        if (b == 2 && px >= 16000 && px < 60000) return dir(2, 1, 2);  // 64 -> 32 at 39,501 px: 6.0 against 7.1
+        if ((b == 3 || b == 4) && px >= 7000) return dir(2, 1, b);     // 48 -> 48 at 32,640 px: 5.9 against 9.7
+        if (b >= 5 && px >= 4096) return dir(2, 1, 3);                 // 64 -> 96 at 5,852 px: 4.7 against 5.2
+    }
+    if (c == 96 && px >= 4096) {  // below the resident grid's line
+        if (b == 1) return px < 60000 ? dir(2, 1, 1, 3) : dir(2, 4, 1);  // 72 -> 5 at 159,960 px: 16.8 against 33.5
+        if (b == 2 || b == 3) return dir(2, 1, b);                       // 96 -> 48 at 8,991 px: 5.7 against 7.3
+        return dir(4, 2, 2);                                             // 96 -> 96 at 8,160 px: 7.1 against 7.6
+    }
+    if (c == 128 && px >= 4096) {
+        if (b == 1) return px < 16000 ? dir(1, 2, 1) : dir(2, 4, 1);  // 128 -> 12 at 10,660 px: 5.3 against 7.7
+        if (b == 2) return px < 16000 ? dir(1, 2, 2) : dir(2, 4, 1);  // 128 -> 32 at 8,160 px: 5.9 against 7.7
+        if (b == 3 && px < 20000) return dir(2, 4, 1);                // 128 -> 48 at 8,160 px: 6.0 against 8.2
+    }
+    if (c == 160 || c == 288) {
+        if (b == 1 && (c == 160 || px < 60000)) return dir(2, 1, 1, 3);  // 279 -> 12 at 4,158 px: 6.8 against 12.1
+        if (c == 160 && (b == 2 || b == 3) && px < 7000) return dir(2, 1, b, 3);  // 155 -> 24 at 4,230 px: 5.1 against 8.7
+        if (in16) {
+            if (b <= 2 && px >= 60000) return gemm(2);  // 155 -> 32 at 60,000 px and up: 1.0 to 1.4
+            if (b == 4 && px >= 7000) return gemm(12);  // 279 -> 64: 1.0 to 1.6
+            if (b >= 7 && px >= (c == 160 ? 7000u : 60000u)) return gemm(12);  // 155 -> 128 at 145,992 px: 101 against 128
+            if (px >= 60000) return gemm(13);           // 155 -> 48 at 155,520 px: 42.3 against 51.9
+        }
+    }
+    return 0;
+}
+
 // The direct configuration the planner takes without a table entry, or -1: among the one-block-per-wave
 // configurations that launch one workgroup per tile, the narrowest channel tile that covers cout in one tile (else
 // the widest there is), and among the tile heights the tallest that still gives about two workgroups per CU (the
@@ -431,7 +526,8 @@ bool configure(fhc_conv_plan& p, const Variant& v, std::string* why, bool pairs 
 int direct_default(const fhc_conv_desc& d, const Geometry& g) {
     const int need = (int)div_ceil(d.cout, 16);
     auto eligible = [&](int i) {
-        return direct_fits(d, i) && kDirectCfgs[i].na == 1 && (kDirectCfgs[i].wk == 1 || kDirectCfgs[i].cin32 > 128);
+        return direct_fits(d, i) && kDirectCfgs[i].na == 1 && !kDirectCfgs[i].persist &&
+               (kDirectCfgs[i].wk == 1 || kDirectCfgs[i].cin32 > 128);
     };
     int best_wn = 0;
     for (int i = 0; i < kNumDirect; i++) {
@@ -444,7 +540,7 @@ int direct_default(const fhc_conv_desc& d, const Geometry& g) {
     uint64_t pick_wgs = 0;
     int pick_th = 0;
     for (int i = 0; i < kNumDirect; i++) {
-        if (!eligible(i) || kDirectCfgs[i].wn != best_wn || kDirectCfgs[i].persist) continue;
+        if (!eligible(i) || kDirectCfgs[i].wn != best_wn) continue;
         const int th = kDirectCfgs[i].fm * kDirectCfgs[i].wm;
         const uint64_t wgs = (uint64_t)d.n * div_ceil(g.hout, th) * div_ceil(g.wout, 16) * div_ceil(d.cout, 16 * best_wn);
         const bool enough = wgs >= 512;
@@ -462,26 +558,40 @@ int direct_default(const fhc_conv_desc& d, const Geometry& g) {
 // and its batched form, and on the 128 -> 128 layer at 1080p/16).
 constexpr int kGemmDefault = 11;
 
-// The MI355X planner's default when neither the caller nor the table chose. The deep-layer kernel serves stride-1
-// 3x3 convs over at least 64 input channels whose input view has 16-byte channel groups; it takes those over 64
-// input channels with at least 4096 output pixels (on smaller ones its fixed cost per launch, the first chunk's
-// load and the epilogue, outweighs the direct kernel's longer chains). Then the direct kernel whenever a
-// configuration serves the input channels, then the deep-layer kernel where it serves, else the chunked kernel.
-uint32_t heuristic_code(const fhc_conv_desc& d, const Geometry& g) {
-    const bool gemm_ok = d.kh == 3 && d.stride == 1 && d.cin >= 64 && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0 &&
-                         (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31);
-    const bool big = d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096;
-    if (gemm_ok && big) return make_code(kGemmDefault, 1, 3);
-    // the same layers in a view of channel pairs, unless the caller splits K: 100 -> 100 at 3 x 135 x 241 in a dense
-    // view 76 us (73 in a padded stride) where the direct kernel took 163 with 2-byte loads
-    const bool unsplit = d.ksplit == 0 && (d.ref_cand == 0xFFu || (d.ref_cand >> 4) == 0);
-    if (big && unsplit && d.kh == 3 && d.stride == 1 && pairs_view(d) &&
-        (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31))
+// The planner's general choice: the deep-layer kernel for stride-1 3x3 convs over more than 64 input channels whose
+// input view has 16-byte channel groups and at least 4096 output pixels (on smaller ones its fixed cost per launch, the
+// first chunk's load and the epilogue, outweighs the direct kernel's longer chains), with `pairs` also in views of
+// channel pairs: 100 -> 100 at 3 x 135 x 241 in a dense view took the direct kernel 163 us with 2-byte loads, this one
+// 76. Then the direct kernel whenever a configuration serves the input channels, then the deep-layer kernel from 64
+// input channels, else the chunked kernel.
+uint32_t general_code(const fhc_conv_desc& d, const Geometry& g, bool pairs) {
+    const bool deep = d.kh == 3 && d.stride == 1 && d.cin >= 64 &&
+                      (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31);
+    const bool gemm_ok = deep && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0;
+    if ((gemm_ok || (deep && pairs && pairs_view(d))) && d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096)
         return make_code(kGemmDefault, 1, 3);
     const int idx = direct_default(d, g);
     if (idx >= 0) return kDirectBase + (uint32_t)idx;
     if (gemm_ok) return make_code(kGemmDefault, 1, 3);
     return (uint32_t)heuristic_cfg(d, g);
+}
+
+// Whether a variant is a one-tile direct configuration with each output's K in one chain, tap by tap: all of these (of
+// one padded channel count) give the same bits
+bool tap_order(uint32_t code) {
+    Variant v;
+    return decode_code(code, &v) && v.family == 1 && kDirectCfgs[v.cfg].na == 1 && kDirectCfgs[v.cfg].wk == 1 &&
+           !kDirectCfgs[v.cfg].persist;
+}
+
+// The MI355X planner's default when neither the caller nor the table chose: measured_code's where it has one, else the
+// general choice. A caller that fixes the K split at 1 keeps the general choice's K order, hence its bits (the frame
+// program does: rounding in another order travels through the whole network): a measured choice then stands only
+// where both are one-tile chains. A split above 1 moves the general choice to its split form.
+uint32_t heuristic_code(const fhc_conv_desc& d, const Geometry& g) {
+    const bool unsplit = d.ksplit == 0 && (d.ref_cand == 0xFFu || (d.ref_cand >> 4) == 0);
+    const uint32_t general = general_code(d, g, unsplit), m = measured_code(d, g);
+    return m && (unsplit || (d.ksplit == 1 && tap_order(m) && tap_order(general))) ? m : general;
 }
 
 int heuristic_cfg(const fhc_conv_desc& d, const Geometry& g) {

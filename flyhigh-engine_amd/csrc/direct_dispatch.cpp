@@ -12,6 +12,7 @@ LaunchFn direct_launcher_s1p(int index, const void** kernel, bool residual);
 LaunchFn direct_launcher_s2(int index, const void** kernel, bool residual);
 LaunchFn direct_launcher_k1(int index, const void** kernel, bool residual);
 LaunchFn direct_launcher_w(int index, const void** kernel, bool residual);
+LaunchFn direct_launcher_s1q(int index, const void** kernel, bool residual);
 
 LaunchFn direct_launcher(int index, const void** kernel, bool residual) {
     if (index < 0 || index >= kNumDirect) return nullptr;
@@ -23,6 +24,7 @@ LaunchFn direct_launcher(int index, const void** kernel, bool residual) {
     if (index >= 77 && index <= 107) return direct_launcher_s2(index, kernel, residual);
     if (index >= 108 && index <= 123) return direct_launcher_k1(index, kernel, residual);
     if (index >= 124 && index <= 131) return direct_launcher_w(index, kernel, residual);
+    if (index >= 132 && index <= 141) return direct_launcher_s1q(index, kernel, residual);
     return nullptr;
 }
 

@@ -431,6 +431,8 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
         // here once: the loop then spends a few full-rate VALU instructions per memory access. Offsets are 32-bit
         // unsigned (the launcher keeps every view below 2^31 bytes); a base that wraps below zero at the image's
         // top-left corner comes back in range for every lane whose access is valid.
+        // a view of channel pairs: a partial last group is the pixel's last 8 channels, moved into place later
+        const int ch_max = a.xvec ? a.cin : a.cin - 8;
         uint32_t hoff[NLD];  // halo element i: byte offset from the tile's first halo pixel
         int hpos[NLD];       // its halo row << 16 | column
         bool hst[NLD];       // inside the halo and below cin (tile-invariant part of its validity)
@@ -439,7 +441,7 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
             const int e = tid + i * NT;
             const int pix = e / GPT, g = e - pix * GPT;
             const int iy = pix / IW, ix = pix - iy * IW;
-            hoff[i] = ((uint32_t)(iy * a.w + ix) * (uint32_t)a.xcs + (uint32_t)(a.xc0 + g * 8)) * 2u;
+            hoff[i] = ((uint32_t)(iy * a.w + ix) * (uint32_t)a.xcs + (uint32_t)(a.xc0 + min(g * 8, ch_max))) * 2u;
             hpos[i] = (iy << 16) | ix;
             hst[i] = ((i + 1) * NT <= HALO || e < HALO) & (g * 8 < a.cin);
         }
@@ -464,8 +466,8 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
                     uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, ok ? base + hoff[i] : kOOB, 0, 0));
             }
         };
-        // the staged halo into LDS; the channels of a partial last group past cin are zeroed only when cin is not
-        // a multiple of 8 (a uniform branch around arithmetic)
+        // the staged halo into LDS; the channels of a partial last group past cin are zeroed (in a view of channel
+        // pairs: the group moved down) only when cin is not a multiple of 8 (uniform branches around arithmetic)
         auto write_halo_b = [&]() {
             if ((a.cin & 7) == 0) {
 #pragma unroll
@@ -474,12 +476,19 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
                     const int pix = e / GPT, g = e - pix * GPT;
                     *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = pre[i];
                 }
+            } else if (a.xvec) {
+#pragma unroll
+                for (int i = 0; i < NLD; i++) {
+                    const int e = tid + i * NT;
+                    const int pix = e / GPT, g = e - pix * GPT;
+                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<true>(pre[i], a.cin - g * 8, a.cin);
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < NLD; i++) {
                     const int e = tid + i * NT;
                     const int pix = e / GPT, g = e - pix * GPT;
-                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = mask_group(pre[i], a.cin - g * 8);
+                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<false>(pre[i], a.cin - g * 8, a.cin);
                 }
             }
         };
@@ -759,13 +768,19 @@ hipError_t launch_tile_split(const ConvKArgs& a, dim3 grid, size_t lds, hipStrea
     return hipGetLastError();
 }
 
+// Whether an input view holds channel pairs at 4-byte alignment that 16-byte buffer loads and LDS DMA (which need
+// dword alignment) can read: every group at a dword, a partial last group as the pixel's last 8 channels
+inline bool pairs_ok(const ConvKArgs& a) {
+    return (uintptr_t)a.x % 4 == 0 && a.xcs % 2 == 0 && a.xc0 % 2 == 0 && a.cin % 2 == 0 && a.cin >= 8;
+}
+
 // Whether a launch can take the buffer-instruction loop of the persistent configurations: 16-byte aligned input
-// whose last 8-channel group lies inside the pixel's stride (the group loads whole), 8-byte aligned output and
-// residual with cout a multiple of 4, and extents within the 2^31 bytes a buffer offset reaches.
+// (whose stride then holds every 8-channel group whole) or one of channel pairs, 8-byte aligned output and residual
+// with cout a multiple of 4, and extents within the 2^31 bytes a buffer offset reaches.
 inline bool buffer_path_ok(const ConvKArgs& a) {
     const uint64_t pin = (uint64_t)a.n * a.h * a.w, pout = (uint64_t)a.n * a.hout * a.wout;
     const uint64_t lim = 1ull << 31;
-    return a.xvec && a.yvec && a.cout % 4 == 0 && (!a.residual || a.rvec) && a.xc0 + ((a.cin + 7) & ~7) <= a.xcs &&
+    return (a.xvec || pairs_ok(a)) && a.yvec && a.cout % 4 == 0 && (!a.residual || a.rvec) &&
            pin * (uint64_t)a.xcs * 2 < lim && view_bytes(pout, a.ycs, a.yc0, a.cout) < lim &&
            (!a.residual || view_bytes(pout, a.rcs, a.rc0, a.cout) < lim);
 }

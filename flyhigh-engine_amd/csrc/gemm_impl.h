@@ -245,8 +245,7 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_gemm(ConvKArgs a) {
 // Whether the kernel's input path serves these views: 16-byte aligned groups, or channel pairs aligned to 4 bytes and
 // an even cin of at least 8, offsets below 2^31.
 inline bool gemm_path_ok(const ConvKArgs& a) {
-    const bool pairs = (uintptr_t)a.x % 4 == 0 && a.xcs % 2 == 0 && a.xc0 % 2 == 0 && a.cin % 2 == 0 && a.cin >= 8;
-    return (a.xvec || pairs) && (uint64_t)a.n * a.h * a.w * a.xcs * 2 < (1ull << 31);
+    return (a.xvec || pairs_ok(a)) && (uint64_t)a.n * a.h * a.w * a.xcs * 2 < (1ull << 31);
 }
 
 // The chunked kernel's configuration that stands in on views the DMA path cannot read: 8 rows x 16 channels, which

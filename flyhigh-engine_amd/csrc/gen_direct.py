@@ -79,6 +79,12 @@ def entries():
         for wn in (2, 4):
             add(1, 1, cin32, 1, 2, wn, 1)
             add(1, 1, cin32, 2, 1, wn, 1)
+    # big layers over more channels, persistent (their codes follow every earlier one's): one wave row of 4 rows, the
+    # weights of up to 8 channel blocks over its waves (by the compiler's register report, not the estimate: the
+    # larger ones keep weights in AGPRs, and (128, 8) spills 6 registers and is still the fastest over 80 channels)
+    for cin32, wns in ((96, (2, 3, 4, 6, 8)), (128, (2, 3, 4, 6, 8))):
+        for wn in wns:
+            out.append((3, 1, cin32, 4, 1, wn, 1, 1, 1))
     # wave-stream kernel (wave_impl.h): 4 independent waves, each FM rows x 16 pixels x all 16 * NA channels of
     # the workgroup's channel tile; weights NA * K / 8 VGPRs per lane at one wave per SIMD
     # ((3, 1, 64, 2, 4) spills: 288 weight registers)
@@ -100,12 +106,12 @@ def group(e):
     if e[8] == 2:
         return "w"
     if e[8]:
-        return "s1p"
+        return "s1p" if cin32 <= 64 else "s1q"
     return {32: "s1a", 64: "s1a", 96: "s1b", 128: "s1c", 160: "s1d", 288: "s1d"}[cin32]
 
 
 def main():
-    order = ["s1a", "s1b", "s1c", "s1d", "s1p", "s2", "k1", "w"]
+    order = ["s1a", "s1b", "s1c", "s1d", "s1p", "s2", "k1", "w", "s1q"]
     es = sorted(entries(), key=lambda e: order.index(group(e)))
     assert len(es) <= 383  # variant codes 128 .. 511
     h = ["// Generated by gen_direct.py: the configurations of the direct conv kernel. Do not edit.",

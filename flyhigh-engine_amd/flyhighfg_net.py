@@ -346,8 +346,11 @@ class GpuBackend(ComposedChains):
         cin, cout, stride, act = self.convs[name]
         n, h, w, xcs = x.buf.shape
         ycs = y.buf.shape[3]
+        # the table's choice, else the planner's in the general choice's K order (K split 1): the network carries a
+        # change of rounding in one conv on to 3% of a frame's bytes
+        tuned = self.fhconv.tune_get(cin, cout, h, w, stride, n=n) is not None
         return self.fhconv.make_desc(n, h, w, cin, cout, stride=stride, act=act, residual=res is not None or mid_res,
-                                     x_cstride=xcs, x_c0=x.c0, y_cstride=ycs, y_c0=y.c0,
+                                     ksplit=0 if tuned else 1, x_cstride=xcs, x_c0=x.c0, y_cstride=ycs, y_c0=y.c0,
                                      r_cstride=res.buf.shape[3] if res is not None else (ycs if mid_res else 0),
                                      r_c0=res.c0 if res is not None else 0)
 

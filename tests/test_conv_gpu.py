@@ -166,17 +166,22 @@ def test_padded_channel_stride_views(shape):
         assert np.array_equal(got[..., cout:], c.y0[..., cout:])
 
 
-# (shape, input view): channel pairs (4-byte aligned) on the deep-layer kernel with a partial last group of 2, 4 and 6
-# channels and with none, the view ending with the tensor and inside a wider one; odd strides, offsets and channel
-# counts (2-byte aligned) on the direct kernel's one-tile forms and the chunked kernel (stride 2 over 64 channels)
-UNALIGNED = [((2, 47, 51, 66, 40, 1), (66, 0)), ((1, 65, 67, 100, 52, 1), (100, 0)), ((1, 64, 64, 78, 20, 1), (86, 6)),
-             ((1, 64, 65, 80, 36, 1), (82, 2)), ((1, 65, 64, 99, 24, 1), (99, 0)), ((1, 19, 37, 9, 24, 1), (9, 0)),
-             ((2, 18, 33, 15, 20, 2), (17, 1)), ((1, 17, 35, 36, 48, 1), (37, 1)), ((1, 30, 54, 155, 48, 1), (155, 0)),
-             ((1, 17, 20, 71, 33, 2), (73, 2)), ((1, 17, 18, 7, 5, 1), (7, 0))]
+# (shape, input view, the planner's form): channel pairs (4-byte aligned) on the deep-layer kernel and the resident
+# grids, with a partial last group of 2, 4 and 6 channels and with none, the view ending with the tensor and inside a
+# wider one; odd strides, offsets and channel counts (2-byte aligned) on the direct kernel's one-tile forms and the
+# chunked kernel (stride 2 over 64 channels)
+UNALIGNED = [((2, 47, 51, 130, 68, 1), (130, 0), "gemm"), ((1, 65, 67, 100, 52, 1), (100, 0), "gemm"),
+             ((1, 64, 64, 126, 68, 1), (134, 6), "gemm"), ((1, 64, 65, 104, 84, 1), (106, 2), "gemm"),
+             ((1, 101, 103, 66, 128, 1), (66, 0), "/p"), ((1, 101, 103, 102, 128, 1), (106, 2), "/p"),
+             ((2, 175, 177, 36, 48, 1), (36, 0), "/p"), ((1, 251, 243, 14, 36, 1), (14, 0), "/p"),
+             ((1, 499, 487, 12, 36, 2), (14, 2), "/p"), ((1, 65, 64, 99, 24, 1), (99, 0), "direct"),
+             ((1, 19, 37, 9, 24, 1), (9, 0), "direct"), ((2, 18, 33, 15, 20, 2), (17, 1), "direct"),
+             ((1, 17, 35, 36, 48, 1), (37, 1), "direct"), ((1, 30, 54, 155, 48, 1), (155, 0), "direct"),
+             ((1, 17, 20, 71, 33, 2), (73, 2), "igemm"), ((1, 17, 18, 7, 5, 1), (7, 0), "direct")]
 
 
-@pytest.mark.parametrize("shape,xv", UNALIGNED, ids=lambda s: "x".join(map(str, s)))
-def test_unaligned_dense_views(shape, xv):
+@pytest.mark.parametrize("shape,xv,form", UNALIGNED, ids=lambda s: s if isinstance(s, str) else "x".join(map(str, s)))
+def test_unaligned_dense_views(shape, xv, form):
     # 16-byte input loads at 2- and 4-byte alignment: a partial last group arrives as the pixel's last 8 channels, so
     # nothing past the view's last channel is read, and the channels before it (its own, or NaN outside the view)
     # never reach another channel's place
@@ -184,10 +189,25 @@ def test_unaligned_dense_views(shape, xv):
     c = Case(n, h, w, cin, cout, stride=s, act=1, xv=xv, poison=xv[0] > cin, seed=cin)
     got, plan = c.run_gpu(return_plan=True)
     say("unaligned", shape, xv, plan.describe()["name"])
-    if cin % 2 == 0 and cin > 64:
-        assert plan.describe()["family"] == "gemm"
+    assert form in plan.describe()["name"]
     ok, md, mref = parity(got, c.run_oracle(threads=8))
     assert ok, (plan.describe()["name"], md, mref)
+
+
+# the resident grids over 96 and 128 padded channels: every width, ragged tiles, several channel tiles with a partial
+# last one, more tiles than workgroups, with and without a residual, a padded and a dense view
+@pytest.mark.parametrize("shape", [(1, 21, 35, 72, 20), (2, 90, 190, 96, 36), (1, 37, 50, 100, 132), (3, 61, 130, 128, 64)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_deep_resident_grids_match_the_oracle(shape):
+    n, h, w, cin, cout = shape
+    for residual in (False, True):
+        c = Case(n, h, w, cin, cout, act=1, residual=residual, seed=cout, xv=((cin + 7) // 8 * 8, 0))
+        want = c.run_oracle(threads=8)
+        codes = [k for k in fhconv.variant_list(c.fhc_desc()) if fhconv.variant_name(k).endswith("/p")]
+        assert codes
+        for code in codes:
+            ok, md, mref = parity(c.run_gpu(variant=code), want)
+            assert ok, (fhconv.variant_name(code), residual, md, mref)
 
 
 def test_batch_images_are_independent():
