@@ -1879,7 +1879,7 @@ __global__ __launch_bounds__(kThreads) void rgba_resize_kernel(const uint32_t* s
 // before its in-order additions.
 constexpr uint32_t kGmNwg = gmfit::kNwg, kGmWg = gmfit::kWg;  // gm_fit_reduce's workgroups and their size
 constexpr uint32_t kGmPart = gmfit::kPart;                     // one round's partial sums [workgroup][channel][9]
-constexpr uint32_t kGmT = 16;                 // the box tile's edge and the cost block's width, in cells
+constexpr uint32_t kGmT = 16;                 // the cost block's width, in cells
 constexpr uint32_t kGmRmax = 32;              // largest box radius: r_dwin = round(16 s), s <= 2
 
 // The repair of several pairs at once: every kernel below takes the pair from one grid dimension (pair k: pictures
@@ -1997,58 +1997,104 @@ __global__ __launch_bounds__(kThreads) void gm_cost_kernel(View a, View b, uint3
     if (second && valid) maps[n + i] = inside ? ca : cms[cl];
 }
 
-// box_h then box_v of radius r (gm_box.wgsl:8-25) on map channel blockIdx.z % 5 of src ([5][hc][wc]) into the same
-// channel of dst, for the block's 16 x 16 tile of cells, pair blockIdx.z / 5. The window of clamped rows and columns
-// the tile's taps reach ((16 + 2r)^2 cells, NB x NB blocks of 16 x 16, dynamic LDS) is staged with every load issued
-// before the first store; box_h runs on every window row (a window row is a clamped map row, so its sums are the
-// map's own), box_v on the tile, each sum over its taps in order.
-template <uint32_t NB>
-__global__ __launch_bounds__(kThreads) void gm_box_kernel(const float* src, float* dst, uint32_t hc, uint32_t wc,
-                                                          uint32_t r, size_t wsf) {
-    extern __shared__ float glds[];
-    const uint32_t t = threadIdx.x, x0 = blockIdx.x * kGmT, y0 = blockIdx.y * kGmT, ch = blockIdx.z % 5;
-    src += (size_t)(blockIdx.z / 5) * wsf, dst += (size_t)(blockIdx.z / 5) * wsf;
-    const uint32_t ty = t / kGmT, tx = t % kGmT;
-    const uint32_t span = 2 * r + 1, rows = kGmT + 2 * r;
-    float* win = glds;                // [rows][rows]
-    float* hs = glds + rows * rows;   // [rows][16]
-    const size_t n = (size_t)hc * wc;
-    const float* plane = src + ch * n;
-    const float den = (float)span;
-    float v[NB][NB];
+// One LDS DMA instruction of a dword a lane: the 4 bytes at byte offset `off` of resource r (zeros out of range) into
+// LDS at lds + lane (lds the same for the whole wave). The LDS address-space cast exists only in the device pass.
+__device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t r, float* lds, uint32_t off) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, off, 0, 0, 0);
+#else
+    (void)r, (void)lds, (void)off;
+#endif
+}
+
+// Four neighbouring box sums acc[k] = sum of v(k) .. v(k + 2r) in order, over the values in groups of four (get(b, v):
+// values 4b .. 4b + 3): every value is read once and added to each sum whose window holds it (a value outside adds +0,
+// which leaves a sum as it is: no sum is -0).
+template <class Get>
+__device__ __forceinline__ void box_sum4(uint32_t r, float (&acc)[4], Get get) {
+    const int last = 2 * (int)r;  // value m is in window k for 0 <= m - k <= last
 #pragma unroll
-    for (uint32_t bj = 0; bj < NB; bj++)
+    for (int k = 0; k < 4; k++) acc[k] = 0.0f;
+    for (int m0 = 0; m0 <= last + 3; m0 += 4) {
+        float v[4];
+        get(m0 >> 2, v);
+        if (m0 >= 4 && m0 + 3 <= last) {
 #pragma unroll
-        for (uint32_t bi = 0; bi < NB; bi++) {
-            const uint32_t j = min(ty + kGmT * bj, rows - 1), i = min(tx + kGmT * bi, rows - 1);
-            const int yy = clampi((int)y0 - (int)r + (int)j, 0, (int)hc - 1);
-            const int xx = clampi((int)x0 - (int)r + (int)i, 0, (int)wc - 1);
-            v[bj][bi] = plane[(size_t)yy * wc + xx];
-        }
+            for (int m = 0; m < 4; m++)
 #pragma unroll
-    for (uint32_t bj = 0; bj < NB; bj++)
+                for (int k = 0; k < 4; k++) acc[k] = acc[k] + v[m];
+        } else {
 #pragma unroll
-        for (uint32_t bi = 0; bi < NB; bi++) {
-            const uint32_t j = ty + kGmT * bj, i = tx + kGmT * bi;
-            if (j < rows && i < rows) win[j * rows + i] = v[bj][bi];
-        }
-    __syncthreads();
+            for (int m = 0; m < 4; m++)
 #pragma unroll
-    for (uint32_t bj = 0; bj < NB; bj++) {
-        const uint32_t j = ty + kGmT * bj;
-        if (j < rows) {
-            const float* row = win + j * rows + tx;
-            float acc = 0.0f;
-#pragma unroll 8
-            for (uint32_t d = 0; d < span; d++) acc = acc + row[d];
-            hs[j * kGmT + tx] = acc / den;
+                for (int k = 0; k < 4; k++) acc[k] = acc[k] + (m0 + m >= k && m0 + m - k <= last ? v[m] : 0.0f);
         }
     }
+}
+
+// box_h then box_v of radius r (gm_box.wgsl:8-25) on map channel blockIdx.z % 5 of src ([5][hc][wc]) into the same
+// channel of dst, for the block's 32 x 32 tile of cells, pair blockIdx.z / 5. The window of clamped rows and columns
+// the tile's taps reach ((32 + 2r) x (32 + 2r) cells, the width rounded up to 4) goes into LDS by DMA; box_h runs on
+// every window row (a window row is a clamped map row, so its sums are the map's own), box_v on the tile, each sum over
+// its taps in order. Bound by its adds and LDS reads: a lane forms four neighbouring sums from one pass over their
+// 2r + 4 values (a sum's taps were read one by one), and the tile's halo rows are shared by 32 output rows (by 16): at
+// 544 x 960 cells with r = 20 56 -> 30 us, 8 pairs of 240 x 432 with r = 5 22 -> 18.7 us.
+constexpr uint32_t kBoxW = 32, kBoxH = 32, kBoxPitch = 40;  // the tile's columns; hs's row pitch (a wave's two row groups differ
+                                                // by half the LDS banks)
+inline uint32_t box_lds_floats(uint32_t r) {
+    const uint32_t w = (kBoxW + 2 * r + 3) & ~3u, h = kBoxH + 2 * r;
+    return (w * h + kThreads - 1) / kThreads * kThreads + h * kBoxPitch;
+}
+__global__ __launch_bounds__(kThreads) void gm_box_kernel(const float* src, float* dst, uint32_t hc, uint32_t wc,
+                                                          uint32_t r, size_t wsf) {
+    extern __shared__ __align__(16) float glds[];
+    const uint32_t t = threadIdx.x, x0 = blockIdx.x * kBoxW, y0 = blockIdx.y * kBoxH, ch = blockIdx.z % 5;
+    src += (size_t)(blockIdx.z / 5) * wsf, dst += (size_t)(blockIdx.z / 5) * wsf;
+    const uint32_t w = (kBoxW + 2 * r + 3) & ~3u, h = kBoxH + 2 * r, cells = w * h;
+    const uint32_t rounds = (cells + kThreads - 1) / kThreads;
+    float* win = glds;                      // [h][w], whole rounds of a cell a lane
+    float* hs = glds + rounds * kThreads;   // [h][kBoxPitch]
+    const size_t n = (size_t)hc * wc;
+    const auto plane = buf_rsrc(src + ch * n, (uint32_t)(n * 4));
+    {
+        uint32_t j = t / w, i = t - j * w;
+        const uint32_t dj = kThreads / w, di = kThreads - dj * w;
+        float* to = win + __builtin_amdgcn_readfirstlane(t & ~63u);
+        for (uint32_t k = 0; k < rounds; k++) {
+            const int yy = clampi((int)(y0 + j) - (int)r, 0, (int)hc - 1), xx = clampi((int)(x0 + i) - (int)r, 0, (int)wc - 1);
+            lds_dma4(plane, to + k * kThreads, ((uint32_t)yy * wc + (uint32_t)xx) * 4u);
+            j += dj, i += di;
+            if (i >= w) i -= w, j++;
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's DMA has landed
     __syncthreads();
-    float acc = 0.0f;
-#pragma unroll 8
-    for (uint32_t d = 0; d < span; d++) acc = acc + hs[(ty + d) * kGmT + tx];
-    if (x0 + tx < wc && y0 + ty < hc) dst[ch * n + (size_t)(y0 + ty) * wc + x0 + tx] = acc / den;
+    const float den = (float)(2 * r + 1);
+    for (uint32_t e = t; e < h * (kBoxW / 4); e += kThreads) {
+        const uint32_t row = e / (kBoxW / 4), q = e % (kBoxW / 4);
+        const float4* p = reinterpret_cast<const float4*>(win + row * w) + q;
+        float acc[4];
+        box_sum4(r, acc, [&](int b, float (&v)[4]) {
+            const float4 u = p[b];
+            v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
+        });
+        *reinterpret_cast<float4*>(hs + row * kBoxPitch + 4 * q) =
+            float4{acc[0] / den, acc[1] / den, acc[2] / den, acc[3] / den};
+    }
+    __syncthreads();
+    const uint32_t col = t % kBoxW, q = t / kBoxW;  // kThreads / kBoxW = kBoxH / 4 groups of four rows
+    const float* p = hs + 4 * q * kBoxPitch + col;
+    float acc[4];
+    const uint32_t top = h - 1 - 4 * q;  // the last group may reach past the window: values no sum holds
+    box_sum4(r, acc, [&](int b, float (&v)[4]) {
+#pragma unroll
+        for (uint32_t m = 0; m < 4; m++) v[m] = p[min(4u * (uint32_t)b + m, top) * kBoxPitch];
+    });
+    if (x0 + col < wc) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (y0 + 4 * q + k < hc) dst[ch * n + (size_t)(y0 + 4 * q + k) * wc + x0 + col] = acc[k] / den;
+    }
 }
 
 // the cost cell the select reads for E8 row i (column j): gm_select.wgsl:17-18
@@ -2080,6 +2126,49 @@ __global__ __launch_bounds__(kThreads) void gm_dwin_h_kernel(const float* tex, f
     for (uint32_t d = 0; d < NT; d++)
         if (d < span) acc = acc + v[d];
     hs[t] = acc / (float)span;
+}
+
+// gm_dwin_h_kernel through LDS, where 64 of the select's columns and their windows span at most kDwinCells cells (the
+// E8 grid's spacing of four cells does): a wave per row and 64 columns loads the row's cells once (a sum's taps, four
+// cells apart from lane to lane, were one cache access a pair of lanes each) and its lanes add their taps from LDS, cell c
+// at (c % 4) * 112 + c / 4, so that lanes four cells apart read consecutive banks. At 3 x 544 rows of 240 columns with
+// r = 32 24 -> 5.2 us, 8 pairs of 3 x 240 rows of 108 with r = 7 21.4 -> 5.8 us.
+constexpr uint32_t kDwinCells = 384, kDwinQ = 112;
+__global__ __launch_bounds__(kThreads) void gm_dwin_h_lds_kernel(const float* tex, float* hs, uint32_t hc, uint32_t wc,
+                                                                 uint32_t w8, uint32_t r, uint32_t segs, uint32_t units,
+                                                                 size_t wsf) {
+    __shared__ float cells[kThreads / 64][4 * kDwinQ];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t u = min(blockIdx.x * (kThreads / 64) + wave, units - 1);  // (row, 64 columns); the last one again past it
+    const uint32_t seg = u % segs, rr = u / segs, row = rr % hc, m = rr / hc;
+    tex += blockIdx.y * wsf, hs += blockIdx.y * wsf;
+    const uint32_t j = min(seg * 64 + lane, w8 - 1);
+    const int x = gm_sel_row(j, wc, w8), first = __builtin_amdgcn_readfirstlane(x) - (int)r;  // the wave's first cell
+    const float* src = tex + m * (size_t)hc * wc + (size_t)row * wc;
+    float v[kDwinCells / 64];
+#pragma unroll
+    for (uint32_t k = 0; k < kDwinCells / 64; k++) v[k] = src[clampi(first + (int)(k * 64 + lane), 0, (int)wc - 1)];
+#pragma unroll
+    for (uint32_t k = 0; k < kDwinCells / 64; k++) {
+        const uint32_t c = k * 64 + lane;
+        cells[wave][(c & 3u) * kDwinQ + (c >> 2)] = v[k];
+    }
+    __syncthreads();
+    const uint32_t c0 = (uint32_t)(x - (int)r - first), span = 2 * r + 1;
+    const float* p[4];
+#pragma unroll
+    for (uint32_t f = 0; f < 4; f++) p[f] = cells[wave] + ((c0 + f) & 3u) * kDwinQ + ((c0 + f) >> 2);
+    float acc = 0.0f;
+    uint32_t d = 0;
+#pragma unroll 4
+    for (; d + 4 <= span; d += 4) {
+#pragma unroll
+        for (uint32_t f = 0; f < 4; f++) acc = acc + p[f][d >> 2];
+    }
+#pragma unroll
+    for (uint32_t f = 0; f < 3; f++)
+        if (d + f < span) acc = acc + p[f][d >> 2];
+    if (seg * 64 + lane < w8) hs[(size_t)rr * w8 + j] = acc / (float)span;
 }
 
 // v of lane K of each aligned group of four lanes, in all four (a DPP quad permutation)
@@ -2870,15 +2959,21 @@ int fhc::gmhs_run(const fhc_tensor* a, const fhc_tensor* b, uint32_t h, uint32_t
                            h, w, in(flow), h8, w8, part[1], coef, raw, p.hc, p.wc, wsf);
         // the texture window over the 5 maps (raw -> maps), then the decision window at the cells the select reads
         // (its rows at their columns, its columns at their rows) and the select (maps -> dec, flow)
-        const uint32_t rows = kGmT + 2 * p.r_blk, nb = (rows + kGmT - 1) / kGmT;  // r <= 32: 2 .. 5 blocks a side
-        auto box = nb <= 2 ? gm_box_kernel<2> : nb == 3 ? gm_box_kernel<3> : nb == 4 ? gm_box_kernel<4> : gm_box_kernel<5>;
-        hipLaunchKernelGGL(box, dim3(tiles.x, tiles.y, 5 * pairs), dim3(kThreads), (rows * rows + rows * kGmT) * 4, st,
-                           raw, maps, p.hc, p.wc, p.r_blk, wsf);
+        hipLaunchKernelGGL(gm_box_kernel, dim3((p.wc + kBoxW - 1) / kBoxW, (p.hc + kBoxH - 1) / kBoxH, 5 * pairs),
+                           dim3(kThreads), box_lds_floats(p.r_blk) * sizeof(float), st, raw, maps, p.hc, p.wc, p.r_blk, wsf);
         const bool wide = 2 * p.r_dwin + 1 > 33;
         const uint32_t nh = 3 * p.hc * w8, ne = h8 * w8;
-        hipLaunchKernelGGL(wide ? gm_dwin_h_kernel<65> : gm_dwin_h_kernel<33>,
-                           dim3((nh + kThreads - 1) / kThreads, pairs), dim3(kThreads), 0, st, maps, hs, p.hc, p.wc, w8,
-                           p.r_dwin, nh, wsf);
+        // the columns of 64 lanes lie at most floor(63 wc / w8) + 1 cells apart
+        const uint64_t reach = 63ull * p.wc / w8 + 1 + 2 * p.r_dwin + 1;
+        if (reach <= kDwinCells) {
+            const uint32_t segs = (w8 + 63) / 64, units = 3 * p.hc * segs;
+            hipLaunchKernelGGL(gm_dwin_h_lds_kernel, dim3((units + 3) / 4, pairs), dim3(kThreads), 0, st, maps, hs, p.hc,
+                               p.wc, w8, p.r_dwin, segs, units, wsf);
+        } else {
+            hipLaunchKernelGGL(wide ? gm_dwin_h_kernel<65> : gm_dwin_h_kernel<33>,
+                               dim3((nh + kThreads - 1) / kThreads, pairs), dim3(kThreads), 0, st, maps, hs, p.hc, p.wc, w8,
+                               p.r_dwin, nh, wsf);
+        }
         hipLaunchKernelGGL(wide ? gm_dwin_v_select_kernel<65> : gm_dwin_v_select_kernel<33>,
                            dim3((4 * ne + kThreads - 1) / kThreads, pairs), dim3(kThreads), 0, st, hs, maps, coef,
                            outv(flow), raw, h8, w8, p.hc, p.wc, p.r_dwin, p.eps, p.dmin, p.tex, ne, wsf);

@@ -86,6 +86,8 @@ CASES = [  # network h, w, padded frame width, flow cstride, level
     (192, 256, 256, 4, 1),    # network = frame (s 2: windows 20 and 32, the largest)
     (100, 150, 160, 8, 1),    # ragged: cost grid 50 x 75, flow 12 x 18
     (70, 90, 128, 6, 2),      # level 2 (no jump gate), odd grids
+    (770, 1106, 2208, 8, 1),  # many texture-window tiles, ragged
+    (64, 128, 2048, 8, 1),    # the smallest windows (radius 1)
 ]
 
 
@@ -99,15 +101,17 @@ def test_gmhs_matches_the_oracle(h, w, full_w, cs, level):
     check(a, b, flow, full_w, level, f"random {h}x{w}")
 
 
-def test_gmhs_with_a_coarser_flow_matches_the_oracle():
+@pytest.mark.parametrize("full_w", [256, 512])
+def test_gmhs_with_a_coarser_flow_matches_the_oracle(full_w):
     """A flow grid of 1/16 the network (the select's cells 8 cost cells apart, where the reference's E8 grid puts
-    them 4 apart), at the largest decision window: the select's sampled rows and columns follow the flow's grid."""
+    them 4 apart), at the largest decision window and at half of it: the select's sampled rows
+    and columns follow the flow's grid."""
     say("gmhs coarse flow")
     h, w = 192, 256
     rng = np.random.default_rng(7)
     a = f16(rng.uniform(0, 1, (1, h, w, 4)))
     b = np.roll(a, (3, 2), axis=(1, 2)).copy()
-    check(a, b, smooth_flow(rng, h // 16, w // 16, 4), w, 1, "coarse flow")
+    check(a, b, smooth_flow(rng, h // 16, w // 16, 4), full_w, 1, "coarse flow")
 
 
 def test_gmhs_repairs_the_striped_scene_as_the_oracle():
