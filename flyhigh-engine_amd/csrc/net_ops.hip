@@ -1390,6 +1390,11 @@ __device__ __forceinline__ uint32_t byte_of(uint16_t hv) {
     return (uint32_t)(fminf(fmaxf(h2f(hv), 0.0f), 1.0f) * 255.0f + 0.5f);
 }
 
+// byte_of for a value already clamped to [0, 1]: the product and the sum are exact, so one FMA forms them
+__device__ __forceinline__ uint32_t byte_in01(uint16_t hv) {
+    return (uint32_t)__builtin_fmaf(h2f(hv), 255.0f, 0.5f);
+}
+
 // one lane per padded pixel; VEC4: the output view has 8-byte 4-channel pixels (channel 3 written 0)
 template <bool VEC4>
 __global__ __launch_bounds__(kThreads) void rgba_in_kernel(const uint32_t* src, uint32_t w, uint32_t h, uint32_t pitch,
@@ -1469,23 +1474,39 @@ __device__ __forceinline__ float bil4m(float v00, float v01, float v10, float v1
     const float gx = 1.0f - fx;
     return mac<true>(mac<true>(v11, fx, v10 * gx), fy, mac<true>(v01, fx, v00 * gx) * (1.0f - fy));
 }
-// bil4m<true> with the four taps as f16: each product v * g is written as an FMA with a zero addend (the same value
-// up to the sign of a zero product, which no later step can see), so every conversion folds into a mixed-precision
-// FMA and no tap needs a conversion instruction of its own
-__device__ __forceinline__ float bil4h(_Float16 v00, _Float16 v01, _Float16 v10, _Float16 v11, float fx, float fy) {
-    const float gx = 1.0f - fx;
-    return __builtin_fmaf(__builtin_fmaf((float)v11, fx, __builtin_fmaf((float)v10, gx, 0.0f)), fy,
-                          __builtin_fmaf((float)v01, fx, __builtin_fmaf((float)v00, gx, 0.0f)) * (1.0f - fy));
+// The bilinear sum of four f16 taps with the corner weights g (00, 01, 10, 11), formed once per pixel for all of its
+// channels: four mixed-precision FMAs (the first with a zero addend, the same value up to the sign of a zero product,
+// which no later step can see), so no tap needs a conversion instruction of its own
+__device__ __forceinline__ float bil4h(_Float16 v00, _Float16 v01, _Float16 v10, _Float16 v11, const float (&g)[4]) {
+    return __builtin_fmaf((float)v11, g[3],
+                          __builtin_fmaf((float)v10, g[2],
+                                         __builtin_fmaf((float)v01, g[1], __builtin_fmaf((float)v00, g[0], 0.0f))));
 }
+// The Keys weights (a = -0.75) of the four taps around a sample t past its second tap. In the exact order, the shader's
+// polynomials. With FMA the outer two factored: with u = 1 - t and p = a t u they are p u and p t, 11 operations in all
+// where the four polynomials take 15, and without their cancellation (the largest error over t against 64 bits: outer
+// 6.0e-7 -> 2.2e-8, inner as before, 1.4e-7)
 template <bool FMA>
-__device__ __forceinline__ float cub1m(float x) {
-    if constexpr (!FMA) return cub1(x);
-    return mac<true>(mac<true>(1.25f, x, -2.25f) * x, x, 1.0f);
+__device__ __forceinline__ void keys4(float t, float (&c)[4]) {
+    if constexpr (FMA) {
+        const float u = 1.0f - t, p = (-0.75f * t) * u;
+        c[0] = p * u, c[3] = p * t;
+        c[1] = mac<true>(mac<true>(1.25f, t, -2.25f) * t, t, 1.0f);
+        c[2] = mac<true>(mac<true>(1.25f, u, -2.25f) * u, u, 1.0f);
+    } else {
+        c[0] = cub2(t + 1.0f), c[1] = cub1(t), c[2] = cub1(1.0f - t), c[3] = cub2(2.0f - t);
+    }
 }
+// floor(g) as an integer and g - floor(g). With FMA one instruction each (v_cvt_flr_i32_f32, v_fract_f32, which stays
+// below 1); in the exact order the shader's four
 template <bool FMA>
-__device__ __forceinline__ float cub2m(float x) {
-    if constexpr (!FMA) return cub2(x);
-    return mac<true>(mac<true>(mac<true>(-0.75f, x, 3.75f), x, -6.0f), x, 3.0f);
+__device__ __forceinline__ void floor_split(float g, int& p, float& t) {
+    if constexpr (FMA) {
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(p) : "v"(g));
+        t = __builtin_amdgcn_fractf(g);
+    } else {
+        p = (int)floorf(g), t = g - (float)p;
+    }
 }
 
 // Channel c of the bicubic sum over the 4 x 4 taps t (rows j, columns i) with the weights cx, cy (render.wgsl:
@@ -1505,39 +1526,23 @@ __device__ __forceinline__ float cubic_sum(const uint32_t (&t)[4][4], const floa
 }
 
 // The three channels of one render.wgsl sample (bicubic: :20-47, bilinear: :9-18) of an RGBA8 frame at the sample
-// point (px + tx, py + ty), px, py = floor of its coordinates, each tap converted as rgba_in converts it. INNER: the
-// columns px - 1 .. px + 2 (bicubic) or px, px + 1 (bilinear) all lie inside the frame for every lane of the wave,
-// so one 16- (8-) byte load per row holds the taps in order; otherwise each tap column is clamped to the frame.
-template <bool CUBIC, bool INNER, bool FMA = false>
+// point (px + tx, py + ty), px, py = floor of its coordinates, each tap converted as rgba_in converts it and each tap
+// column clamped to the frame.
+template <bool CUBIC, bool FMA>
 __device__ __forceinline__ void sample_rgba(const uint32_t* src, uint32_t pitch, uint32_t w, uint32_t h, int px,
                                             int py, float tx, float ty, const float* tab, float (&o)[3]) {
     if constexpr (CUBIC) {
-        const float cx[4] = {cub2m<FMA>(tx + 1.0f), cub1m<FMA>(tx), cub1m<FMA>(1.0f - tx), cub2m<FMA>(2.0f - tx)};
-        const float cy[4] = {cub2m<FMA>(ty + 1.0f), cub1m<FMA>(ty), cub1m<FMA>(1.0f - ty), cub2m<FMA>(2.0f - ty)};
+        float cx[4], cy[4];
+        keys4<FMA>(tx, cx), keys4<FMA>(ty, cy);
         uint32_t t[4][4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t yy = (uint32_t)clampi(py - 1 + j, 0, (int)h - 1);
-            if constexpr (INNER) {
-                const u32x4_a4 q = *reinterpret_cast<const u32x4_a4*>(src + (size_t)yy * pitch + (px - 1));
-                t[j][0] = q.x, t[j][1] = q.y, t[j][2] = q.z, t[j][3] = q.w;
-            } else {
-                row_taps4(src, pitch, yy, px, w, t[j]);
-            }
-        }
+        for (int j = 0; j < 4; j++) row_taps4(src, pitch, (uint32_t)clampi(py - 1 + j, 0, (int)h - 1), px, w, t[j]);
 #pragma unroll
         for (int c = 0; c < 3; c++) o[c] = cubic_sum<FMA>(t, cx, cy, tab, c);
     } else {
         uint32_t t0[2], t1[2];
-        const uint32_t ya = (uint32_t)clampi(py, 0, (int)h - 1), yb = (uint32_t)clampi(py + 1, 0, (int)h - 1);
-        if constexpr (INNER) {
-            const u32x2_a4 q0 = *reinterpret_cast<const u32x2_a4*>(src + (size_t)ya * pitch + px);
-            const u32x2_a4 q1 = *reinterpret_cast<const u32x2_a4*>(src + (size_t)yb * pitch + px);
-            t0[0] = q0.x, t0[1] = q0.y, t1[0] = q1.x, t1[1] = q1.y;
-        } else {
-            row_taps2(src, pitch, ya, px, w, t0);
-            row_taps2(src, pitch, yb, px, w, t1);
-        }
+        row_taps2(src, pitch, (uint32_t)clampi(py, 0, (int)h - 1), px, w, t0);
+        row_taps2(src, pitch, (uint32_t)clampi(py + 1, 0, (int)h - 1), px, w, t1);
 #pragma unroll
         for (int c = 0; c < 3; c++)
             o[c] = bil4m<FMA>(unit_tab(tab, t0[0], c), unit_tab(tab, t0[1], c), unit_tab(tab, t1[0], c),
@@ -1551,38 +1556,32 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uin
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
-// sample_rgba's INNER case (every tap column inside the frame for the whole wave) through a buffer resource over
-// the frame: row y's taps at byte offset y * pitch4 + 4 (px - 1) (bicubic) or y * pitch4 + 4 px (bilinear); the same
-// taps, the same arithmetic. ROWS: every tap row inside the frame too for the whole wave, so no row is clamped and
-// row j's offset is the first row's plus the wave-uniform j * pitch4 (the load's scalar offset).
-template <bool CUBIC, bool FMA, bool ROWS = false>
-__device__ __forceinline__ void sample_rgba_inner(__amdgpu_buffer_rsrc_t rs, uint32_t pitch4, int hm1, int px, int py,
+// sample_rgba where every tap column lies inside the frame for the whole wave, through a buffer resource over the
+// frame: the taps are the words at columns col .. col + 3 (bicubic) or col, col + 1 (bilinear) of the rows row .. , one
+// 16- (8-) byte load a row at byte offset y * pitch4 + 4 col; the same taps, the same arithmetic. ROWS: every tap row
+// inside the frame too for the whole wave, so no row is clamped and row j's offset is the first row's plus the
+// wave-uniform j * pitch4 (the load's scalar offset).
+template <bool CUBIC, bool FMA, bool ROWS>
+__device__ __forceinline__ void sample_rgba_inner(__amdgpu_buffer_rsrc_t rs, uint32_t pitch4, int hm1, int col, int row,
                                                   float tx, float ty, const float* tab, float (&o)[3]) {
+    const uint32_t col4 = (uint32_t)col * 4u;
+    const uint32_t row0 = ROWS ? __umul24((uint32_t)row, pitch4) + col4 : 0u;
+    auto at = [&](int j) { return ROWS ? row0 : __umul24((uint32_t)min(max(row + j, 0), hm1), pitch4) + col4; };
+    auto so = [&](int j) { return ROWS ? (uint32_t)j * pitch4 : 0u; };
     if constexpr (CUBIC) {
-        const float cx[4] = {cub2m<FMA>(tx + 1.0f), cub1m<FMA>(tx), cub1m<FMA>(1.0f - tx), cub2m<FMA>(2.0f - tx)};
-        const float cy[4] = {cub2m<FMA>(ty + 1.0f), cub1m<FMA>(ty), cub1m<FMA>(1.0f - ty), cub2m<FMA>(2.0f - ty)};
-        const uint32_t col4 = (uint32_t)(px - 1) * 4u;
-        const uint32_t row0 = ROWS ? __umul24((uint32_t)(py - 1), pitch4) + col4 : 0u;
+        float cx[4], cy[4];
+        keys4<FMA>(tx, cx), keys4<FMA>(ty, cy);
         uint32_t t[4][4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            uint4 q;
-            if constexpr (ROWS) {
-                q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, row0, (uint32_t)j * pitch4, 0));
-            } else {
-                const uint32_t yy = (uint32_t)min(max(py - 1 + j, 0), hm1);
-                q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, __umul24(yy, pitch4) + col4, 0, 0));
-            }
+            const uint4 q = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, at(j), so(j), 0));
             t[j][0] = q.x, t[j][1] = q.y, t[j][2] = q.z, t[j][3] = q.w;
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) o[c] = cubic_sum<FMA>(t, cx, cy, tab, c);
     } else {
-        const uint32_t col4 = (uint32_t)px * 4u;
-        const uint32_t ya = ROWS ? (uint32_t)py : (uint32_t)min(max(py, 0), hm1);
-        const uint32_t yb = ROWS ? (uint32_t)py + 1u : (uint32_t)min(max(py + 1, 0), hm1);
-        const uint2 q0 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, __umul24(ya, pitch4) + col4, 0, 0));
-        const uint2 q1 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, __umul24(yb, pitch4) + col4, 0, 0));
+        const uint2 q0 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, at(0), so(0), 0));
+        const uint2 q1 = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, at(1), so(1), 0));
 #pragma unroll
         for (int c = 0; c < 3; c++)
             o[c] = bil4m<FMA>(unit_tab(tab, q0.x, c), unit_tab(tab, q0.y, c), unit_tab(tab, q1.x, c),
@@ -1590,40 +1589,45 @@ __device__ __forceinline__ void sample_rgba_inner(__amdgpu_buffer_rsrc_t rs, uin
     }
 }
 
-// One frame pixel of render_rgba from its upsampled flow f (x, y for A, then for B, in frame pixels), visibility
-// logits v and residual r: the blend weights, A and B sampled at the displaced positions, the blend, rgba_out.
+// One frame pixel of render_rgba from its sample points f (x, y in A, then in B, in frame pixels, less the first tap's
+// offset: 1 bicubic, 0 bilinear), visibility logits v and residual r: the blend weights, A and B sampled, the blend,
+// rgba_out.
 template <bool CUBIC, bool FL, bool FMA>
 __device__ __forceinline__ void render_rgba_px(uint32_t x, uint32_t y, const float (&f)[4], const float (&v)[3],
                                                const float (&r)[3], const uint32_t* fa, const uint32_t* fb, uint32_t w,
                                                uint32_t h, uint32_t pitch, const float* tab, uint32_t flags,
-                                               uint32_t* dst, uint32_t opitch) {
+                                               uint32_t* dst, uint32_t opitch, uint16_t* pic = nullptr) {
     const float m = fmaxf(v[0], fmaxf(v[1], v[2]));
     float wa_w, wb_w;
     if constexpr (FMA) {  // the hardware exponential and reciprocal (s >= 1: the largest term is exp(0))
         const float e0 = __expf(v[0] - m), e1 = __expf(v[1] - m), e2 = __expf(v[2] - m);
         const float inv = __builtin_amdgcn_rcpf(e0 + e1 + e2);
-        wa_w = (e0 + 0.5f * e2) * inv, wb_w = (e1 + 0.5f * e2) * inv;
+        wa_w = mac<true>(0.5f, e2, e0) * inv, wb_w = mac<true>(0.5f, e2, e1) * inv;
     } else {
         const float e0 = expf(v[0] - m), e1 = expf(v[1] - m), e2 = expf(v[2] - m), s = e0 + e1 + e2;
         wa_w = (e0 + 0.5f * e2) / s, wb_w = (e1 + 0.5f * e2) / s;
     }
-    float ca[3], cb[3];
-    const float gxa = (float)x + f[0], gya = (float)y + f[1], gxb = (float)x + f[2], gyb = (float)y + f[3];
-    const int pxa = (int)floorf(gxa), pya = (int)floorf(gya), pxb = (int)floorf(gxb), pyb = (int)floorf(gyb);
-    const float txa = gxa - (float)pxa, tya = gya - (float)pya, txb = gxb - (float)pxb, tyb = gyb - (float)pyb;
-    const int lo = CUBIC ? 1 : 0, hi = (int)w - (CUBIC ? 3 : 2), hir = (int)h - (CUBIC ? 3 : 2);
-    const bool inner = pxa >= lo && pxa <= hi && pxb >= lo && pxb <= hi;
-    const bool rows = pya >= lo && pya <= hir && pyb >= lo && pyb <= hir;
-    const uint32_t fbytes = ((h - 1) * pitch + w) * 4u, pitch4 = pitch * 4u;
+    float ca[3], cb[3], t[4];
+    int p[4];  // first tap's column and row in A, then in B
+#pragma unroll
+    for (int k = 0; k < 4; k++) floor_split<FMA>(f[k], p[k], t[k]);
+    constexpr int kLo = CUBIC ? 1 : 0, kTaps = CUBIC ? 4 : 2;
+    if constexpr (!FMA) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) p[k] -= kLo;
+    }
+    const uint32_t pitch4 = pitch * 4u, fbytes = ((h - 1) * pitch + w) * 4u;
+    const bool inner = max((uint32_t)p[0], (uint32_t)p[2]) <= w - kTaps;
+    const bool rows = h >= (uint32_t)kTaps && max((uint32_t)p[1], (uint32_t)p[3]) <= h - kTaps;
     if (__all(inner && rows)) {
-        sample_rgba_inner<CUBIC, FMA, true>(buf_rsrc(fa, fbytes), pitch4, (int)h - 1, pxa, pya, txa, tya, tab, ca);
-        sample_rgba_inner<CUBIC, FMA, true>(buf_rsrc(fb, fbytes), pitch4, (int)h - 1, pxb, pyb, txb, tyb, tab, cb);
+        sample_rgba_inner<CUBIC, FMA, true>(buf_rsrc(fa, fbytes), pitch4, (int)h - 1, p[0], p[1], t[0], t[1], tab, ca);
+        sample_rgba_inner<CUBIC, FMA, true>(buf_rsrc(fb, fbytes), pitch4, (int)h - 1, p[2], p[3], t[2], t[3], tab, cb);
     } else if (__all(inner)) {
-        sample_rgba_inner<CUBIC, FMA>(buf_rsrc(fa, fbytes), pitch4, (int)h - 1, pxa, pya, txa, tya, tab, ca);
-        sample_rgba_inner<CUBIC, FMA>(buf_rsrc(fb, fbytes), pitch4, (int)h - 1, pxb, pyb, txb, tyb, tab, cb);
+        sample_rgba_inner<CUBIC, FMA, false>(buf_rsrc(fa, fbytes), pitch4, (int)h - 1, p[0], p[1], t[0], t[1], tab, ca);
+        sample_rgba_inner<CUBIC, FMA, false>(buf_rsrc(fb, fbytes), pitch4, (int)h - 1, p[2], p[3], t[2], t[3], tab, cb);
     } else {
-        sample_rgba<CUBIC, false, FMA>(fa, pitch, w, h, pxa, pya, txa, tya, tab, ca);
-        sample_rgba<CUBIC, false, FMA>(fb, pitch, w, h, pxb, pyb, txb, tyb, tab, cb);
+        sample_rgba<CUBIC, FMA>(fa, pitch, w, h, p[0] + kLo, p[1] + kLo, t[0], t[1], tab, ca);
+        sample_rgba<CUBIC, FMA>(fb, pitch, w, h, p[2] + kLo, p[3] + kLo, t[2], t[3], tab, cb);
     }
     float bwa = wa_w, bwb = wb_w, rk = 1.0f, stillw = 0.0f, own[3] = {0.0f, 0.0f, 0.0f};
     const float third = 1.0f / 3.0f;
@@ -1657,17 +1661,20 @@ __device__ __forceinline__ void render_rgba_px(uint32_t x, uint32_t y, const flo
         bwb = wb_w * (1.0f - k) + (1.0f - pa) * k;
         rk = 1.0f - k;
     }
-    uint32_t bytes[3];
+    uint16_t hv[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         if constexpr (FL) {
             const float mixed = mac<FMA>(r[c], rk, mac<FMA>(cb[c], bwb, ca[c] * bwa));
-            bytes[c] = byte_of(f2h(fminf(fmaxf(mac<FMA>(own[c], stillw, mixed * (1.0f - stillw)), 0.0f), 1.0f)));
+            hv[c] = f2h(fminf(fmaxf(mac<FMA>(own[c], stillw, mixed * (1.0f - stillw)), 0.0f), 1.0f));
         } else {
-            bytes[c] = byte_of(f2h(fminf(fmaxf(mac<FMA>(cb[c], bwb, ca[c] * bwa) + r[c], 0.0f), 1.0f)));
+            hv[c] = f2h(fminf(fmaxf(mac<FMA>(cb[c], bwb, ca[c] * bwa) + r[c], 0.0f), 1.0f));
         }
     }
-    dst[(size_t)y * opitch + x] = bytes[2] | (bytes[1] << 8) | (bytes[0] << 16) | 0xff000000u;
+    if (pic) pic[0] = hv[0], pic[1] = hv[1], pic[2] = hv[2];
+    if (x < w && y < h)  // with pic the lanes cover the padding too
+        dst[(size_t)y * opitch + x] =
+            byte_in01(hv[2]) | (byte_in01(hv[1]) << 8) | (byte_in01(hv[0]) << 16) | 0xff000000u;
 }
 
 // render_pix of the padded frame (hp x wp) from the two RGBA8 frames, written as RGBA8 (rgba_out of the f16 result),
@@ -1679,7 +1686,8 @@ __device__ __forceinline__ void render_rgba_px(uint32_t x, uint32_t y, const flo
 // quotients the reference forms per pixel). FL: flags may be nonzero. Without flags (the engine's default) stillw = 0
 // and rk = 1, so r * rk is r and mixed * (1 - stillw) + own * stillw is mixed (or +0 for a mixed of -0, which the
 // clamp and the byte conversion turn into the same byte 0): that variant leaves those terms out.
-template <bool CUBIC, bool QV, bool FL, bool FMA>
+// PIC: also the f16 picture (hp x wp, its padding included) into pic, image j * per + p.
+template <bool CUBIC, bool QV, bool FL, bool FMA, bool PIC = false>
 // blockIdx.z: generated frame z of `phases` per pair, pair-major (pair p = z / phases, phase j): its frames at
 // p * pstride words past fa and fb, its maps image j * per + p of fl, vis and rt, its output frame j * per + p,
 // ostride words apart (one frame: z = 0)
@@ -1688,35 +1696,41 @@ __global__ __launch_bounds__(kThreads) void render_rgba_kernel(const uint32_t* f
                                                                View fl, View vis, View rt, uint32_t hq, uint32_t wq,
                                                                float fsx, float fsy, uint32_t flags, uint32_t* dst,
                                                                uint32_t opitch, uint64_t pstride, uint32_t per,
-                                                               uint32_t phases, uint64_t ostride) {
+                                                               uint32_t phases, uint64_t ostride, OView pic,
+                                                               uint32_t hp, uint32_t wp) {
     __shared__ float tab[256];
     if (blockIdx.z) {
         const uint32_t p = blockIdx.z / phases, img = (blockIdx.z - p * phases) * per + p;
         fa += p * pstride, fb += p * pstride, dst += img * ostride;
         const size_t q = (size_t)img * hq * wq;
         fl.p += q * fl.cs, vis.p += q * vis.cs, rt.p += q * rt.cs;
+        if constexpr (PIC) pic.p += (size_t)img * hp * wp * pic.cs;
     }
     fill_unit_table(tab);
-    const uint32_t x = blockIdx.x * 64 + (threadIdx.x & 63u), y = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (x >= w || y >= h) return;
+    // a wave is a segment of one row: its row, and what depends on it alone, in scalar registers
+    const uint32_t x = blockIdx.x * 64 + (threadIdx.x & 63u);
+    const uint32_t y = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (x >= (PIC ? wp : w) || y >= (PIC ? hp : h)) return;
     const float iy = ((float)y + 0.5f) * sh - 0.5f, ix = ((float)x + 0.5f) * sw - 0.5f;
-    const int qy0 = (int)floorf(iy), qx0 = (int)floorf(ix);
-    const float qfy = iy - (float)qy0, qfx = ix - (float)qx0;
+    int qy0, qx0;
+    float qfy, qfx;
+    floor_split<FMA>(iy, qy0, qfy), floor_split<FMA>(ix, qx0, qfx);
+    qy0 = __builtin_amdgcn_readfirstlane(qy0);
     const uint32_t y0 = clampi(qy0, 0, (int)hq - 1), y1 = clampi(qy0 + 1, 0, (int)hq - 1);
     const uint32_t x0 = clampi(qx0, 0, (int)wq - 1), x1 = clampi(qx0 + 1, 0, (int)wq - 1);
-    const uint32_t r0 = __umul24(y0, wq), r1 = __umul24(y1, wq);
-    const uint32_t qs[4] = {r0 + x0, r0 + x1, r1 + x0, r1 + x1};
-    float fq[4][4], vq[4][3], rq[4][3];
+    const uint32_t r0 = y0 * wq, r1 = y1 * wq;
     const uint32_t nq = hq * wq;
     const auto rfl = buf_rsrc(fl.p, QV ? nq * 16u : 0u), rrt = buf_rsrc(rt.p, QV ? nq * rt.cs * 2u : 0u);
+    constexpr float kLo = CUBIC ? 1.0f : 0.0f;
     float f[4], v[3], r[3];
     if constexpr (QV && FMA) {  // the taps stay f16 and feed bil4h
+        const uint32_t xs[2] = {x0, x1}, ro[2] = {r0, r1};
         _Float16 hq4[4][8], hr4[4][4];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint4 a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rfl, qs[k] * 16u, 0, 0));
-            const uint2 b =
-                __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rrt, (qs[k] * rt.cs + rt.c0) * 2u, 0, 0));
+        for (int k = 0; k < 4; k++) {  // the map row as the load's scalar offset
+            const uint4 a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rfl, xs[k & 1] * 16u, ro[k >> 1] * 16u, 0));
+            const uint2 b = __builtin_bit_cast(
+                uint2, __builtin_amdgcn_raw_buffer_load_b64(rrt, (__umul24(xs[k & 1], rt.cs) + rt.c0) * 2u, ro[k >> 1] * rt.cs * 2u, 0));
             const uint32_t wv[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
 #pragma unroll
             for (int c = 0; c < 8; c++) hq4[k][c] = __builtin_bit_cast(_Float16, (uint16_t)(wv[c >> 1] >> (16 * (c & 1))));
@@ -1724,17 +1738,21 @@ __global__ __launch_bounds__(kThreads) void render_rgba_kernel(const uint32_t* f
             for (int c = 0; c < 4; c++)
                 hr4[k][c] = __builtin_bit_cast(_Float16, (uint16_t)(wv[4 + (c >> 1)] >> (16 * (c & 1))));
         }
+        const float gy = 1.0f - qfy, gx = 1.0f - qfx, g[4] = {gx * gy, qfx * gy, gx * qfy, qfx * qfy};
+        const float fx = (float)x - kLo, fy = (float)y - kLo;
 #pragma unroll
         for (uint32_t c = 0; c < 4; c++)
-            f[c] = bil4h(hq4[0][c], hq4[1][c], hq4[2][c], hq4[3][c], qfx, qfy) * ((c & 1u) == 0 ? fsx : fsy);
+            f[c] = __builtin_fmaf(bil4h(hq4[0][c], hq4[1][c], hq4[2][c], hq4[3][c], g), c & 1u ? fsy : fsx, c & 1u ? fy : fx);
 #pragma unroll
         for (uint32_t c = 0; c < 3; c++) {
-            v[c] = bil4h(hq4[0][4 + c], hq4[1][4 + c], hq4[2][4 + c], hq4[3][4 + c], qfx, qfy) * vis.scale;
-            r[c] = bil4h(hr4[0][c], hr4[1][c], hr4[2][c], hr4[3][c], qfx, qfy);
+            v[c] = bil4h(hq4[0][4 + c], hq4[1][4 + c], hq4[2][4 + c], hq4[3][4 + c], g) * vis.scale;
+            r[c] = bil4h(hr4[0][c], hr4[1][c], hr4[2][c], hr4[3][c], g);
         }
         render_rgba_px<CUBIC, FL, FMA>(x, y, f, v, r, fa, fb, w, h, pitch, tab, flags, dst, opitch);
         return;
     }
+    const uint32_t qs[4] = {r0 + x0, r0 + x1, r1 + x0, r1 + x1};
+    float fq[4][4], vq[4][3], rq[4][3];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         if constexpr (QV) {
@@ -1755,14 +1773,18 @@ __global__ __launch_bounds__(kThreads) void render_rgba_kernel(const uint32_t* f
         }
     }
 #pragma unroll
-    for (uint32_t c = 0; c < 4; c++)
+    for (uint32_t c = 0; c < 4; c++) {
         f[c] = bil4m<FMA>(fq[0][c], fq[1][c], fq[2][c], fq[3][c], qfx, qfy) * ((c & 1u) == 0 ? fsx : fsy);
+        f[c] = (float)(c & 1u ? y : x) + f[c] - (FMA ? kLo : 0.0f);
+    }
 #pragma unroll
     for (uint32_t c = 0; c < 3; c++) {
         v[c] = bil4m<FMA>(vq[0][c], vq[1][c], vq[2][c], vq[3][c], qfx, qfy) * vis.scale;
         r[c] = bil4m<FMA>(rq[0][c], rq[1][c], rq[2][c], rq[3][c], qfx, qfy);
     }
-    render_rgba_px<CUBIC, FL, FMA>(x, y, f, v, r, fa, fb, w, h, pitch, tab, flags, dst, opitch);
+    uint16_t* to = nullptr;
+    if constexpr (PIC) to = pic.p + ((size_t)y * wp + x) * pic.cs + pic.c0;
+    render_rgba_px<CUBIC, FL, FMA>(x, y, f, v, r, fa, fb, w, h, pitch, tab, flags, dst, opitch, to);
 }
 
 // The antialiased resize of n padded RGBA8 frames (hp x wp, rgba_in's BGR f16) to oh x ow, into a view of 8-byte
@@ -2824,7 +2846,7 @@ namespace {
 int render_rgba_run(const void* a, const void* b, uint64_t pstride, uint32_t pairs, uint32_t phases, uint32_t w,
                     uint32_t h, uint32_t pitch, uint32_t hp, uint32_t wp, const fhc_tensor* flow, const fhc_tensor* vis,
                     const fhc_tensor* rt, uint32_t hq, uint32_t wq, float fsx, float fsy, int cubic, uint32_t flags,
-                    void* out, uint32_t opitch, uint64_t ostride, void* stream) {
+                    void* out, uint32_t opitch, uint64_t ostride, const fhc_tensor* pic, void* stream) {
     return guard(-3, [&]() -> int {
         clear_error();
         if ((uint64_t)h * w * pairs * phases == 0) return 0;
@@ -2841,13 +2863,16 @@ int render_rgba_run(const void* a, const void* b, uint64_t pstride, uint32_t pai
         FHC_TRY(check(flow, "render_rgba flow", 4, false));
         FHC_TRY(check(vis, "render_rgba vis", 3, true));
         FHC_TRY(check(rt, "render_rgba rt", 3, false));
+        if (pic) FHC_TRY(check(pic, "render_rgba pic", 3, false, true));
+        if (pic && !(flags & 4u)) return fail(-1, "render_rgba: the picture comes with the exact f32 order (bit 2)");
         // the tap rows' 32-bit byte offsets (24-bit row multiply) and the quarter maps' buffer sizes
         if ((uint64_t)pitch * 4 >= (1u << 24) || (uint64_t)h * pitch * 4 >= (1u << 31) ||
             (uint64_t)hq * wq * std::max(16u, 2 * rt->cstride) >= (1u << 31) || hq >= (1u << 24) || wq >= (1u << 24))
             return fail(-1, "render_rgba: frame (pitch %u, %u rows) or quarter maps (%u x %u) too large", pitch, h, wq, hq);
         const bool qv = flow->p == vis->p && flow->cstride == 8 && vis->cstride == 8 && flow->c0 == 0 &&
                         vis->c0 == 4 && reinterpret_cast<uintptr_t>(flow->p) % 16 == 0 && vec4(4, {rt});
-        if ((uint64_t)h * w >= kMaxItems || h > 4u * 65535u)
+        const uint32_t gw = pic ? wp : w, gh = pic ? hp : h;
+        if ((uint64_t)gh * gw >= kMaxItems || gh > 4u * 65535u)
             return fail(-1, "render_rgba: %u x %u pixels exceed the launch limits", w, h);
         using K = decltype(&render_rgba_kernel<true, true, true, true>);
         // [exact order][cubic][quarter-map vectors][mode flags]
@@ -2860,12 +2885,18 @@ int render_rgba_run(const void* a, const void* b, uint64_t pstride, uint32_t pai
               {render_rgba_kernel<false, true, false, false>, render_rgba_kernel<false, true, true, false>}},
              {{render_rgba_kernel<true, false, false, false>, render_rgba_kernel<true, false, true, false>},
               {render_rgba_kernel<true, true, false, false>, render_rgba_kernel<true, true, true, false>}}}};
+        static const K ps[2][2][2] = {  // with the picture: exact order
+            {{render_rgba_kernel<false, false, false, false, true>, render_rgba_kernel<false, false, true, false, true>},
+             {render_rgba_kernel<false, true, false, false, true>, render_rgba_kernel<false, true, true, false, true>}},
+            {{render_rgba_kernel<true, false, false, false, true>, render_rgba_kernel<true, false, true, false, true>},
+             {render_rgba_kernel<true, true, false, false, true>, render_rgba_kernel<true, true, true, false, true>}}};
         const uint32_t modes = flags & 3u;
-        hipLaunchKernelGGL(ks[(flags >> 2) & 1u][cubic ? 1 : 0][qv ? 1 : 0][modes ? 1 : 0],
-                           dim3((w + 63) / 64, (h + 3) / 4, pairs * phases), dim3(kThreads), 0, (hipStream_t)stream,
+        hipLaunchKernelGGL((pic ? ps[cubic ? 1 : 0] : ks[(flags >> 2) & 1u][cubic ? 1 : 0])[qv ? 1 : 0][modes ? 1 : 0],
+                           dim3((gw + 63) / 64, (gh + 3) / 4, pairs * phases), dim3(kThreads), 0, (hipStream_t)stream,
                            static_cast<const uint32_t*>(a), static_cast<const uint32_t*>(b), w, h, pitch,
                            (float)hq / (float)hp, (float)wq / (float)wp, in(flow), in(vis), in(rt), hq, wq, fsx, fsy,
-                           modes, static_cast<uint32_t*>(out), opitch, pstride, pairs, phases, ostride);
+                           modes, static_cast<uint32_t*>(out), opitch, pstride, pairs, phases, ostride,
+                           pic ? outv(pic) : OView{nullptr, 0, 0}, hp, wp);
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? 0 : fail(-2, "render_rgba: launch failed: %s", hipGetErrorString(e));
     });
@@ -2877,7 +2908,21 @@ extern "C" int fhc_render_rgba(const void* a, const void* b, uint32_t w, uint32_
                                uint32_t hq, uint32_t wq, float fsx, float fsy, int cubic, uint32_t flags, void* out,
                                uint32_t opitch, void* stream) {
     return render_rgba_run(a, b, 0, 1, 1, w, h, pitch, hp, wp, flow, vis, rt, hq, wq, fsx, fsy, cubic, flags, out,
-                           opitch, 0, stream);
+                           opitch, 0, nullptr, stream);
+}
+
+extern "C" int fhc_render_rgba_pic_n(const void* frames, uint32_t pairs, uint32_t phases, uint32_t w, uint32_t h,
+                                     uint32_t pitch, uint64_t fstride, uint32_t hp, uint32_t wp, const fhc_tensor* flow,
+                                     const fhc_tensor* vis, const fhc_tensor* rt, uint32_t hq, uint32_t wq, float fsx,
+                                     float fsy, int cubic, uint32_t flags, void* out, uint32_t opitch, uint64_t ostride,
+                                     const fhc_tensor* pic, void* stream) {
+    if (pairs && fstride < (uint64_t)pitch * h) {
+        clear_error();
+        return fail(-1, "render_rgba: frame stride below pitch * h");
+    }
+    const void* b = frames ? static_cast<const uint32_t*>(frames) + fstride : nullptr;
+    return render_rgba_run(frames, b, 2 * fstride, pairs, phases, w, h, pitch, hp, wp, flow, vis, rt, hq, wq, fsx, fsy,
+                           cubic, flags, out, opitch, ostride, pic, stream);
 }
 
 extern "C" int fhc_render_rgba_n(const void* frames, uint32_t pairs, uint32_t phases, uint32_t w, uint32_t h,
@@ -2885,13 +2930,8 @@ extern "C" int fhc_render_rgba_n(const void* frames, uint32_t pairs, uint32_t ph
                                  const fhc_tensor* vis, const fhc_tensor* rt, uint32_t hq, uint32_t wq, float fsx,
                                  float fsy, int cubic, uint32_t flags, void* out, uint32_t opitch, uint64_t ostride,
                                  void* stream) {
-    if (pairs && fstride < (uint64_t)pitch * h) {
-        clear_error();
-        return fail(-1, "render_rgba: frame stride below pitch * h");
-    }
-    const void* b = frames ? static_cast<const uint32_t*>(frames) + fstride : nullptr;
-    return render_rgba_run(frames, b, 2 * fstride, pairs, phases, w, h, pitch, hp, wp, flow, vis, rt, hq, wq, fsx, fsy,
-                           cubic, flags, out, opitch, ostride, stream);
+    return fhc_render_rgba_pic_n(frames, pairs, phases, w, h, pitch, fstride, hp, wp, flow, vis, rt, hq, wq, fsx, fsy,
+                                 cubic, flags, out, opitch, ostride, nullptr, stream);
 }
 
 extern "C" int fhc_gmhs_params(uint32_t h, uint32_t w, uint32_t full_w, uint32_t level, fhc_gmhs_par* out) {

@@ -229,6 +229,12 @@ class ComposedChains:
         self.render(V(self.image(full, 0)), V(self.image(full, 1)), flow, vis, rt, V(pic), cubic, flags, fsx, fsy)
         self.rgba_out(V(pic), out_frames)
 
+    def frame_render_pic(self, frames, flow: V, vis: V, rt: V, out_frames, out: V, cubic: bool, flags: int,
+                         phases: int) -> bool:
+        """render_pix of every generated frame at the frames' own padded size and rgba_out, from the frames; False where
+        the caller runs the two ops."""
+        return False
+
     def frame_render_n(self, frames, full, pic, flow: V, vis: V, rt: V, out_frames, hp: int, wp: int, fsx: float,
                        fsy: float, cubic: bool, flags: int, phases: int):
         """frame_render of every generated frame, pair by pair (a pair's phases read the same two frames): phase j of
@@ -578,6 +584,22 @@ class GpuBackend(ComposedChains):
                  lambda: self.fh.render_rgba(fa, fb, vf, vv, vr, hp, wp, cubic, fl, fsx, fsy, out=out_frames,
                                              stream=self.stream),
                  4 * (frames.numel() + out_frames.numel()) + 2 * 10 * self._px(flow))
+
+    def frame_render_pic(self, frames, flow: V, vis: V, rt: V, out_frames, out: V, cubic: bool, flags: int,
+                         phases: int) -> bool:
+        """The network-size mode's render: its samples read from the 8-bit frames (a tap row one 16-byte load, where
+        the f16 pictures take four 8-byte ones), in the reference's f32 order, the bytes beside the picture. 2 million
+        pixels: 43 us, render_pix and rgba_out 60 + 6.5."""
+        _, h, w = frames.shape
+        _, hp, wp, _ = out.buf.shape
+        if not self.chains or w < 4 or w >= 1 << 22 or h * w >= 1 << 29:
+            return False
+        vf, vv, vr, vo = self._v(V(flow.buf, flow.c0)), self._v(vis), self._v(rt), self._v(out)
+        self._go("frame_render (render_pix + rgba_out)",
+                 lambda: self.fh.render_rgba_n(frames, vf, vv, vr, hp, wp, phases, cubic, flags | 4, flow.scale,
+                                               flow.scale, out=out_frames, stream=self.stream, pic=vo),
+                 4 * (frames.numel() * phases + out_frames.numel()) + 2 * 10 * self._px(flow) + 2 * 3 * self._px(out))
+        return True
 
     def frame_render_n(self, frames, full, pic, flow: V, vis: V, rt: V, out_frames, hp: int, wp: int, fsx: float,
                        fsy: float, cubic: bool, flags: int, phases: int):
@@ -960,6 +982,10 @@ class FlyHighFG:
         if self.frame is not None and self.internal:  # the render at the frame size, to the RGBA8 frames
             be.frame_render_n(self.frames, self.full, self.pic, V(self.up7, 0), V(self.up7, 4), V(self.Rt), self.rgba,
                               self.hp, self.wp, self.fsx, self.fsy, self.cubic, self.render_flags, self.M)
+            return
+        # 82 and rgba_out from the frames in one launch where the backend has it, writing the picture too
+        if self.frame is not None and be.frame_render_pic(self.frames, V(self.up7, 0), V(self.up7, 4), V(self.Rt),
+                                                          self.rgba, V(self.out), self.cubic, self.render_flags, self.M):
             return
         for i in (j * P + p for p in range(P) for j in range(self.M)):
             p = i % P

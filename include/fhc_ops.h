@@ -160,6 +160,14 @@ int fhc_render_rgba_n(const void* frames, uint32_t pairs, uint32_t phases, uint3
                       uint64_t fstride, uint32_t hp, uint32_t wp, const fhc_tensor* flow, const fhc_tensor* vis,
                       const fhc_tensor* rt, uint32_t hq, uint32_t wq, float fsx, float fsy, int cubic, uint32_t flags,
                       void* out, uint32_t opitch, uint64_t ostride, void* stream);
+/* fhc_render_rgba_n (flags bit 2 set) that also stores each generated frame's f16 picture (render_pix's result, hp x wp
+ * with the padding, BGR in channels 0-2) as image j * pairs + p of pic (NULL: none): the network-size mode's render and
+ * rgba_out from the frames, bit-identical to rgba_in, fhc_render and fhc_rgba_out in turn. */
+int fhc_render_rgba_pic_n(const void* frames, uint32_t pairs, uint32_t phases, uint32_t w, uint32_t h, uint32_t pitch,
+                          uint64_t fstride, uint32_t hp, uint32_t wp, const fhc_tensor* flow, const fhc_tensor* vis,
+                          const fhc_tensor* rt, uint32_t hq, uint32_t wq, float fsx, float fsy, int cubic,
+                          uint32_t flags, void* out, uint32_t opitch, uint64_t ostride, const fhc_tensor* pic,
+                          void* stream);
 
 /* ---- The graph's op chains, fused. Each computes what its ops compute one after another (the same f32 operations
  * and f16 roundings at the tensors the ops store); no reference counterpart as one call: each replaces the listed

@@ -391,6 +391,35 @@ def test_render_rgba_n_equals_one_call_per_frame(P, M, flags, size):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("P,M,cubic,flags,size", [(1, 1, True, 0, (97, 130)), (2, 2, True, 3, (64, 80)),
+                                                  (1, 2, False, 0, (33, 5))])
+def test_render_rgba_with_pictures_equals_the_ops(P, M, cubic, flags, size):
+    """The render with the f16 pictures beside the bytes (the network-size mode from the frames) against rgba_in, render
+    and rgba_out run one by one on the GPU: pictures (their padding included) and bytes bit-identical."""
+    import torch
+    say("render_rgba pictures", P, M, cubic, flags, size)
+    fh = fhops()
+    rng = np.random.default_rng(size[0] + M)
+    h, w = size
+    hp, wp = (h + 31) // 32 * 32, (w + 31) // 32 * 32
+    hq, wq = hp // 4, wp // 4
+    dfr = dev32(_frames(rng, 2 * P, h, w))
+    up = np.zeros((M * P, hq, wq, 8), np.float32)
+    up[..., :4] = rng.uniform(-9, 9, (M * P, hq, wq, 4))
+    up[..., 4:7] = rng.normal(0, 2, (M * P, hq, wq, 3))
+    dup, drt = dev(f16_bits(up)), dev(rand(rng, (M * P, hq, wq, 4), -0.1, 0.1))
+    pic = torch.full((M * P, hp, wp, 4), -1, dtype=torch.int16, device="cuda")
+    got = host32(fh.render_rgba_n(dfr, dup, fh.View(dup, 4), drt, hp, wp, M, cubic=cubic, flags=flags | 4, pic=pic))
+    full = fh.rgba_in(dfr, hp, wp)
+    for i in range(M * P):
+        p = i % P
+        one = fh.render(full[2 * p:2 * p + 1], full[2 * p + 1:2 * p + 2], dup[i:i + 1], fh.View(dup[i:i + 1], 4),
+                        drt[i:i + 1], cubic=cubic, flags=flags)
+        exact(host(pic[i:i + 1])[..., :3], host(one)[..., :3], f"picture {i}")
+        exact(got[i:i + 1], host32(fh.rgba_out(one, h, w)), f"bytes {i}")
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("cubic,flags,amp,size,qdiv", [(True, 0, 6, (1080, 1920), 9), (False, 0, 6, (1080, 1920), 9),
                                                        (True, 2, 3, (150, 300), 9), (True, 3, 6, (150, 300), 9),
                                                        (False, 3, 2, (97, 130), 9), (True, 0, 40, (97, 130), 9),
