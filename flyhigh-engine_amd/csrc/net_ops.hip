@@ -458,11 +458,11 @@ __global__ __launch_bounds__(kThreads) void interp_aa_kernel(View x, OView out, 
 }
 
 // The same resize for views of at most 4 channels through LDS: a workgroup computes 16 x 16 output pixels from the
-// union of their windows (at most kAaExt x kAaExt input pixels, the host checks the worst tile), staged once with
-// coalesced loads, 4 channels a pixel (one 8-byte LDS read per tap); the L1 then serves no overlapping windows.
-// Staging is a fixed kAaR x kAaR grid of clamped, unconditional loads per lane (lanes past the window rewrite its
-// last row / column with the same values), so it takes one memory round trip. The per-output sum is the one above.
-constexpr uint32_t kAaT = 16, kAaR = 5, kAaExt = kAaT * kAaR;
+// PX x PY input pixels from the first of its windows, staged once with coalesced loads, 4 channels a pixel (one
+// 8-byte LDS read per tap); the L1 then serves no overlapping windows. Staging is a fixed grid of clamped,
+// unconditional loads per lane, so it takes one memory round trip. Rows lie an odd number of cells apart: at a 4x scale
+// a wave's four rows would share their banks otherwise. The per-output sum is the one above.
+constexpr uint32_t kAaT = 16;
 
 // PYR (3 channels, pairs of pictures: images 2k, 2k + 1 are pair k's): the tile's outputs also go through the pair()
 // pyramid (avgpool k 2 twice and the luma, graph.json ops 14-18, 21-24) from LDS: a 16 x 16 tile holds whole 2 x 2
@@ -473,103 +473,128 @@ struct PyrOut {
     OView i8, i16, l16;
 };
 
-// V4: the input view's pixels are 8-byte aligned 4-channel groups (cs and c0 multiples of 4): one load a pixel
-template <int KM, bool PYR, bool V4>
+// One row of KMX taps (f16 cells, channels in halves of .x and .y) into the sums, in the reference's order: each product
+// as an FMA with +0, which takes the f16 tap as it is (one mixed-precision FMA) and gives the product's value, or +0
+// for a product of -0, which the sum cannot tell apart (it starts at +0, and a sum of f32 values is -0 only when both
+// are), then the add
+template <int KMX, int NC>
+__device__ __forceinline__ void aa_row(const uint2 (&q)[KMX], const float (&wx)[KMX], float wy, float (&acc)[4],
+                                       float& norm) {
+#pragma unroll
+    for (int jx = 0; jx < KMX; jx++) {
+        const float wgt = wx[jx] * wy;
+        const float v[4] = {h2f((uint16_t)q[jx].x), h2f((uint16_t)(q[jx].x >> 16)), h2f((uint16_t)q[jx].y),
+                            h2f((uint16_t)(q[jx].y >> 16))};
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[c] = acc[c] + __builtin_fmaf(v[c], wgt, 0.0f);
+        norm = norm + wgt;
+    }
+}
+
+// V4: the input view's pixels are 8-byte aligned 4-channel groups (cs and c0 multiples of 4): one load a pixel. NC: the
+// channels summed (at least c).
+// Bound by VALU issue, 8 instructions a tap: the KMX x KMY taps are those of the scale (5 x 5 where an 8 x 8 form served
+// everything above 4), each a fixed offset from the lane's first, and the LDS is what the taps reach: two 1088 x 1920
+// pictures to 480 x 864 30.4 -> 15.2 us, two of 480 x 864 to 120 x 216 with the pyramid 5.75 -> 6.2, sixteen 23.2 -> 22.4. A tap outside its window has weight +0 and
+// adds +0, as the reference's skipped tap leaves the sums, unless the pixel there is infinite or NaN: a lane whose
+// sums come out so sums again over its window's taps alone.
+template <int KMX, int KMY, int PX, int PY, bool PYR, bool V4, int NC = PYR ? 3 : 4>
 __global__ __launch_bounds__(kThreads) void interp_aa_lds_kernel(View x, OView out, uint32_t ih, uint32_t iw,
                                                                  uint32_t oh, uint32_t ow, uint32_t c,
                                                                  uint32_t tiles_x, uint32_t tiles_y, PyrOut pyr) {
-    // rows of kAaExt + 1 cells: the last cell of each row, and a whole extra row, hold zeros, the value every tap
-    // outside its pixel's window reads (times its weight +0 it adds +0 to the sums, which never hold -0: what the
-    // reference's skipped tap leaves, for any input values)
-    constexpr uint32_t S = kAaExt + 1;
-    __shared__ uint2 tile[S * kAaExt + S];
+    constexpr int RX = (PX + kAaT - 1) / kAaT, RY = (PY + kAaT - 1) / kAaT, P = PX | 1;
+    __shared__ uint2 tile[PY * P];
     __shared__ float qt[PYR ? kAaT * kAaT * 3 : 1], q8[PYR ? 64 * 3 : 1];
+    __shared__ float wxs[kAaT * KMX], wys[kAaT * KMY];
+    __shared__ int lx0[kAaT], ly0[kAaT], ntx[kAaT], nty[kAaT];  // the outputs' first taps in the tile, their numbers
     const uint32_t tid = threadIdx.x, tx = tid % kAaT, ty = tid / kAaT;
     const uint32_t bt = blockIdx.x, txi = bt % tiles_x, r = bt / tiles_x, tyi = r % tiles_y, img = r / tiles_y;
     const uint32_t ox0 = txi * kAaT, oy0 = tyi * kAaT;
-    const uint32_t ox_last = min(ox0 + kAaT, ow) - 1, oy_last = min(oy0 + kAaT, oh) - 1;
     const float sh = (float)ih / (float)oh, sw = (float)iw / (float)ow;
     const float fsh = fmaxf(sh, 1.0f), fsw = fmaxf(sw, 1.0f);
     const int ylo = max(0, (int)floorf(((float)oy0 + 0.5f) * sh - fsh + 0.5f));
-    const int yhi = min((int)ih, (int)floorf(((float)oy_last + 0.5f) * sh + fsh + 0.5f));
     const int xlo = max(0, (int)floorf(((float)ox0 + 0.5f) * sw - fsw + 0.5f));
-    const int xhi = min((int)iw, (int)floorf(((float)ox_last + 0.5f) * sw + fsw + 0.5f));
-    const int ny = max(1, min(yhi - ylo, (int)kAaExt)), nx = max(1, min(xhi - xlo, (int)kAaExt));
-    // the window's first pixel (uniform), then 32-bit byte offsets of the lane's rows and columns (the window is at
-    // most kAaExt pixels square, so row * iw * cs stays far below 2^32 for any frame)
+    // the window's first pixel (uniform), then 32-bit byte offsets of the lane's rows and columns (a few rows of the
+    // picture at most, so row * iw * cs stays far below 2^32 for any frame)
     const char* wbase = reinterpret_cast<const char*>(x.p + (((size_t)img * ih + ylo) * iw + xlo) * x.cs + x.c0);
-    uint32_t roff[kAaR], coff[kAaR];
+    uint32_t roff[RY], coff[RX];
 #pragma unroll
-    for (uint32_t i = 0; i < kAaR; i++) {
-        roff[i] = (uint32_t)min((int)(ty + kAaT * i), ny - 1) * iw * x.cs * 2u;
-        coff[i] = (uint32_t)min((int)(tx + kAaT * i), nx - 1) * x.cs * 2u;
-    }
+    for (uint32_t i = 0; i < RY; i++) roff[i] = min(ty + kAaT * i, ih - 1 - ylo) * iw * x.cs * 2u;
 #pragma unroll
-    for (uint32_t i = 0; i < kAaR; i++)
+    for (uint32_t j = 0; j < RX; j++) coff[j] = min(tx + kAaT * j, iw - 1 - xlo) * x.cs * 2u;
+    uint2 cell[RY][RX];
 #pragma unroll
-        for (uint32_t j = 0; j < kAaR; j++) {
-            const int row = min((int)(ty + kAaT * i), ny - 1), col = min((int)(tx + kAaT * j), nx - 1);
+    for (uint32_t i = 0; i < RY; i++)
+#pragma unroll
+        for (uint32_t j = 0; j < RX; j++) {
             const uint16_t* src = reinterpret_cast<const uint16_t*>(wbase + (roff[i] + coff[j]));
-            if constexpr (V4) {  // channels past c are never read from the tile
-                tile[row * S + col] = *reinterpret_cast<const uint2*>(src);
+            if constexpr (V4) {  // channels past c reach sums that are not stored
+                cell[i][j] = *reinterpret_cast<const uint2*>(src);
             } else {
                 uint16_t v[4];
 #pragma unroll
                 for (uint32_t k = 0; k < 4; k++) v[k] = src[min(k, c - 1)];
-                tile[row * S + col] =
-                    uint2{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)};
+                cell[i][j] = uint2{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)};
             }
         }
-    if (tid < kAaExt) tile[tid * S + kAaExt] = uint2{0u, 0u};  // the zero column
-    if (tid < S) tile[kAaExt * S + tid] = uint2{0u, 0u};       // the zero row
-    // The tap weights and LDS offsets of the tile's columns (threads 0 .. 16 KM - 1: column t / KM, tap t % KM) and
-    // rows (threads 128 ..), computed once for the tile: an invalid column or row (past the output) takes the
-    // clamped pixel's, whose lanes store nothing. A tap outside its pixel's window gets weight 0 and the zero cell.
-    __shared__ float wxs[kAaT * KM], wys[kAaT * KM];
-    __shared__ int lcs[kAaT * KM], lrs[kAaT * KM];
-    if (tid < kAaT * KM) {
-        const uint32_t k = tid / KM, j = tid % KM;
-        const float cx = ((float)min(ox0 + k, ow - 1) + 0.5f) * sw;
-        const int xmin = max(0, (int)floorf(cx - fsw + 0.5f)), xmax = min((int)iw, (int)floorf(cx + fsw + 0.5f));
-        const int xx = xmin + (int)j;
-        wxs[tid] = xx < xmax ? fmaxf(0.0f, 1.0f - fabsf(((float)xx + 0.5f - cx) / fsw)) : 0.0f;
-        lcs[tid] = xx < xmax ? xx - xlo : (int)kAaExt;
-    } else if (tid >= 128 && tid < 128 + kAaT * KM) {
-        const uint32_t k = (tid - 128) / KM, j = (tid - 128) % KM;
-        const float cy = ((float)min(oy0 + k, oh - 1) + 0.5f) * sh;
-        const int ymin = max(0, (int)floorf(cy - fsh + 0.5f)), ymax = min((int)ih, (int)floorf(cy + fsh + 0.5f));
-        const int y = ymin + (int)j;
-        wys[tid - 128] = y < ymax ? fmaxf(0.0f, 1.0f - fabsf(((float)y + 0.5f - cy) / fsh)) : 0.0f;
-        lrs[tid - 128] = y < ymax ? (y - ylo) * (int)S : (int)(kAaExt * S);
+    // The tap weights and first taps of the tile's columns (entries 0 .. 16 KMX - 1) and rows (the rest), computed once
+    // for the tile: an invalid column or row (past the output) takes the clamped pixel's, whose lanes store nothing.
+    for (uint32_t e = tid; e < kAaT * (KMX + KMY); e += kThreads) {
+        const bool rows = e >= kAaT * KMX;
+        const uint32_t k = rows ? (e - kAaT * KMX) / KMY : e / KMX, tap = rows ? (e - kAaT * KMX) % KMY : e % KMX;
+        const uint32_t o = rows ? min(oy0 + k, oh - 1) : min(ox0 + k, ow - 1);
+        const float sc = rows ? sh : sw, fs = rows ? fsh : fsw, cc = ((float)o + 0.5f) * sc;
+        const int n = rows ? (int)ih : (int)iw;
+        const int tmin = max(0, (int)floorf(cc - fs + 0.5f)), tmax = min(n, (int)floorf(cc + fs + 0.5f));
+        const int tt = tmin + (int)tap;
+        const float wgt = tt < tmax ? fmaxf(0.0f, 1.0f - fabsf(((float)tt + 0.5f - cc) / fs)) : 0.0f;
+        if (rows) wys[e - kAaT * KMX] = wgt;
+        else wxs[e] = wgt;
+        if (tap == 0) {
+            if (rows) ly0[k] = tmin - ylo, nty[k] = tmax - tmin;
+            else lx0[k] = tmin - xlo, ntx[k] = tmax - tmin;
+        }
     }
+#pragma unroll
+    for (uint32_t i = 0; i < RY; i++)
+#pragma unroll
+        for (uint32_t j = 0; j < RX; j++) {
+            const uint32_t row = ty + kAaT * i, col = tx + kAaT * j;
+            if ((kAaT * (i + 1) <= PY || row < PY) && (kAaT * (j + 1) <= PX || col < PX)) tile[row * P + col] = cell[i][j];
+        }
     __syncthreads();
     const uint32_t ox = ox0 + tx, oy = oy0 + ty;
     const bool valid = ox < ow && oy < oh;
     if (!PYR && !valid) return;
     // an invalid lane (PYR only: it must reach the barriers) computes a clamped pixel and stores nothing
-    float wx[KM];
-    int lc[KM];
-#pragma unroll
-    for (int j = 0; j < KM; j++) wx[j] = wxs[tx * KM + j], lc[j] = lcs[tx * KM + j];
-    constexpr int NC = PYR ? 3 : 4;  // the channels summed: the pyramid's pictures have 3
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, norm = 0.0f;
+    const uint2* first = tile + ly0[ty] * P + lx0[tx];
+    {
+        float wx[KMX];
 #pragma unroll
-    for (int jy = 0; jy < KM; jy++) {
-        const float wy = wys[ty * KM + jy];
-        const uint2* lrow = tile + lrs[ty * KM + jy];
+        for (int j = 0; j < KMX; j++) wx[j] = wxs[tx * KMX + j];
 #pragma unroll
-        for (int jx = 0; jx < KM; jx++) {
-            const float wgt = wx[jx] * wy;
-            const uint2 q = lrow[lc[jx]];
-            const float v[4] = {h2f((uint16_t)q.x), h2f((uint16_t)(q.x >> 16)), h2f((uint16_t)q.y),
-                                h2f((uint16_t)(q.y >> 16))};
-            // each product as an FMA with +0, which takes the f16 tap as it is (one mixed-precision FMA): the
-            // product's value, or +0 for a product of -0, which the sum cannot tell apart (it starts at +0 and a
-            // sum of f32 values is -0 only when both are)
+        for (int jy = 0; jy < KMY; jy++) {
+            uint2 q[KMX];
 #pragma unroll
-            for (int i = 0; i < NC; i++) acc[i] = acc[i] + __builtin_fmaf(v[i], wgt, 0.0f);
-            norm = norm + wgt;
+            for (int j = 0; j < KMX; j++) q[j] = first[jy * P + j];
+            aa_row<KMX, NC>(q, wx, wys[ty * KMY + jy], acc, norm);
         }
+    }
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < NC; i++) finite &= i >= (int)c || fabsf(acc[i]) < INFINITY;
+    if (!finite) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] = 0.0f;
+        for (int jy = 0; jy < nty[ty]; jy++)
+            for (int jx = 0; jx < ntx[tx]; jx++) {
+                const float wgt = wxs[tx * KMX + jx] * wys[ty * KMY + jy];
+                const uint2 t = first[jy * P + jx];
+                const uint16_t hv[4] = {(uint16_t)t.x, (uint16_t)(t.x >> 16), (uint16_t)t.y, (uint16_t)(t.y >> 16)};
+#pragma unroll
+                for (int i = 0; i < NC; i++) acc[i] = acc[i] + h2f(hv[i]) * wgt;
+            }
     }
     float val[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -614,6 +639,8 @@ __global__ __launch_bounds__(kThreads) void interp_aa_lds_kernel(View x, OView o
     }
 }
 
+constexpr uint32_t kAaExt = 72;  // the most input rows and columns of a tile of interp_aa_lds_kernel (8 taps reach 69)
+
 // Whether interp_aa_lds_kernel's 32-bit byte offsets within a staged window (kAaExt rows of iw pixels) hold.
 bool aa_window_offsets_fit(uint32_t iw, uint32_t cs) { return (uint64_t)kAaExt * iw * cs * 2 < (1ull << 32); }
 
@@ -626,6 +653,20 @@ uint32_t aa_tile_extent(uint32_t in, uint32_t outn) {
         const int lo = std::max(0, (int)floorf(((float)o0 + 0.5f) * s - f + 0.5f));
         const int hi = std::min((int)in, (int)floorf(((float)o1 + 0.5f) * s + f + 0.5f));
         most = std::max(most, hi - lo);
+    }
+    return (uint32_t)most;
+}
+
+// The largest number of input rows (columns) from the first one of a tile of t outputs to the last of the k that each of
+// its outputs reads from its first tap on, from the kernel's f32 formulas.
+uint32_t aa_tile_reach(uint32_t in, uint32_t outn, uint32_t t, uint32_t k) {
+    const float s = (float)in / (float)outn, f = fmaxf(s, 1.0f);
+    int most = 0;
+    for (uint32_t o0 = 0; o0 < outn; o0 += t) {
+        const uint32_t o1 = std::min(o0 + t, outn) - 1;
+        const int lo = std::max(0, (int)floorf(((float)o0 + 0.5f) * s - f + 0.5f));
+        const int hi = std::max(0, (int)floorf(((float)o1 + 0.5f) * s - f + 0.5f));
+        most = std::max(most, hi - lo + (int)k);
     }
     return (uint32_t)most;
 }
@@ -1787,103 +1828,89 @@ __global__ __launch_bounds__(kThreads) void render_rgba_kernel(const uint32_t* f
     render_rgba_px<CUBIC, FL, FMA>(x, y, f, v, r, fa, fb, w, h, pitch, tab, flags, dst, opitch, to);
 }
 
+// The f16 BGR cell of an RGBA8 word: unit_f16 of each byte, each product rounded once (the same f16 for all 256 bytes)
+__device__ __forceinline__ uint2 bgr_cell(uint32_t v) {
+    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+    auto unit = [](uint32_t b) { return (_Float16)__builtin_fmaf((float)b, 1.0f / 255.0f, 0.0f); };
+    const h2v bg = {unit((v >> 16) & 0xffu), unit((v >> 8) & 0xffu)}, r = {unit(v & 0xffu), (_Float16)0.0f};
+    return uint2{__builtin_bit_cast(uint32_t, bg), __builtin_bit_cast(uint32_t, r)};
+}
+
 // The antialiased resize of n padded RGBA8 frames (hp x wp, rgba_in's BGR f16) to oh x ow, into a view of 8-byte
 // 4-channel pixels (channel 3 written 0): rgba_in.wgsl then interp.wgsl:11-45 with antialias, as
-// interp_aa_lds_kernel computes it. A workgroup stages the union of its 16 x 16 outputs' windows, at most
-// EXT x EXT padded pixels (EXT <= 16 * R, the lanes' R x R load stripes covering it), each converted once; the
-// values are those of the f16 picture rgba_in writes, held in LDS as f16: each tap's product is one mixed-precision
-// FMA that takes the f16 value as it is. SPLIT: a staged pixel's B, G in a 4-byte cell and its R in a 2-byte cell of
-// a second array (6 bytes, two reads a tap) rather than one 8-byte cell (one read). The LDS a workgroup holds sets
-// how many share a CU: the 6-byte cells let four 78 x 78 windows share one where three 80 x 80 8-byte windows do
-// not fit. Measured warm: sixteen 2160p frames (10 taps, a 78-pixel window) 334 us in 8-byte cells, 310 us split;
-// two 1080p frames (40 x 40 cells, occupancy bound by waves either way) 12.9 us in 8-byte cells against 14.8 us
-// for an f32 pair plus an f32 (12 bytes, all-f32 arithmetic); with each tap widened one instruction at a time the
-// 8-byte cells were the slower layout (13.1 against 12.8 us, and 379 us at 2160p).
-template <int KM, int R, int EXT, bool SPLIT>
-__global__ __launch_bounds__(kThreads) void rgba_resize_kernel(const uint32_t* src, uint32_t w, uint32_t h,
-                                                               uint32_t pitch, uint64_t fstride, uint32_t ih,
-                                                               uint32_t iw, OView out, uint32_t oh, uint32_t ow,
-                                                               uint32_t tiles_x, uint32_t tiles_y, float sh, float sw) {
-    static_assert(EXT <= kAaT * R, "the load stripes cover the window");
-    using Cell = typename std::conditional<SPLIT, uint32_t, uint2>::type;
-    __shared__ Cell tile[EXT * EXT];
-    __shared__ uint16_t tileb[SPLIT ? EXT * EXT : 1];
-    __shared__ uint16_t tab[256];  // entry b: the f16 bits rgba_in stores for byte b
-    __shared__ float wxs[kAaT * KM], wys[kAaT * KM];
-    __shared__ int lcs[kAaT * KM], lrs[kAaT * KM];
-    const uint32_t tid = threadIdx.x, tx = tid % kAaT, ty = tid / kAaT;
+// interp_aa_lds_kernel computes it. A workgroup stages PX x PY padded pixels from the first of its 16 x TH
+// outputs' windows, each converted once, as f16 cells of 8 bytes; past the windows' union lie further (clamped) frame
+// pixels, so a lane's KMX x KMY cells from its first tap on always hold values in [0, 1], and a tap outside its window
+// (weight +0) adds +0, leaving the sums as the reference's skipped tap leaves them. Bound by VALU issue: 8 instructions
+// a tap. Every tap is therefore a fixed offset from the lane's first (no address arithmetic), the taps of the axes are counted apart and a last row that no lane of the wave uses is skipped.
+// Sixteen 2160p frames (9 x 10 taps) 312 -> 245 us, eight 1440p frames (6 x 6) 78 -> 52, two 1080p frames (5 x 5,
+// bound by the latency of staging, then summing) 14.0 -> 13.7.
+template <int KMX, int KMY, int TH, int PX, int PY>
+__global__ __launch_bounds__(16 * TH) void rgba_resize_kernel(const uint32_t* src, uint32_t w, uint32_t h,
+                                                              uint32_t pitch, uint64_t fstride, uint32_t ih,
+                                                              uint32_t iw, OView out, uint32_t oh, uint32_t ow,
+                                                              uint32_t tiles_x, uint32_t tiles_y, float sh, float sw) {
+    constexpr int NT = 16 * TH, RX = (PX + 15) / 16, RY = (PY + TH - 1) / TH, P = PX | 1;
+    __shared__ uint2 tile[PY * P];
+    __shared__ float wxs[16 * KMX], wys[TH * KMY];
+    __shared__ int lx0[16], ly0[TH];  // the outputs' first taps in the tile
+    const uint32_t tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
     const uint32_t bt = blockIdx.x, txi = bt % tiles_x, rr = bt / tiles_x, tyi = rr % tiles_y, img = rr / tiles_y;
-    const uint32_t ox0 = txi * kAaT, oy0 = tyi * kAaT;
-    const uint32_t ox_last = min(ox0 + kAaT, ow) - 1, oy_last = min(oy0 + kAaT, oh) - 1;
+    const uint32_t ox0 = txi * 16, oy0 = tyi * TH;
     const float fsh = fmaxf(sh, 1.0f), fsw = fmaxf(sw, 1.0f);  // sh = ih / oh, sw = iw / ow from the host
     const int ylo = max(0, (int)floorf(((float)oy0 + 0.5f) * sh - fsh + 0.5f));
-    const int yhi = min((int)ih, (int)floorf(((float)oy_last + 0.5f) * sh + fsh + 0.5f));
     const int xlo = max(0, (int)floorf(((float)ox0 + 0.5f) * sw - fsw + 0.5f));
-    const int xhi = min((int)iw, (int)floorf(((float)ox_last + 0.5f) * sw + fsw + 0.5f));
-    const int ny = max(1, min(yhi - ylo, (int)EXT)), nx = max(1, min(xhi - xlo, (int)EXT));
-    // the tap weights and window indices of the block's 16 columns (entries 0 .. kAaT KM - 1) and 16 rows (the next
-    // kAaT KM): interp_aa.wgsl's per-tap weight, which depends on the output column (row) alone, once per block
-    tab[tid] = unit_f16(tid << 16, 0);
-    for (uint32_t e = tid; e < 2 * kAaT * KM; e += kThreads) {
-        const bool rows = e >= kAaT * KM;
-        const uint32_t k = rows ? e - kAaT * KM : e;
-        const uint32_t o = (rows ? oy0 : ox0) + k / KM;
-        const float sc = rows ? sh : sw, fs = rows ? fsh : fsw;
-        const int n = rows ? (int)ih : (int)iw, lo = rows ? ylo : xlo, nn = rows ? ny : nx;
-        const float c = ((float)o + 0.5f) * sc;
-        const int tmin = max(0, (int)floorf(c - fs + 0.5f)), tmax = min(n, (int)floorf(c + fs + 0.5f));
-        const int tt = tmin + (int)(k % KM);
-        const float wgt = tt < tmax ? fmaxf(0.0f, 1.0f - fabsf(((float)tt + 0.5f - c) / fs)) : 0.0f;
-        const int li = min(max(tt - lo, 0), nn - 1);
-        if (rows) wys[k] = wgt, lrs[k] = li;
-        else wxs[k] = wgt, lcs[k] = li;
-    }
-    __syncthreads();
-    // the frame through a buffer resource: a tap's byte offset is one 24-bit multiply-add
+    // the frame through a buffer resource: a pixel's byte offset is one 24-bit multiply-add
     const auto rf = buf_rsrc(src + img * fstride, ((h - 1) * pitch + w) * 4u);
     const uint32_t pitch4 = pitch * 4u;
+    uint32_t v[RY][RX];
 #pragma unroll
-    for (uint32_t i = 0; i < R; i++)
+    for (uint32_t i = 0; i < RY; i++)
 #pragma unroll
-        for (uint32_t j = 0; j < R; j++) {
-            const int row = min((int)(ty + kAaT * i), ny - 1), col = min((int)(tx + kAaT * j), nx - 1);
-            const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(
-                rf, __umul24((uint32_t)min(ylo + row, (int)h - 1), pitch4) + (uint32_t)min(xlo + col, (int)w - 1) * 4u,
+        for (uint32_t j = 0; j < RX; j++)
+            v[i][j] = __builtin_amdgcn_raw_buffer_load_b32(
+                rf, __umul24(min((uint32_t)ylo + ty + TH * i, h - 1), pitch4) + min((uint32_t)xlo + tx + 16 * j, w - 1) * 4u,
                 0, 0);
-            const uint32_t c01 = (uint32_t)tab[(v >> 16) & 0xffu] | ((uint32_t)tab[(v >> 8) & 0xffu] << 16);
-            if constexpr (SPLIT)
-                tile[row * EXT + col] = c01, tileb[row * EXT + col] = tab[v & 0xffu];
-            else
-                tile[row * EXT + col] = uint2{c01, (uint32_t)tab[v & 0xffu]};
+    // the tap weights and first taps of the block's 16 columns (entries 0 .. 16 KMX - 1) and TH rows (the rest):
+    // interp_aa.wgsl's per-tap weight, which depends on the output column (row) alone, once per block
+    for (uint32_t e = tid; e < 16 * KMX + TH * KMY; e += NT) {
+        const bool rows = e >= 16 * KMX;
+        const uint32_t k = rows ? (e - 16 * KMX) / KMY : e / KMX, tap = rows ? (e - 16 * KMX) % KMY : e % KMX;
+        const float sc = rows ? sh : sw, fs = rows ? fsh : fsw;
+        const float c = ((float)((rows ? oy0 : ox0) + k) + 0.5f) * sc;
+        const int n = rows ? (int)ih : (int)iw;
+        const int tmin = max(0, (int)floorf(c - fs + 0.5f)), tmax = min(n, (int)floorf(c + fs + 0.5f));
+        const int tt = tmin + (int)tap;
+        const float wgt = tt < tmax ? fmaxf(0.0f, 1.0f - fabsf(((float)tt + 0.5f - c) / fs)) : 0.0f;
+        if (rows) wys[e - 16 * KMX] = wgt;
+        else wxs[e] = wgt;
+        if (tap == 0) {  // the clamp: outputs past the last, which store nothing
+            if (rows) ly0[k] = min(max(tmin - ylo, 0), PY - KMY);
+            else lx0[k] = min(max(tmin - xlo, 0), PX - KMX);
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < RY; i++)
+#pragma unroll
+        for (uint32_t j = 0; j < RX; j++) {
+            const uint32_t row = ty + TH * i, col = tx + 16 * j;
+            if ((TH * (i + 1) <= PY || row < PY) && (16 * (j + 1) <= PX || col < PX)) tile[row * P + col] = bgr_cell(v[i][j]);
         }
     __syncthreads();
     const uint32_t ox = ox0 + tx, oy = oy0 + ty;
     if (ox >= ow || oy >= oh) return;
-    float wx[KM];
-    int lc[KM];
+    float wx[KMX];
 #pragma unroll
-    for (int j = 0; j < KM; j++) wx[j] = wxs[tx * KM + j], lc[j] = lcs[tx * KM + j];
-    float acc[3] = {0.0f, 0.0f, 0.0f}, norm = 0.0f;
+    for (int j = 0; j < KMX; j++) wx[j] = wxs[tx * KMX + j];
+    const uint2* first = tile + ly0[ty] * P + lx0[tx];
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, norm = 0.0f;
 #pragma unroll
-    for (int jy = 0; jy < KM; jy++) {
-        const float wy = wys[ty * KM + jy];
-        const uint32_t lrow = lrs[ty * KM + jy] * EXT;
+    for (int jy = 0; jy < KMY; jy++) {
+        uint2 q[KMX];
 #pragma unroll
-        for (int jx = 0; jx < KM; jx++) {
-            // a tap outside the window has weight +0 and a value in [0, 1]: it adds +0, leaving acc and norm as the
-            // reference's skipped tap leaves them (interp_aa_lds_kernel, whose views may hold any value, points such
-            // taps at a zero cell instead)
-            const float wgt = wx[jx] * wy;
-            const Cell q = tile[lrow + lc[jx]];
-            float vv[3];
-            if constexpr (SPLIT) vv[0] = h2f((uint16_t)q), vv[1] = h2f((uint16_t)(q >> 16)), vv[2] = h2f(tileb[lrow + lc[jx]]);
-            else vv[0] = h2f((uint16_t)q.x), vv[1] = h2f((uint16_t)(q.x >> 16)), vv[2] = h2f((uint16_t)q.y);
-            // each product as an FMA with +0, which takes the f16 tap as it is (one mixed-precision FMA, no
-            // widening) and rounds as the product does (taps and weights are >= 0, so no product is -0)
-#pragma unroll
-            for (int i = 0; i < 3; i++) acc[i] = acc[i] + __builtin_fmaf(vv[i], wgt, 0.0f);
-            norm = norm + wgt;
-        }
+        for (int j = 0; j < KMX; j++) q[j] = first[jy * P + j];
+        const float wy = wys[ty * KMY + jy];
+        if (jy + 1 < KMY || __any(wy > 0.0f)) aa_row<KMX, 3>(q, wx, wy, acc, norm);
     }
     *reinterpret_cast<uint2*>(out.p + (((size_t)img * oh + oy) * ow + ox) * out.cs) =
         uint2{(uint32_t)f2h(acc[0] / norm) | ((uint32_t)f2h(acc[1] / norm) << 16), (uint32_t)f2h(acc[2] / norm)};
@@ -2472,13 +2499,28 @@ extern "C" int fhc_interpolate(const fhc_tensor* x, const fhc_tensor* out, uint3
         const uint32_t groups = (c + 3) / 4;
         if (antialias) {
             const uint32_t taps = std::max(aa_taps(ih, oh), aa_taps(iw, ow));
-            if (c <= 4 && taps <= 8 && aa_tile_extent(ih, oh) <= kAaExt && aa_tile_extent(iw, ow) <= kAaExt &&
+            if (c <= 4 && taps <= 8 && aa_tile_reach(ih, oh, kAaT, 8) <= kAaExt && aa_tile_reach(iw, ow, kAaT, 8) <= kAaExt &&
                 aa_window_offsets_fit(iw, x->cstride)) {
                 const uint32_t tx = (ow + kAaT - 1) / kAaT, ty = (oh + kAaT - 1) / kAaT;
                 if ((uint64_t)n * tx * ty >= kMaxItems) return fail(-1, "interpolate: too many tiles");
                 const bool v4 = vec4(4, {x});
-                auto kl = taps <= 4 ? (v4 ? interp_aa_lds_kernel<4, false, true> : interp_aa_lds_kernel<4, false, false>)
-                                    : (v4 ? interp_aa_lds_kernel<8, false, true> : interp_aa_lds_kernel<8, false, false>);
+                // the smallest form whose taps and reach serve the scale (8 taps reach at most 69 pixels); three channels
+                // or fewer of 8-byte pixels are summed apart from four
+                const int f = !v4 ? 0 : c == 4 ? 1 : 2;
+                using KL = decltype(&interp_aa_lds_kernel<8, 8, 72, 72, false, true>);
+                static const KL kls[4][3] = {
+                    {interp_aa_lds_kernel<4, 4, 36, 36, false, false>, interp_aa_lds_kernel<4, 4, 36, 36, false, true>,
+                     interp_aa_lds_kernel<4, 4, 36, 36, false, true, 3>},
+                    {interp_aa_lds_kernel<5, 5, 44, 44, false, false>, interp_aa_lds_kernel<5, 5, 44, 44, false, true>,
+                     interp_aa_lds_kernel<5, 5, 44, 44, false, true, 3>},
+                    {interp_aa_lds_kernel<6, 6, 56, 56, false, false>, interp_aa_lds_kernel<6, 6, 56, 56, false, true>,
+                     interp_aa_lds_kernel<6, 6, 56, 56, false, true, 3>},
+                    {interp_aa_lds_kernel<8, 8, 72, 72, false, false>, interp_aa_lds_kernel<8, 8, 72, 72, false, true>,
+                     interp_aa_lds_kernel<8, 8, 72, 72, false, true, 3>}};
+                auto serves = [&](uint32_t k, uint32_t r) {
+                    return taps <= k && aa_tile_reach(ih, oh, kAaT, k) <= r && aa_tile_reach(iw, ow, kAaT, k) <= r;
+                };
+                const KL kl = kls[serves(4, 36) ? 0 : serves(5, 44) ? 1 : serves(6, 56) ? 2 : 3][f];
                 hipLaunchKernelGGL(kl, dim3(n * tx * ty), dim3(kThreads), 0, (hipStream_t)stream, in(x), outv(out),
                                    ih, iw, oh, ow, c, tx, ty, PyrOut{});
                 const hipError_t e = hipGetLastError();
@@ -2663,7 +2705,7 @@ extern "C" int fhc_pair_input_n(const fhc_tensor* ab, const fhc_tensor* q, const
         FHC_TRY(check(i16, "pair_input i16", 6, false, true));
         FHC_TRY(check(l16, "pair_input l16", 2, false, true));
         const uint32_t taps = std::max(aa_taps(ih, oh), aa_taps(iw, ow));
-        if (!(taps <= 8 && aa_tile_extent(ih, oh) <= kAaExt && aa_tile_extent(iw, ow) <= kAaExt &&
+        if (!(taps <= 8 && aa_tile_reach(ih, oh, kAaT, 8) <= kAaExt && aa_tile_reach(iw, ow, kAaT, 8) <= kAaExt &&
               aa_window_offsets_fit(iw, ab->cstride))) {
             // no one-launch form for this scale: the resize of every picture, then each pair's pyramid
             FHC_TRY(fhc_interpolate(ab, q, 2 * pairs, 3, ih, iw, oh, ow, 1, stream));
@@ -2682,8 +2724,9 @@ extern "C" int fhc_pair_input_n(const fhc_tensor* ab, const fhc_tensor* q, const
         if (oh < 4 || ow < 4) return fail(-1, "pair_input: %u x %u is below 4 x 4", oh, ow);
         const uint32_t tx = (ow + kAaT - 1) / kAaT, ty = (oh + kAaT - 1) / kAaT;
         const bool v4 = vec4(4, {ab});
-        auto kl = taps <= 4 ? (v4 ? interp_aa_lds_kernel<4, true, true> : interp_aa_lds_kernel<4, true, false>)
-                            : (v4 ? interp_aa_lds_kernel<8, true, true> : interp_aa_lds_kernel<8, true, false>);
+        const bool small = taps <= 4 && std::max(aa_tile_reach(ih, oh, kAaT, 4), aa_tile_reach(iw, ow, kAaT, 4)) <= 36;
+        auto kl = small ? (v4 ? interp_aa_lds_kernel<4, 4, 36, 36, true, true> : interp_aa_lds_kernel<4, 4, 36, 36, true, false>)
+                        : (v4 ? interp_aa_lds_kernel<8, 8, 72, 72, true, true> : interp_aa_lds_kernel<8, 8, 72, 72, true, false>);
         if ((uint64_t)2 * pairs * tx * ty >= kMaxItems / kThreads) return fail(-1, "pair_input: too many tiles");
         hipLaunchKernelGGL(kl, dim3(2 * pairs * tx * ty), dim3(kThreads), 0, (hipStream_t)stream, in(ab), outv(q), ih,
                            iw, oh, ow, 3u, tx, ty, PyrOut{outv(i8), outv(i16), outv(l16)});
@@ -2820,24 +2863,33 @@ extern "C" int fhc_rgba_resize(const void* rgba, uint32_t n, uint32_t w, uint32_
         if (taps > 10 || ext > 84)
             return fail(-1, "rgba_resize: %u x %u -> %u x %u needs %u taps, a %u-pixel tile window (at most 10 and 84)",
                         wp, hp, ow, oh, taps, ext);
-        const uint32_t tx = (ow + kAaT - 1) / kAaT, ty = (oh + kAaT - 1) / kAaT;
-        // the 40-pixel window covers the common downscales (1080p to 864 x 480: 39 x 38); 2160p to 864 x 480 takes
-        // 10 taps and a 78 x 76 window (4096 x 2176: 81 columns); the windows above 48 pixels hold 6-byte cells
-        // (78 x 78: 40,096 bytes of LDS with the tables, four workgroups a CU)
-        auto k = ext <= 40 && taps <= 5 ? rgba_resize_kernel<5, 3, 40, false>
-                 : ext <= 3 * kAaT
-                     ? (taps <= 5 ? rgba_resize_kernel<5, 3, 48, false> : taps <= 6 ? rgba_resize_kernel<6, 3, 48, false>
-                                                                        : rgba_resize_kernel<8, 3, 48, false>)
-                 : ext <= 5 * kAaT && taps <= 8
-                     ? (taps <= 6 ? rgba_resize_kernel<6, 5, 80, true> : rgba_resize_kernel<8, 5, 80, true>)
-                 : ext <= 78 ? rgba_resize_kernel<10, 5, 78, true> : rgba_resize_kernel<10, 6, 84, true>;
         if ((uint64_t)pitch * 4 >= (1u << 24) || (uint64_t)h * pitch * 4 >= (1u << 31))
             return fail(-1, "rgba_resize: frames of pitch %u and %u rows are too large", pitch, h);
-        hipLaunchKernelGGL(k, dim3(n * tx * ty), dim3(kThreads), 0, (hipStream_t)stream,
-                           static_cast<const uint32_t*>(rgba), w, h, pitch, fstride, hp, wp, outv(out), oh, ow, tx, ty,
-                           (float)hp / (float)oh, (float)wp / (float)ow);
-        const hipError_t e = hipGetLastError();
-        return e == hipSuccess ? 0 : fail(-2, "rgba_resize: launch failed: %s", hipGetErrorString(e));
+        const uint32_t kx = aa_taps(wp, ow), ky = aa_taps(hp, oh);
+        // by the taps an axis and the pixels a tile's lanes reach: 1080p to 864 x 480 5 x 5 taps and 48 x 48 pixels, 1440p
+        // 6 x 6 and 56 x 56, 2160p 9 x 10 and 80 x 80 (16 rows of outputs 245 us for sixteen frames, 8 rows 270)
+        using K = decltype(&rgba_resize_kernel<5, 5, 16, 48, 48>);
+        struct Form {
+            uint32_t kx, ky, th, px, py;
+            K k;
+        };
+        static const Form forms[] = {{5, 5, 16, 48, 48, rgba_resize_kernel<5, 5, 16, 48, 48>},
+                                     {6, 6, 16, 56, 56, rgba_resize_kernel<6, 6, 16, 56, 56>},
+                                     {8, 8, 16, 72, 72, rgba_resize_kernel<8, 8, 16, 72, 72>},
+                                     {9, 10, 16, 80, 80, rgba_resize_kernel<9, 10, 16, 80, 80>},
+                                     {10, 10, 8, 86, 48, rgba_resize_kernel<10, 10, 8, 86, 48>}};
+        for (const Form& f : forms) {
+            if (kx > f.kx || ky > f.ky || aa_tile_reach(wp, ow, 16, f.kx) > f.px ||
+                aa_tile_reach(hp, oh, f.th, f.ky) > f.py)
+                continue;
+            const uint32_t tx = (ow + 15) / 16, ty = (oh + f.th - 1) / f.th;
+            hipLaunchKernelGGL(f.k, dim3(n * tx * ty), dim3(16 * f.th), 0, (hipStream_t)stream,
+                               static_cast<const uint32_t*>(rgba), w, h, pitch, fstride, hp, wp, outv(out), oh, ow, tx, ty,
+                               (float)hp / (float)oh, (float)wp / (float)ow);
+            const hipError_t e = hipGetLastError();
+            return e == hipSuccess ? 0 : fail(-2, "rgba_resize: launch failed: %s", hipGetErrorString(e));
+        }
+        return fail(-1, "rgba_resize: no form serves %u x %u -> %u x %u", wp, hp, ow, oh);
     });
 }
 
