@@ -282,21 +282,29 @@ __global__ __launch_bounds__(kCvThreads) void convex_tile_kernel(View wt, View x
 }
 
 // ---- film_modulate: shaders/film.wgsl:11-14 ---------------------------------------------------------------------
+// Grid y is the phase: its vectors (one per image of h) and its images of out, whose pixels begin at phase * pixels.
+// VEC: the views and vectors hold 8-byte groups of 4 channels. HBM-bound in its bytes, at 8 pairs x 3 phases of
+// 60 x 108 x 48 some 10 us: the vectors by 2-byte loads 13, a launch a phase 20.
+struct FilmVectors {
+    const uint16_t* g[kMaxPhases];
+};
 template <bool VEC>
-__global__ __launch_bounds__(kThreads) void film_kernel(View hv, const uint16_t* g, OView out, uint32_t hw,
-                                                        uint32_t c, uint32_t groups, uint32_t items) {
+__global__ __launch_bounds__(kThreads) void film_kernel(View hv, FilmVectors g, OView out, uint32_t hw, uint32_t c,
+                                                        uint32_t groups, uint32_t items, uint32_t pixels) {
     const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
     if (t >= items) return;
     const uint32_t pix = t / groups, ch = (t - pix * groups) * 4;
-    const uint16_t* gi = g + (size_t)(pix / hw) * 2 * c;
-    float v[4], o[4];
+    const uint16_t* gi = g.g[blockIdx.y] + (size_t)(pix / hw) * 2 * c;
+    View gv = hv;
+    gv.p = gi, gv.cs = 0, gv.c0 = 0;
+    float v[4], scale[4], shift[4], o[4];
     ld4<VEC>(hv, pix, ch, c, v);
+    ld4<VEC>(gv, 0, ch, c, scale);
+    gv.c0 = c;
+    ld4<VEC>(gv, 0, ch, c, shift);
 #pragma unroll
-    for (uint32_t i = 0; i < 4; i++) {
-        const uint32_t cc = ch + i < c ? ch + i : 0;  // channels past c are not stored
-        o[i] = v[i] * (1.0f + h2f(gi[cc])) + h2f(gi[c + cc]);
-    }
-    st4<VEC>(out, pix, ch, c, o);
+    for (uint32_t i = 0; i < 4; i++) o[i] = v[i] * (1.0f + scale[i]) + shift[i];
+    st4<VEC>(out, blockIdx.y * pixels + pix, ch, c, o);
 }
 
 // ---- blend_weights and blendmix: shaders/blend.wgsl:11-20, blendmix.wgsl:14-27 ------------------------------------
@@ -2421,21 +2429,47 @@ extern "C" int fhc_convex_upsample(const fhc_tensor* wt, const fhc_tensor* x, co
     });
 }
 
+namespace {
+int film_run(const char* op, const fhc_tensor* hv, const FilmVectors& gv, uint32_t phases, const fhc_tensor* out,
+             uint32_t n, uint32_t h, uint32_t w, uint32_t c, void* stream) {
+    FHC_TRY(check(hv, "film_modulate h", c, false));
+    FHC_TRY(check(out, "film_modulate out", c, false, true));
+    const uint32_t groups = (c + 3) / 4;
+    bool v = vec4(c, {hv, out});
+    for (uint32_t j = 0; j < phases; j++) v = v && reinterpret_cast<uintptr_t>(gv.g[j]) % 8 == 0;
+    if ((uint64_t)n * h * w * groups * phases >= kMaxItems) return fail(-1, "%s: too many work items", op);
+    return launch(op, (uint64_t)n * h * w * groups, [&](dim3 g, uint32_t items) {
+        auto k = v ? film_kernel<true> : film_kernel<false>;
+        hipLaunchKernelGGL(k, dim3(g.x, phases), dim3(kThreads), 0, (hipStream_t)stream, in(hv), gv, outv(out), h * w, c,
+                           groups, items, n * h * w);
+    });
+}
+}  // namespace
+
 extern "C" int fhc_film_modulate(const fhc_tensor* hv, const void* gvec, const fhc_tensor* out, uint32_t n,
                                  uint32_t h, uint32_t w, uint32_t c, void* stream) {
     return guard(-3, [&]() -> int {
         clear_error();
         if ((uint64_t)n * h * w * c == 0) return 0;
         if (!gvec) return fail(-1, "film_modulate: null g");
-        FHC_TRY(check(hv, "film_modulate h", c, false));
-        FHC_TRY(check(out, "film_modulate out", c, false, true));
-        const uint32_t groups = (c + 3) / 4;
-        const bool v = vec4(c, {hv, out});
-        return launch("film_modulate", (uint64_t)n * h * w * groups, [&](dim3 g, uint32_t items) {
-            auto k = v ? film_kernel<true> : film_kernel<false>;
-            hipLaunchKernelGGL(k, g, dim3(kThreads), 0, (hipStream_t)stream, in(hv),
-                               static_cast<const uint16_t*>(gvec), outv(out), h * w, c, groups, items);
-        });
+        return film_run("film_modulate", hv, FilmVectors{{static_cast<const uint16_t*>(gvec)}}, 1, out, n, h, w, c, stream);
+    });
+}
+
+extern "C" int fhc_film_modulate_n(const fhc_tensor* hv, const void* const* gvecs, uint32_t phases,
+                                   const fhc_tensor* out, uint32_t n, uint32_t h, uint32_t w, uint32_t c,
+                                   void* stream) {
+    return guard(-3, [&]() -> int {
+        clear_error();
+        if ((uint64_t)n * h * w * c * phases == 0) return 0;
+        if (phases > kMaxPhases) return fail(-1, "film_modulate_n: %u phases (at most %u)", phases, kMaxPhases);
+        if (!gvecs) return fail(-1, "film_modulate_n: null g");
+        FilmVectors gv{};
+        for (uint32_t j = 0; j < phases; j++) {
+            if (!gvecs[j]) return fail(-1, "film_modulate_n: null g of phase %u", j);
+            gv.g[j] = static_cast<const uint16_t*>(gvecs[j]);
+        }
+        return film_run("film_modulate_n", hv, gv, phases, out, n, h, w, c, stream);
     });
 }
 

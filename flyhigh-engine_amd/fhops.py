@@ -66,6 +66,7 @@ def _lib():
             "fhc_sad_volume": [T, T, T, U, U, U, U, P],
             "fhc_convex_upsample": [T, T, T, U, U, U, U, P],
             "fhc_film_modulate": [T, P, T, U, U, U, U, P],
+            "fhc_film_modulate_n": [T, P, U, T, U, U, U, U, P],
             "fhc_blend_weights": [T, T, U, U, U, P],
             "fhc_blendmix": [T, T, T, T, U, U, U, P],
             "fhc_avgpool": [T, T, U, U, U, U, U, P],
@@ -177,6 +178,20 @@ def film(hv, g, c: Optional[int] = None, out=None, stream=None):
     _run("film_modulate",
          _lib().fhc_film_modulate(_ref(hv), g.data_ptr(), _ref(o), n, h, w, c, _stream_handle(stream)))
     return o.t
+
+
+def film_phases(hv, gs, c, out, stream=None):
+    """film(hv, g, c) of each phase's vectors g in gs (at most 8), phase j's images at j * n .. of out: one launch."""
+    hv = _v(hv)
+    n, h, w, _ = hv.shape
+    for g in gs:
+        if not g.is_contiguous() or g.numel() != n * 2 * c or g.element_size() != 2:
+            raise FhcError(f"film_phases: each g needs {n * 2 * c} contiguous f16 values")
+    o = _v(out)
+    if o.shape[0] != n * len(gs):
+        raise FhcError(f"film_phases: out holds {o.shape[0]} images for {len(gs)} phases of {n}")
+    arr = (ctypes.c_void_p * len(gs))(*(g.data_ptr() for g in gs))
+    _run("film_modulate", _lib().fhc_film_modulate_n(_ref(hv), arr, len(gs), _ref(o), n, h, w, c, _stream_handle(stream)))
 
 
 def blend(vis, out=None, stream=None):

@@ -63,6 +63,10 @@ int fhc_convex_upsample(const fhc_tensor* wt, const fhc_tensor* x, const fhc_ten
  * "film_modulate" arm (net/build.rs:360-363). */
 int fhc_film_modulate(const fhc_tensor* hv, const void* g, const fhc_tensor* out, uint32_t n, uint32_t h,
                       uint32_t w, uint32_t c, void* stream);
+/* fhc_film_modulate of the same h for each of `phases` phases (at most 8) in one launch: g[j] (a host array of device
+ * pointers, read during the call) holds phase j's n vectors, and its images are j * n .. of out (phases * n images). */
+int fhc_film_modulate_n(const fhc_tensor* hv, const void* const* g, uint32_t phases, const fhc_tensor* out, uint32_t n,
+                        uint32_t h, uint32_t w, uint32_t c, void* stream);
 
 /* Visibility blend weights: the softmax (p0, p1, p2) of 3 logits -> 2 channels (p0 + p2 / 2, p1 + p2 / 2). The
  * scale applies. Replaces Gpu::blend (ops/network.rs:63-68, shaders/blend.wgsl:9-21), "blend_weights" unfused. */

@@ -144,6 +144,20 @@ def test_film_modulate_matches_oracle(n, h, w, c, cs, c0):
     exact(got, want, "film")
 
 
+@pytest.mark.parametrize("n,h,w,c,cs,c0,phases", [(1, 60, 108, 48, 48, 0, 2), (3, 13, 17, 48, 52, 4, 3),
+                                                  (2, 5, 7, 7, 11, 3, 8), (1, 1, 1, 1, 1, 0, 2)])
+def test_film_phases_match_oracle(n, h, w, c, cs, c0, phases):
+    say("film_phases", n, h, w, c, cs, c0, phases)
+    fh = fhops()
+    rng = np.random.default_rng(n * h * w + c + phases)
+    hv, gs = rand(rng, (n, h, w, cs), -3, 3), [rand(rng, (n, 2 * c), -1, 1) for _ in range(phases)]
+    out, gd = dev(rand(rng, (phases * n, h, w, c), -1, 1)), [dev(g) for g in gs]
+    if phases == 3:  # one phase's vectors off 8-byte alignment
+        gd[1] = dev(np.concatenate([gs[1].ravel()[:1], gs[1].ravel()]))[1:]
+    fh.film_phases(fh.View(dev(hv), c0), gd, c, out)
+    exact(host(out), np.concatenate([oracle.film(hv, g, c, c0=c0) for g in gs]), "film_phases")
+
+
 @pytest.mark.parametrize("n,h,w,cs,c0,scale", [(1, 120, 216, 3, 0, 1.0), (2, 13, 17, 7, 4, 2.0),
                                                 (1, 60, 108, 5, 2, 0.5)])
 def test_blend_weights_and_blendmix_match_oracle(n, h, w, cs, c0, scale):
