@@ -652,14 +652,21 @@ constexpr uint32_t kAaExt = 72;  // the most input rows and columns of a tile of
 // Whether interp_aa_lds_kernel's 32-bit byte offsets within a staged window (kAaExt rows of iw pixels) hold.
 bool aa_window_offsets_fit(uint32_t iw, uint32_t cs) { return (uint64_t)kAaExt * iw * cs * 2 < (1ull << 32); }
 
+// (int)floorf(v) of a value in int's range without the library call (these run for every output row and column on each
+// call)
+inline int floor_int(float v) {
+    const int i = (int)v;
+    return i - (v < (float)i);
+}
+
 // The largest input extent (rows or columns) of any kAaT-output tile's windows, from the kernel's f32 formulas.
 uint32_t aa_tile_extent(uint32_t in, uint32_t outn) {
     const float s = (float)in / (float)outn, f = fmaxf(s, 1.0f);
     int most = 0;
     for (uint32_t o0 = 0; o0 < outn; o0 += kAaT) {
         const uint32_t o1 = std::min(o0 + kAaT, outn) - 1;
-        const int lo = std::max(0, (int)floorf(((float)o0 + 0.5f) * s - f + 0.5f));
-        const int hi = std::min((int)in, (int)floorf(((float)o1 + 0.5f) * s + f + 0.5f));
+        const int lo = std::max(0, floor_int(((float)o0 + 0.5f) * s - f + 0.5f));
+        const int hi = std::min((int)in, floor_int(((float)o1 + 0.5f) * s + f + 0.5f));
         most = std::max(most, hi - lo);
     }
     return (uint32_t)most;
@@ -672,8 +679,8 @@ uint32_t aa_tile_reach(uint32_t in, uint32_t outn, uint32_t t, uint32_t k) {
     int most = 0;
     for (uint32_t o0 = 0; o0 < outn; o0 += t) {
         const uint32_t o1 = std::min(o0 + t, outn) - 1;
-        const int lo = std::max(0, (int)floorf(((float)o0 + 0.5f) * s - f + 0.5f));
-        const int hi = std::max(0, (int)floorf(((float)o1 + 0.5f) * s - f + 0.5f));
+        const int lo = std::max(0, floor_int(((float)o0 + 0.5f) * s - f + 0.5f));
+        const int hi = std::max(0, floor_int(((float)o1 + 0.5f) * s - f + 0.5f));
         most = std::max(most, hi - lo + (int)k);
     }
     return (uint32_t)most;
@@ -686,7 +693,7 @@ uint32_t aa_taps(uint32_t in, uint32_t outn) {
     int most = 0;
     for (uint32_t o = 0; o < outn; o++) {
         const float cc = ((float)o + 0.5f) * s;
-        const int lo = std::max(0, (int)floorf(cc - f + 0.5f)), hi = std::min((int)in, (int)floorf(cc + f + 0.5f));
+        const int lo = std::max(0, floor_int(cc - f + 0.5f)), hi = std::min((int)in, floor_int(cc + f + 0.5f));
         most = std::max(most, hi - lo);
     }
     return (uint32_t)most;
