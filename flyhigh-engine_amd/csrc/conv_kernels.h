@@ -30,7 +30,7 @@ struct ConvKArgs {
     int tiles_x, tiles_y, ntn;  // output tiles: columns of 16, rows of TH, channel tiles of BN
     int chunks_per_split;       // global split-K: chunks handled by one z
     int np;                     // output channels padded to ntn * BN
-    int xvec, yvec, rvec;       // vector paths: 16-byte input loads, 8-byte output stores / residual loads
+    int xvec, yvec, rvec;       // vector paths: 16-byte aligned input groups, 8-byte output stores / residual loads
                                 // (rvec also needs cout % 4 == 0)
     int post;                   // 1: the f16 output goes through affine_out, 2 / (1 + exp(-v)) - 1, rounded again
                                 // (the one-tile pair kernel's second conv, cout <= 4, no residual)

@@ -244,8 +244,8 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
     };
 
     // the halo of tile t, staged in registers: element e = tid + i*NT is 8 channels (group g) of halo pixel pix.
-    // MODE 1: 16-byte loads; MODE 0: 2-byte loads at clamped addresses. (MODE 2 and 3, the persistent loop without
-    // and with a residual, have their own buffer-instruction versions below.)
+    // 16-byte loads, in MODE 0 at the view's own alignment (load_group). (MODE 2 and 3, the persistent loop without and
+    // with a residual, have their own buffer-instruction versions below.)
     uint4 pre[NLD];
     // the input resource of the persistent loop spans the full strided extent (n*h*w*xcs halves, which the input
     // buffer holds): a 16-byte group that crossed the resource's end would read zeros, valid channels included
@@ -786,7 +786,7 @@ inline bool buffer_path_ok(const ConvKArgs& a) {
 }
 
 // Launches a persistent configuration on its resident grid when the views allow the buffer loop, else one
-// workgroup per tile, with 16-byte input loads when the input view is 16-byte aligned.
+// workgroup per tile, its input loads by the view's alignment.
 template <int KS, int S, int CIN32, int FM, int WM, int WN, int NA, int WK, bool PERSIST>
 hipError_t launch_direct(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     (void)lds;
