@@ -470,7 +470,9 @@ uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
         }
     }
     if (loop && b >= 2 && d.stride == 2) {
-        if (c == 32 && b >= 3 && px >= 60000) return dir(2, 2, 4, 1, 1);  // 32 -> 64 at 130,560 px: 15.1 against 19
+        // one wave row of 4 rows: each weight load feeds four rows. 32 -> 64 at 64,000 px: 8.8 against 9.6 on two wave
+        // rows of 2, at 130,560 14.7 against 15.1 (19 on one tile a workgroup); 32 -> 96 at 155,520 21.9 against 23.8
+        if (c == 32 && b >= 3 && px >= 60000) return dir(4, 1, 4, 1, 1);
         if (c == 64 && (b == 2 ? px >= 60000 : work >= 120000))            // 64 -> 96 at 113,430 px: 27.4 against 47.3
             return dir(2, 2, b == 2 ? 2 : 4, 1, 1);
     }
