@@ -213,6 +213,9 @@ bool pairs_view(const fhc_conv_desc& d) {
     return d.x_cstride % 2 == 0 && d.x_c0 % 2 == 0 && d.cin % 2 == 0 && d.cin >= 8;
 }
 
+// Whether the deep-layer kernel's 32-bit buffer offsets reach every byte of the input view
+bool input_in_reach(const fhc_conv_desc& d) { return (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31); }
+
 // The direct kernel's launch geometry for configuration `idx`: input channels padded to 32 in one pass, weights
 // resident; one workgroup per spatial tile (grid x) and channel tile (grid y). False if it does not serve the conv.
 bool configure_direct(fhc_conv_plan& p, int idx, std::string* why) {
@@ -359,7 +362,7 @@ bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why, bo
         *why = "the deep-layer configuration serves 3x3 convs of stride " + std::to_string(c.s) + " only";
         return false;
     }
-    if (((d.x_cstride % 8 || d.x_c0 % 8) && !(pairs && pairs_view(d))) || (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 >= (1ull << 31)) {
+    if (((d.x_cstride % 8 || d.x_c0 % 8) && !(pairs && pairs_view(d))) || !input_in_reach(d)) {
         *why = "the deep-layer kernel needs an input view of 16-byte channel groups below 2^31 bytes";
         return false;
     }
@@ -510,7 +513,7 @@ uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
     if (c == 160 || c == 288) {
         if (b == 1 && (c == 160 || px < 60000)) return dir(2, 1, 1, 3);  // 279 -> 12 at 4,158 px: 6.8 against 12.1
         if (c == 160 && (b == 2 || b == 3) && px < 7000) return dir(2, 1, b, 3);  // 155 -> 24 at 4,230 px: 5.1 against 8.7
-        if (in16) {
+        if (in16 && input_in_reach(d)) {
             if (b <= 2 && px >= 60000) return gemm(2);  // 155 -> 32 at 60,000 px and up: 1.0 to 1.4
             if (b == 4 && px >= 7000) return gemm(12);  // 279 -> 64: 1.0 to 1.6
             if (b >= 7 && px >= (c == 160 ? 7000u : 60000u)) return gemm(12);  // 155 -> 128 at 145,992 px: 101 against 128
@@ -567,8 +570,7 @@ constexpr int kGemmDefault = 11;
 // 76. Then the direct kernel whenever a configuration serves the input channels, then the deep-layer kernel from 64
 // input channels, else the chunked kernel.
 uint32_t general_code(const fhc_conv_desc& d, const Geometry& g, bool pairs) {
-    const bool deep = d.kh == 3 && d.stride == 1 && d.cin >= 64 &&
-                      (uint64_t)d.n * d.h * d.w * d.x_cstride * 2 < (1ull << 31);
+    const bool deep = d.kh == 3 && d.stride == 1 && d.cin >= 64 && input_in_reach(d);
     const bool gemm_ok = deep && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0;
     if ((gemm_ok || (deep && pairs && pairs_view(d))) && d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096)
         return make_code(kGemmDefault, 1, 3);

@@ -131,6 +131,15 @@ def test_direct_kernel_where_the_channels_fit():
     assert d["family"] == "direct" and d["cc"] == 64 and d["tile_channels"] == 48 and d["ntn"] == 1
 
 
+# (batch, cin, cout, input channel stride): 544 x 960 tensors of 2^31 bytes and more, past the deep-layer kernel's reach
+@pytest.mark.parametrize("n,cin,cout,cs", [(24, 155, 48, 160), (16, 155, 64, 160), (24, 155, 128, 160), (16, 279, 32, 288),
+                                           (8, 279, 128, 288), (16, 96, 48, 160)])
+def test_tensors_past_the_deep_layer_kernels_reach_keep_the_direct_kernel(n, cin, cout, cs):
+    d = fhconv.make_desc(n, 544, 960, cin, cout, x_cstride=cs)
+    assert n * 544 * 960 * cs * 2 >= 2 ** 31
+    assert fhconv.plan_dry(d)["family"] == "direct"
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_mi355x_plan_covers_the_output(shape):
     n, h, w, cin, cout, k, s = shape
