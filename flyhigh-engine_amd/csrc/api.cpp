@@ -350,8 +350,8 @@ bool configure_igemm(fhc_conv_plan& p, int cfg, uint32_t ks, std::string* why) {
 // The deep-layer kernel's launch geometry for configuration `idx` and global split `ks`: chunks of CK input
 // channels (the packed weights of the chunked layout with cc = CK), one workgroup per spatial tile (grid x), channel
 // tile (grid y) and split (grid z). False if it does not serve the conv: 3x3 of its stride, an input view of
-// 16-byte groups (with `pairs` also of channel pairs) below 2^31 bytes, at least `ks` chunks.
-bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why, bool pairs = false) {
+// 16-byte groups or of channel pairs below 2^31 bytes, at least `ks` chunks.
+bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why) {
     const fhc_conv_desc& d = p.d;
     if (idx < 0 || idx >= kNumGemm) {
         *why = "unknown deep-layer configuration";
@@ -362,8 +362,9 @@ bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why, bo
         *why = "the deep-layer configuration serves 3x3 convs of stride " + std::to_string(c.s) + " only";
         return false;
     }
-    if (((d.x_cstride % 8 || d.x_c0 % 8) && !(pairs && pairs_view(d))) || !input_in_reach(d)) {
-        *why = "the deep-layer kernel needs an input view of 16-byte channel groups below 2^31 bytes";
+    if (((d.x_cstride % 8 || d.x_c0 % 8) && !pairs_view(d)) || !input_in_reach(d)) {
+        *why = "the deep-layer kernel needs an input view of 16-byte channel groups, or of channel pairs with an even "
+               "cin of at least 8, below 2^31 bytes";
         return false;
     }
     LaunchFn fn = gemm_launcher(idx, nullptr);
@@ -412,9 +413,7 @@ bool configure_gemm(fhc_conv_plan& p, int idx, uint32_t ks, std::string* why, bo
 int heuristic_cfg(const fhc_conv_desc& d, const Geometry& g);
 void* static_scratch(int dev);
 
-// pairs: the deep-layer kernel may read a view of channel pairs (the planner's own choice; a variant that the caller
-// or the table names is held to views of 16-byte groups)
-bool configure(fhc_conv_plan& p, const Variant& v, std::string* why, bool pairs = false) {
+bool configure(fhc_conv_plan& p, const Variant& v, std::string* why) {
     if (v.family == 1) {
         if (v.ks > 1) {
             *why = "the direct kernel has no split-K";
@@ -422,7 +421,7 @@ bool configure(fhc_conv_plan& p, const Variant& v, std::string* why, bool pairs 
         }
         return configure_direct(p, v.cfg, why);
     }
-    if (v.family == 3) return configure_gemm(p, v.cfg, v.ks, why, pairs);
+    if (v.family == 3) return configure_gemm(p, v.cfg, v.ks, why);
     return configure_igemm(p, v.cfg, v.ks, why);
 }
 
@@ -746,7 +745,6 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
     p.g.cin8 = div_ceil(d.cin, 8) * 8;
     // the choice: forced variant, then the table, then the heuristic (conv_pick, autotune.rs:186-233)
     Variant v{};
-    bool own = false;  // the planner's own choice
     if (d.variant != 0) {
         if (!decode_code(d.variant, &v)) {
             *why = "unknown variant " + std::to_string(d.variant);
@@ -754,7 +752,7 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
         }
     } else {
         const int hit = fhc_tune_get_ex(d.cin, d.cout, d.h, d.w, d.stride, d.n, d.kh);
-        if (hit < 0 || !decode_code((uint32_t)hit, &v)) own = decode_code(heuristic_code(d, p.g), &v);
+        if (hit < 0 || !decode_code((uint32_t)hit, &v)) decode_code(heuristic_code(d, p.g), &v);
     }
     // a forced split (or the reference code's split nibble, candidates.rs:4) moves to the chunked kernel
     uint32_t ks = 0;
@@ -775,7 +773,7 @@ bool plan_choose(const fhc_conv_desc& d, fhc_conv_plan& p, std::string* why) {
             v.ks = ks;
         }
     }
-    if (!configure(p, v, why, own)) {
+    if (!configure(p, v, why)) {
         // a table entry or heuristic that does not fit this shape falls back to the chunked 4-row tile
         const uint32_t code = variant_code(v);
         if (d.variant != 0 || !configure(p, Variant{0, d.cout <= 32 ? 5 : 4, v.family == 1 ? 1u : v.ks}, why)) {

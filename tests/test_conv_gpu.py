@@ -499,6 +499,23 @@ def test_gemm_variants_match_the_oracle(shape):
         assert np.array_equal(got[..., mask], c.y0[..., mask])
 
 
+# views of channel pairs: a partial last group of 2, 4 and 6 channels and none, chunks of 32 and 64, splits
+@pytest.mark.parametrize("shape,xv", [((1, 19, 33, 130, 48, 1), (130, 0)), ((2, 13, 20, 100, 64, 1), (106, 4)),
+                                      ((1, 9, 18, 78, 96, 1), (82, 2)), ((1, 12, 35, 96, 20, 1), (98, 2))],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_gemm_variants_on_channel_pairs_match_the_oracle(shape, xv):
+    n, h, w, cin, cout, _ = shape
+    c = Case(n, h, w, cin, cout, act=1, residual=True, xv=xv, poison=xv[0] > cin, seed=cin)
+    want = c.run_oracle(threads=8)
+    codes = [k for k in fhconv.variant_list(c.fhc_desc()) if fhconv.variant_name(k).startswith("gemm")]
+    assert codes
+    for code in codes:
+        got = c.run_gpu(variant=code)
+        say("gemm pairs", shape, fhconv.variant_name(code))
+        ok, md, mref = parity(got, want)
+        assert ok, (fhconv.variant_name(code), md, mref)
+
+
 def test_gemm_variant_unaligned_input_falls_back():
     # an input pointer off 16-byte alignment cannot take the LDS DMA: the launcher runs the chunked kernel on the
     # same packed weights instead, with and without a split

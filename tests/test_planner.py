@@ -177,6 +177,27 @@ def test_variant_list_and_forced_variants():
         fhconv.plan_dry(fhconv.make_desc(1, 68, 120, 128, 128, variant=31))
 
 
+@pytest.mark.parametrize("cin,cs,c0", [(130, 130, 0), (100, 102, 2), (258, 262, 4)])
+def test_a_view_of_channel_pairs_takes_its_own_plans_code(cin, cs, c0):
+    # the deep-layer kernel reads views of channel pairs by dword-aligned loads, so its codes are listed (and timed by
+    # autotune) on them, can be forced and stay what they are when the table names them; an odd view has none
+    shape, view = (2, 47, 51, cin, 68), dict(x_cstride=cs, x_c0=c0)
+    fhconv.tune_clear()
+    try:
+        codes = {c: fhconv.variant_name(c) for c in fhconv.variant_list(fhconv.make_desc(*shape, **view))}
+        deep = [c for c in codes if codes[c].startswith("gemm")]
+        assert deep and fhconv.plan_dry(fhconv.make_desc(*shape, **view))["variant"] in codes
+        for code in deep:
+            assert fhconv.plan_dry(fhconv.make_desc(*shape, variant=code, **view))["variant"] == code
+            fhconv.parse_tune(f"{cin},68,47,51,1,2,3={code}")
+            assert fhconv.plan_dry(fhconv.make_desc(*shape, **view))["variant"] == code
+        odd = fhconv.make_desc(*shape, variant=deep[0], x_cstride=cs + 1, x_c0=c0)
+        with pytest.raises(fhconv.FhcError, match="channel pairs"):
+            fhconv.plan_dry(odd)
+    finally:
+        fhconv.tune_clear()
+
+
 def test_forced_split_k_and_reference_hint():
     p = fhconv.plan_dry(fhconv.make_desc(1, 68, 120, 128, 128, ksplit=4))
     np_ = -(-128 // p["tile_channels"]) * p["tile_channels"]
