@@ -562,16 +562,35 @@ int direct_default(const fhc_conv_desc& d, const Geometry& g) {
 // and its batched form, and on the 128 -> 128 layer at 1080p/16).
 constexpr int kGemmDefault = 11;
 
+// Where the deep-layer kernel (48-channel tiles of 8 rows) is faster in a view of channel pairs than what such a view
+// takes otherwise, by some 760 shapes of 4,096 to 10^6 output pixels. Against the direct forms: over 128 channels from
+// three blocks and a workgroup a CU on (126 -> 144 at 81,921 px 71 us against 156; 100 -> 52 at 4,420 8.9 against 6.5),
+// over 160 where 48-channel tiles are no more than 64-channel ones (130 -> 48 at 322,816 px 95 against 150; 160 -> 64 at
+// 183,456 104 against 83), over 288 from two blocks and two workgroups a CU on (288 -> 36 at 58,760 px 38 against 85;
+// 288 -> 12 at 105,468 51 against 39). Against the chunked kernel at other depths: one round of workgroups, or where that
+// kernel's tiles are 48 channels wide (0.84 of its time on average, at most 1.09) or 16 for a wider cout (0.44); its wider
+// tiles read the input fewer times (200 -> 60 at 477,576 px 332 against 193).
+bool pairs_faster(const fhc_conv_desc& d, const Geometry& g) {
+    const uint64_t c = div_ceil(d.cin, 32) * 32, b = div_ceil(d.cout, 16), b3 = (b + 2) / 3, b4 = (b + 3) / 4;
+    auto tiles = [&](uint32_t th) { return (uint64_t)d.n * div_ceil(g.hout, th) * div_ceil(g.wout, 16); };
+    if (c <= 96) return false;
+    if (c == 128) return b >= 3 && tiles(2) * b4 > 256;
+    if (c == 160) return b >= 3 && b3 == b4 && tiles(2) * b4 > (b == 3 ? 512 : 256);
+    if (c == 288) return b >= 2 && tiles(2) * ((b + 1) / 2) > 512;
+    const int chunked = heuristic_cfg(d, g);
+    return tiles(8) * b3 <= 256 || chunked == 9 || (chunked == 3 && b >= 2);
+}
+
 // The planner's general choice: the deep-layer kernel for stride-1 3x3 convs over more than 64 input channels whose
 // input view has 16-byte channel groups and at least 4096 output pixels (on smaller ones its fixed cost per launch, the
 // first chunk's load and the epilogue, outweighs the direct kernel's longer chains), with `pairs` also in views of
-// channel pairs: 100 -> 100 at 3 x 135 x 241 in a dense view took the direct kernel 163 us with 2-byte loads, this one
-// 76. Then the direct kernel whenever a configuration serves the input channels, then the deep-layer kernel from 64
+// channel pairs where pairs_faster. Then the direct kernel whenever a configuration serves the input channels, then the deep-layer kernel from 64
 // input channels, else the chunked kernel.
 uint32_t general_code(const fhc_conv_desc& d, const Geometry& g, bool pairs) {
     const bool deep = d.kh == 3 && d.stride == 1 && d.cin >= 64 && input_in_reach(d);
     const bool gemm_ok = deep && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0;
-    if ((gemm_ok || (deep && pairs && pairs_view(d))) && d.cin > 64 && (uint64_t)d.n * g.hout * g.wout >= 4096)
+    if ((gemm_ok || (deep && pairs && pairs_view(d) && pairs_faster(d, g))) && d.cin > 64 &&
+        (uint64_t)d.n * g.hout * g.wout >= 4096)
         return make_code(kGemmDefault, 1, 3);
     const int idx = direct_default(d, g);
     if (idx >= 0) return kDirectBase + (uint32_t)idx;

@@ -198,6 +198,21 @@ def test_a_view_of_channel_pairs_takes_its_own_plans_code(cin, cs, c0):
         fhconv.tune_clear()
 
 
+# (cin, cout, n, h, w, deep-layer kernel): both sides of each line for views of channel pairs, cin + 2 channels apart
+@pytest.mark.parametrize("cin,cout,n,h,w,deep", [
+    (124, 144, 1, 329, 249, True), (100, 52, 1, 85, 52, False), (124, 16, 2, 100, 200, False),
+    (130, 48, 4, 208, 388, True), (130, 48, 2, 61, 61, False), (160, 64, 14, 91, 144, False), (130, 72, 2, 47, 51, True),
+    (288, 36, 4, 113, 130, True), (288, 12, 2, 282, 187, False), (288, 24, 2, 46, 72, False),
+    (200, 60, 18, 134, 198, False), (200, 48, 18, 134, 198, True), (256, 80, 2, 134, 198, True),
+    (256, 16, 2, 400, 300, False), (512, 128, 1, 64, 80, True), (512, 256, 1, 767, 683, False),
+    (90, 52, 2, 134, 198, False), (90, 20, 2, 134, 198, False)])
+def test_channel_pairs_take_the_deep_layer_kernel_where_it_is_faster(cin, cout, n, h, w, deep):
+    d = fhconv.make_desc(n, h, w, cin, cout, x_cstride=cin + 2, y_cstride=cout + 1)  # off the resident grids
+    assert (fhconv.plan_dry(d)["family"] == "gemm") == deep, fhconv.plan_dry(d)["name"]
+    d.ksplit = 1  # a fixed K split keeps the choice such a view always had
+    assert fhconv.plan_dry(d)["family"] != "gemm"
+
+
 def test_forced_split_k_and_reference_hint():
     p = fhconv.plan_dry(fhconv.make_desc(1, 68, 120, 128, 128, ksplit=4))
     np_ = -(-128 // p["tile_channels"]) * p["tile_channels"]
