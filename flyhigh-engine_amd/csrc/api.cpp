@@ -437,13 +437,18 @@ int direct_index(const fhc_conv_desc& d, int fm, int wm, int wn, int wk, int per
 
 // The 3x3 configurations measured faster than the general choices below, by the input channels padded to 32 (c), the
 // output channel blocks of 16 (b) and the output pixels (px); 0 where none is. The lines come from every variant's
-// time over some 400 shapes of the layers' ranges (17 to 544 rows, batches to 24), each lying where one family's times
-// cross the other's; over all of them the chosen variant is within 5% of the fastest on average, where the general
-// choices alone were 30% off (each line: an example with both sides' times, us).
+// time over some 400 shapes of the layers' ranges (17 to 544 rows, batches to 24), and from both sides of each line over
+// 12,000 more (8 to 1,100 rows, padded, dense and odd views), each lying where one family's times cross the other's
+// (each line: an example with both sides' times, us). Where both sides are one workgroup a tile, the crossing is in
+// rounds: the workgroups that the chip's 256 CUs hold at once, so a variant whose count just passes a multiple pays a
+// whole round more.
 uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
     if (d.kh != 3) return 0;
     const uint32_t c = div_ceil(d.cin, 32) * 32, b = div_ceil(d.cout, 16);
     const uint64_t px = (uint64_t)d.n * g.hout * g.wout, work = px * b;
+    auto tiles = [&](uint32_t th) { return (uint64_t)d.n * div_ceil(g.hout, th) * div_ceil(g.wout, 16); };
+    const uint64_t t2 = tiles(2), t8 = tiles(8), b2 = div_ceil(b, 2u), b3 = div_ceil(b, 3u), b4 = div_ceil(b, 4u);
+    auto rounds = [](uint64_t wgs) { return (wgs + 255) / 256; };
     auto dir = [&](int fm, int wm, int wn, int wk = 1, int persist = 0) -> uint32_t {
         const int i = direct_index(d, fm, wm, wn, wk, persist);
         return i < 0 ? 0 : kDirectBase + (uint32_t)i;
@@ -480,17 +485,20 @@ uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
     }
     if (d.stride == 2) {  // two rows a wave: half the weight loads. 64 -> 72 at 14,400 px: 6.9 against 10.1
         if (c == 32 && b >= 3 && px >= 16000 && px < 60000) return dir(2, 1, b == 4 || b > 6 ? 4 : 3);
-        if (c == 64 && b >= 5 && px >= 5000) return dir(2, 1, 3);
+        // (where it pads cout less than four blocks a workgroup, or those leave CUs idle: 48 -> 98 at 38,688 px 23% slower)
+        if (c == 64 && b >= 5 && px >= 5000 && (b3 * 3 < b4 * 4 || tiles(4) * b4 < 512)) return dir(2, 1, 3);
         return 0;
     }
     if (c == 64 || c == 96) {  // small tensors: a third of the chain a wave. 96 -> 96 at 960 px: 3.7 against 5.1
         if (b == 1 && px < (c == 64 ? 16000u : 7000u)) return dir(1, 1, 1, 3);
         if (b == 2 && px < 4096) return dir(1, 1, 2, 3);
         if (b == 3 && px < 7000) return dir(1, 1, 3, 3);
-        if (b >= 4 && px < (c == 64 ? 2500u : 4096u)) return dir(1, 1, 3, 3);
+        // (two workgroups a CU at most: 96 -> 52 at 3,822 px, 588 of them, 6.5 against 5.6)
+        if (b >= 4 && px < (c == 64 ? 2500u : 4096u) && tiles(1) * b3 <= 512) return dir(1, 1, 3, 3);
     }
     if (c == 32) {
-        if (b == 2 && px >= 24000 && px < 60000) return dir(4, 2, 2);  // 14 -> 24 at 58,880 px: 5.0 against 6.0
+        // 14 -> 24 at 58,880 px: 5.0 against 6.0 (14 -> 32 at 24,192, 1,512 two-row tiles: 5.8 against 5.1)
+        if (b == 2 && t2 > 1536 && px < 60000) return dir(4, 2, 2);
         if (b == 3 && px >= 10000) return dir(2, 1, 3);                // 32 -> 48 at 12,480 px: 3.8 against 4.0
         if (b >= 5 && px >= 7000) return px < 16000 ? dir(2, 1, 2) : dir(4, 2, 2);  // 32 -> 128 at 40,000: 1.0 to 1.7
     }
@@ -501,22 +509,35 @@ uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
     }
     if (c == 96 && px >= 4096) {  // below the resident grid's line
         if (b == 1) return px < 60000 ? dir(2, 1, 1, 3) : dir(2, 4, 1);  // 72 -> 5 at 159,960 px: 16.8 against 33.5
-        if (b == 2 || b == 3) return dir(2, 1, b);                       // 96 -> 48 at 8,991 px: 5.7 against 7.3
-        return dir(4, 2, 2);                                             // 96 -> 96 at 8,160 px: 7.1 against 7.6
+        if (b == 2) return in16 ? dir(2, 1, 2) : 0;  // 96 -> 32 against the deep-layer kernel: 0.78 over 120 shapes
+        // one 8-row deep-layer tile a CU is one round of 8.3 us, this form 5.5 to 512 tiles, then 9: 96 -> 48 at 8,991
+        // px 5.7 against 7.3, at 22,576 9.7 against 8.6, at 52,611 19.0 against 22.0; large outputs off the resident
+        // grid (72 -> 46 at 683,012 px) 164 against 145. Unaligned views: against the direct forms, 0.72
+        if (b == 3) return !in16 || t2 <= 512 || (t8 > 256 && px < 70000) ? dir(2, 1, 3) : 0;
+        // 96 -> 96 at 8,160 px: 7.1 against 7.6; 96 -> 80 at 9,360, 315 workgroups against 210: 8.9 against 8.3
+        return (in16 ? t8 * b2 <= 256 || t8 * b3 > 256 : t2 * b4 > 256) ? dir(4, 2, 2) : 0;
     }
     if (c == 128 && px >= 4096) {
-        if (b == 1) return px < 16000 ? dir(1, 2, 1) : dir(2, 4, 1);  // 128 -> 12 at 10,660 px: 5.3 against 7.7
-        if (b == 2) return px < 16000 ? dir(1, 2, 2) : dir(2, 4, 1);  // 128 -> 32 at 8,160 px: 5.9 against 7.7
-        if (b == 3 && px < 20000) return dir(2, 4, 1);                // 128 -> 48 at 8,160 px: 6.0 against 8.2
+        // 128 -> 12 at 10,660 px: 5.3 against 7.7
+        if (b == 1) return px < 16000 ? dir(1, 2, 1) : in16 || t2 > 768 ? dir(2, 4, 1) : 0;
+        // 128 -> 32 at 8,160 px: 5.9 against 7.7 (level past two workgroups a CU)
+        if (b == 2) return px >= 16000 ? dir(2, 4, 1) : !in16 || t2 <= 512 ? dir(1, 2, 2) : 0;
+        // 128 -> 48 at 8,160 px: 6.0 against 8.2 (126 -> 48 at 19,680, three rounds against one: 12.9 against 9.3)
+        if (b == 3 && px < 20000 && (in16 ? t8 * 3 <= 512 : t2 > 256)) return dir(2, 4, 1);
     }
     if (c == 160 || c == 288) {
-        if (b == 1 && (c == 160 || px < 60000)) return dir(2, 1, 1, 3);  // 279 -> 12 at 4,158 px: 6.8 against 12.1
+        // 279 -> 12 at 4,158 px: 6.8 against 12.1 (288 -> 12 at 48,972, 812 tiles against 203: 26.6 against 25.2)
+        if (b == 1 && (c == 160 || (px < 60000 && (!in16 || t2 <= 768 || t8 > 256)))) return dir(2, 1, 1, 3);
         if (c == 160 && (b == 2 || b == 3) && px < 7000) return dir(2, 1, b, 3);  // 155 -> 24 at 4,230 px: 5.1 against 8.7
         if (in16 && input_in_reach(d)) {
             if (b <= 2 && px >= 60000) return gemm(2);  // 155 -> 32 at 60,000 px and up: 1.0 to 1.4
-            if (b == 4 && px >= 7000) return gemm(12);  // 279 -> 64: 1.0 to 1.6
-            if (b >= 7 && px >= (c == 160 ? 7000u : 60000u)) return gemm(12);  // 155 -> 128 at 145,992 px: 101 against 128
-            if (px >= 60000) return gemm(13);           // 155 -> 48 at 155,520 px: 42.3 against 51.9
+            // a 64-channel tile costs 1.17 of a 48-channel one, so it has to save rounds: 155 -> 128 at 145,992 px 101
+            // against 128, 279 -> 64 at 7,000 px and up 1.0 to 1.6; 279 -> 130 (9 blocks) at 393,156 623 against 537
+            if ((b == 4 || b >= 7) && px >= (b == 4 || c == 160 ? 7000u : 60000u))
+                return rounds(t8 * b4) < rounds(t8 * b3) ? gemm(12) : 0;
+            // a 16-row tile costs 1.6 of an 8-row one: 155 -> 48 at 155,520 px 42.3 against 51.9, 130 -> 48 at 79,101, two
+            // rounds against three, 31.1 against 29.1
+            if (px >= 60000 && 5 * rounds(t8 * b3) >= 8 * rounds(tiles(16) * b3)) return gemm(13);
         }
     }
     return 0;

@@ -140,6 +140,82 @@ def test_tensors_past_the_deep_layer_kernels_reach_keep_the_direct_kernel(n, cin
     assert fhconv.plan_dry(d)["family"] == "direct"
 
 
+# (cin, cout, n, h, w, stride), the input's and the output's (channel stride, offset), and the variant measured faster:
+# one shape inside each of the planner's lines, and one past each that has a far side
+MEASURED = [
+    ((72, 38, 10, 167, 281, 1), (72, 0), (38, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((72, 36, 10, 167, 281, 1), (72, 0), (38, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((128, 16, 1, 97, 204, 1), (128, 0), (16, 0), "direct.c128.t2x4.n16"),
+    ((100, 12, 3, 114, 145, 1), (103, 1), (16, 0), "direct.c128.t2x4.n16"),
+    ((100, 12, 1, 122, 115, 1), (104, 0), (16, 0), "direct.c128.t1x2.n16"),
+    ((128, 18, 5, 403, 363, 1), (128, 0), (22, 0), "direct.c128.t2x4.n16"),
+    ((102, 18, 1, 85, 123, 1), (104, 0), (21, 1), "direct.c128.t1x2.n32"),
+    ((100, 48, 5, 50, 32, 1), (103, 1), (48, 0), "direct.c128.t1x2.n48"),
+    ((126, 38, 1, 82, 125, 1), (128, 0), (40, 0), "direct.c128.t2x4.n16"),
+    ((102, 38, 13, 28, 37, 1), (105, 1), (41, 1), "direct.c128.t2x4.n16"),
+    ((126, 36, 22, 19, 39, 1), (128, 0), (40, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((24, 32, 12, 37, 56, 1), (24, 0), (34, 0), "direct.c32.t1x2.n32"),
+    ((24, 18, 1, 182, 300, 1), (24, 0), (24, 0), "direct.c32.t4x2.n32"),
+    ((14, 36, 10, 216, 403, 1), (17, 1), (40, 0), "direct.c32.t2x1.n48"),
+    ((9, 130, 2, 102, 208, 1), (12, 2), (134, 0), "direct.c32.t4x2.n32"),
+    ((16, 112, 19, 33, 24, 1), (19, 1), (115, 1), "direct.c32.t2x1.n32"),
+    ((64, 24, 5, 64, 71, 1), (64, 0), (24, 0), "direct.c64.t2x1.n32"),
+    ((33, 36, 11, 36, 76, 1), (35, 1), (39, 1), "direct.c64.t2x1.n48"),
+    ((48, 64, 8, 175, 349, 1), (51, 1), (67, 1), "direct.c64.t2x1.n64"),
+    ((64, 128, 9, 38, 58, 1), (67, 1), (128, 0), "direct.c64.t2x1.n48"),
+    ((66, 7, 8, 421, 385, 1), (72, 0), (9, 1), "direct.c96.t2x4.n16"),
+    ((72, 16, 8, 53, 44, 1), (72, 0), (16, 0), "direct.c96.t2x1.n16/rows"),
+    ((66, 18, 18, 45, 34, 1), (72, 0), (22, 0), "direct.c96.t2x1.n32"),
+    ((90, 24, 11, 143, 145, 1), (93, 1), (24, 0), "direct.c96.t4x2.n32"),
+    ((90, 48, 8, 30, 42, 1), (96, 0), (48, 0), "direct.c96.t2x1.n48"),
+    ((72, 36, 21, 20, 36, 1), (75, 1), (36, 0), "direct.c96.t2x1.n48"),
+    ((72, 38, 2, 188, 214, 1), (72, 0), (40, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((72, 52, 4, 23, 47, 1), (75, 1), (56, 0), "direct.c96.t1x2.n64"),
+    ((72, 84, 4, 52, 51, 1), (72, 0), (88, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((96, 160, 2, 275, 290, 1), (96, 0), (163, 1), "direct.c96.t4x2.n32"),
+    ((72, 72, 2, 398, 438, 1), (75, 1), (72, 0), "direct.c96.t4x2.n32"),
+    ((279, 52, 12, 31, 21, 1), (280, 0), (56, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((160, 52, 1, 162, 338, 1), (160, 0), (56, 0), "gemm.t8x16.n64.f4x2.w2x2.c32.p2"),
+    ((258, 256, 3, 178, 131, 1), (264, 0), (256, 0), "gemm.t8x16.n64.f4x2.w2x2.c32.p2"),
+    ((288, 130, 2, 186, 220, 1), (288, 0), (136, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((288, 36, 2, 175, 343, 1), (288, 0), (36, 0), "gemm.t16x16.n48.f4x3.w4x1.c32.p2"),
+    ((160, 36, 1, 242, 515, 1), (160, 0), (39, 1), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((288, 16, 8, 94, 173, 1), (288, 0), (18, 0), "gemm.t8x16.n32.f4x2.w2x1.c32.p2"),
+    ((128, 64, 2, 552, 683, 1), (128, 0), (64, 0), "direct.c128.t4x1.n64/p"),
+    ((24, 128, 1, 595, 682, 1), (24, 0), (128, 0), "direct.c32.t8x1.n64/p"),
+    ((33, 64, 4, 218, 194, 1), (40, 0), (64, 0), "direct.c64.t4x1.n64/p"),
+    ((90, 56, 1, 456, 546, 1), (96, 0), (56, 0), "direct.c96.t4x1.n64/p"),
+    ((160, 12, 2, 157, 117, 1), (160, 0), (16, 0), "direct.c160.t2x1.n16/rows"),
+    ((130, 24, 2, 55, 50, 1), (136, 0), (26, 0), "direct.c160.t2x1.n32/rows"),
+    ((279, 12, 1, 96, 66, 1), (280, 0), (12, 0), "direct.c288.t2x1.n16/rows"),
+    ((288, 5, 2, 102, 139, 1), (288, 0), (8, 0), "gemm.t8x16.n48.f2x3.w4x1.c32.p2"),
+    ((64, 16, 3, 10, 8, 1), (64, 0), (16, 0), "direct.c64.t1x1.n16/rows"),
+    ((33, 30, 1, 9, 14, 1), (36, 2), (32, 0), "direct.c64.t1x1.n32/rows"),
+    ((64, 48, 5, 10, 18, 1), (67, 1), (51, 1), "direct.c64.t1x1.n48/rows"),
+    ((48, 192, 1, 10, 21, 1), (48, 0), (192, 0), "direct.c64.t1x1.n48/rows"),
+    ((33, 56, 15, 9, 18, 1), (40, 0), (58, 0), "direct.c64.t1x2.n64"),
+    ((90, 16, 8, 22, 23, 1), (96, 0), (19, 1), "direct.c96.t1x1.n16/rows"),
+    ((90, 18, 23, 9, 8, 1), (93, 1), (22, 0), "direct.c96.t1x1.n32/rows"),
+    ((66, 48, 1, 31, 56, 1), (69, 1), (48, 0), "direct.c96.t1x1.n48/rows"),
+    ((72, 52, 5, 17, 29, 1), (72, 0), (54, 0), "direct.c96.t1x1.n48/rows"),
+    ((96, 56, 5, 19, 35, 1), (99, 1), (56, 0), "direct.c96.t1x2.n64"),
+    ((14, 144, 6, 339, 256, 2), (16, 0), (144, 0), "direct.s2.c32.t4x1.n64/p"),
+    ((36, 192, 8, 219, 358, 2), (40, 0), (192, 0), "direct.s2.c64.t2x2.n64/p"),
+    ((3, 128, 6, 173, 155, 2), (6, 2), (128, 0), "direct.s2.c32.t2x1.n64"),
+    ((63, 72, 2, 162, 142, 2), (64, 0), (72, 0), "direct.s2.c64.t2x1.n48"),
+    ((48, 98, 2, 345, 739, 2), (51, 1), (100, 0), "direct.s2.c64.t2x2.n64"),
+]
+
+
+@pytest.mark.parametrize("shape,xv,yv,name", MEASURED, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_the_planner_takes_the_measured_variant(shape, xv, yv, name):
+    cin, cout, n, h, w, stride = shape
+    d = fhconv.make_desc(n, h, w, cin, cout, stride=stride, x_cstride=xv[0], x_c0=xv[1], y_cstride=yv[0], y_c0=yv[1])
+    assert fhconv.plan_dry(d)["name"] == name
+    d.ksplit = 1  # a fixed K split keeps the one-chain K order: no resident loop
+    assert not fhconv.plan_dry(d)["name"].endswith("/p")
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_mi355x_plan_covers_the_output(shape):
     n, h, w, cin, cout, k, s = shape
