@@ -631,10 +631,11 @@ bool tap_order(uint32_t code) {
 // general choice. A caller that fixes the K split at 1 keeps the general choice's K order, hence its bits (the frame
 // program does: rounding in another order travels through the whole network): a measured choice then stands only
 // where both are one-tile chains. A split above 1 moves the general choice to its split form.
+bool split_open(const fhc_conv_desc& d) { return d.ksplit == 0 && (d.ref_cand == 0xFFu || (d.ref_cand >> 4) == 0); }
 uint32_t heuristic_code(const fhc_conv_desc& d, const Geometry& g) {
-    const bool unsplit = d.ksplit == 0 && (d.ref_cand == 0xFFu || (d.ref_cand >> 4) == 0);
-    const uint32_t general = general_code(d, g, unsplit), m = measured_code(d, g);
-    return m && (unsplit || (d.ksplit == 1 && tap_order(m) && tap_order(general))) ? m : general;
+    const bool open = split_open(d);
+    const uint32_t general = general_code(d, g, open), m = measured_code(d, g);
+    return m && (open || (d.ksplit == 1 && tap_order(m) && tap_order(general))) ? m : general;
 }
 
 int heuristic_cfg(const fhc_conv_desc& d, const Geometry& g) {
@@ -1610,14 +1611,19 @@ extern "C" int fhc_conv_sibling_plan_create(const fhc_conv_desc* desc_a, const u
         if ((A.act == FHC_ACT_PRELU && !slope_a) || (B.act == FHC_ACT_PRELU && !slope_b))
             return fail(-1, "%s: PReLU needs a slope", who);
         // the combined conv: A's channels, zero channels up to a multiple of 4, B's. Its K order per output channel
-        // is the kernel-row split's or the plain chain's: the one the planner gives both convs alone when it gives
-        // both a direct configuration with the same split (the outputs are then bit-identical), else the split's
+        // is the kernel-row split's or the plain chain's: the one the planner gives both convs alone at a K split of 1
+        // when it gives both a direct configuration with the same split (where those are one-tile configurations, the
+        // outputs are then bit-identical), else the split's. The choice for an open split may differ between the two
+        // (at 100 x 108, 48 -> 7 splits the kernel rows and 48 -> 36 does not) or add K in the resident grid's order
         const uint32_t split = (A.cout + 3) & ~3u, total = split + B.cout, cin32 = div_ceil(A.cin, 32) * 32;
         int wk = 3;
         {
             fhc_conv_plan pa{}, pb{};
             std::string w1, w2;
-            if (plan_choose(A, pa, &w1) && plan_choose(B, pb, &w2) && pa.family == 1 && pb.family == 1 &&
+            fhc_conv_desc one_a = A, one_b = B;
+            for (fhc_conv_desc* d : {&one_a, &one_b})
+                if (split_open(*d)) d->ksplit = 1;
+            if (plan_choose(one_a, pa, &w1) && plan_choose(one_b, pb, &w2) && pa.family == 1 && pb.family == 1 &&
                 kDirectCfgs[pa.cfg].na == 1 && kDirectCfgs[pb.cfg].na == 1 &&
                 kDirectCfgs[pa.cfg].wk == kDirectCfgs[pb.cfg].wk && kDirectCfgs[pa.cfg].cin32 == (int)cin32 &&
                 kDirectCfgs[pb.cfg].cin32 == (int)cin32)

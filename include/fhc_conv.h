@@ -49,7 +49,8 @@ typedef struct fhc_conv_desc {
     float alpha;                 /* FHC_ACT_LEAKY slope                                                         */
     uint32_t residual;           /* 1: y = f16(f32(f16(act(acc + bias))) + f32(r)) (conv_tiled.wgsl:57-61)      */
     uint32_t variant;            /* 0: planner (tune table, else heuristic); else a forced MI355X variant code  */
-    uint32_t ksplit;             /* 0: planner; else a forced split-K count (1, 2, 4, 8)                        */
+    uint32_t ksplit;             /* 0: planner; else a forced split-K count (1, 2, 4, 8). 1 also keeps the order
+                                    in which the planner's general choice adds K, hence its bits               */
     uint32_t ref_cand;           /* 0xFF: none; else the reference's candidate code (candidates.rs:3-16), taken
                                     as a hint: its forced split-K nibble applies when ksplit is 0              */
 } fhc_conv_desc;
@@ -147,7 +148,8 @@ int fhc_conv_pair_plan_create(const fhc_conv_desc* desc_a, const uint16_t* w_a, 
 
 /* Sibling convs: two convs A and B that read the same input view with the same geometry, as one launch (the
  * one-tile direct kernel computing A's output channels, zero channels up to a multiple of 4, then B's, each with
- * the K loop the same configuration runs for it alone). A may take a residual; B takes none; identity or PReLU
+ * the K loop the same configuration runs for it alone: where the table or a variant names no other kernel, the bits of
+ * the two convs planned at ksplit 1). A may take a residual; B takes none; identity or PReLU
  * activations. Instantiated: 3x3 stride 1, 33-64 input channels, A.cout rounded up to 4 plus B.cout at most 48
  * (graph.json's fine.out and up.w, which both read the fine block's h: 48 -> 7 + 36). The plan runs with
  * fhc_conv_sibling_run only (fhc_conv_run refuses it) and is freed by fhc_conv_plan_destroy. No counterpart in the

@@ -631,3 +631,22 @@ def test_resident_pair_full_size_ladder(loop):
         want = band.run_oracle(threads=8)[:, r0 - a0:r0 - a0 + 4]
         ok, md, mref = parity(got[:, r0:r0 + 4], want)
         assert ok, (r0, md, mref)
+
+
+# grids on both sides of the lines where the planner's choice for an open K split leaves the one-chain order: the
+# kernel-row split for 48 -> 7 but not 48 -> 36 (7,000 to 16,000 px), the resident grid (from 60,000)
+@pytest.mark.parametrize("h,w,ca,cb", [(60, 108, 7, 36), (100, 108, 7, 36), (100, 100, 4, 36), (200, 320, 36, 4),
+                                       (210, 301, 7, 36)])
+def test_sibling_convs_equal_the_two_convs_at_one_split(h, w, ca, cb):
+    import torch
+    say("siblings", h, w, ca, cb)
+    A = Case(1, h, w, 48, ca, act=1, seed=h)
+    B = Case(1, h, w, 48, cb, act=1, seed=w)
+    B.x = A.x
+    dev = torch.device("cuda", 0)
+    x = torch.from_numpy(A.x.view(np.int16)).to(dev)
+    ya, yb = (torch.from_numpy(c.y0.view(np.int16)).to(dev) for c in (A, B))
+    fhconv.ConvSiblingPlan(A.fhc_desc(), A.wt, A.bias, A.slope, B.fhc_desc(), B.wt, B.bias, B.slope).run(x, ya, None, yb)
+    torch.cuda.synchronize()
+    for c, y in ((A, ya), (B, yb)):
+        assert np.array_equal(y.cpu().numpy().view(np.uint16), c.run_gpu(ksplit=1)), c.cout
