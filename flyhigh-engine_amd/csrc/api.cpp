@@ -1162,11 +1162,18 @@ extern "C" int fhc_conv_pair_plan_create(const fhc_conv_desc* desc_a, const uint
         // the configuration for channels per tap cp: by default the resident-grid loop when it is instantiated and
         // there are at least 8 tiles per CU of an MI355X (256), one wave row where that is instantiated (else two),
         // and the tallest instantiated tile that still gives 256 workgroups, else the shortest; -1 if none
+        // whether the resident grids' buffer loops can read and write these views (pair_buffer_ok; the base pointers are
+        // the launch's to check)
+        const bool ext = B.residual && !res_mid;
+        const bool buffers = A.x_cstride % 8 == 0 && A.x_c0 % 8 == 0 && B.cout % 4 == 0 && B.y_cstride % 4 == 0 &&
+                             B.y_c0 % 4 == 0 && (!ext || (B.r_cstride % 4 == 0 && B.r_c0 % 4 == 0)) && input_in_reach(A) &&
+                             (uint64_t)B.n * B.h * B.w * std::max(B.y_cstride, ext ? B.r_cstride : 0u) * 2 < (1ull << 31);
         auto select = [&](int cp) {
             auto serves = [&](const PairCfg& c) { return serves_cp(c, cp); };
             // the resident grids measured fastest over batches 1-24 of the network's pairs (the same bits in every
-            // loop), from the tiles where they pass the one-tile kernel
-            if (!loop_req && !th_req && !wm_req) {
+            // loop), from the tiles where they pass the one-tile kernel. Other views run one tile a workgroup, in the
+            // split of the choice below: dense 3 -> 36 -> 36 at 3 x 520 x 637 on the two wave rows 103 us against 68
+            if (buffers && !loop_req && !th_req && !wm_req) {
                 int th = 0, wm = 0, persist = 0;
                 if (A.stride == 1 && ca32 == 32 && cb32 == 32 && tiles_at(8) >= 1024)
                     th = 8, wm = 2, persist = 1;  // 14 -> 24 -> 24 at 622,080 px: 37.9 us against 45.5 on separate waves

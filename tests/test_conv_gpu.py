@@ -650,3 +650,37 @@ def test_sibling_convs_equal_the_two_convs_at_one_split(h, w, ca, cb):
     torch.cuda.synchronize()
     for c, y in ((A, ya), (B, yb)):
         assert np.array_equal(y.cpu().numpy().view(np.uint16), c.run_gpu(ksplit=1)), c.cout
+
+
+# fused pairs over their resident grids' lines: the grid's loop where its buffer loop reads and writes the views, else
+# the earlier choice's (whose one-tile form such views run)
+@pytest.mark.parametrize("n,h,w,c,stride,xcs,ycs,loop", [
+    (4, 322, 454, (3, 36, 36), 2, 8, 40, "w2.k8/p"), (4, 322, 454, (3, 36, 36), 2, 3, 36, "w1.k8/ws"),
+    (4, 322, 454, (3, 36, 36), 2, 8, 37, "w1.k8/ws"), (13, 146, 215, (3, 36, 36), 2, 6, 36, "w1.k8"),
+    (8, 120, 216, (48, 48, 48), 1, 48, 48, "w1/ws"), (8, 120, 216, (48, 48, 48), 1, 48, 49, "t4x14.w1/ws"),
+    (4, 60, 216, (48, 48, 48), 1, 52, 48, "t4x14.w1"), (9, 184, 320, (14, 24, 24), 1, 16, 24, "t8x14.w2.k16/p"),
+    (2, 184, 320, (14, 24, 24), 1, 14, 24, "w1.k16/ws")])
+def test_fused_pairs_take_the_grid_that_their_views_allow(n, h, w, c, stride, xcs, ycs, loop):
+    import torch
+    ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+    a = fhconv.make_desc(n, h, w, c[0], c[1], stride=stride, act=0, x_cstride=xcs)
+    b = fhconv.make_desc(n, ho, wo, c[1], c[2], act=0, y_cstride=ycs)
+    rng = np.random.default_rng(w)
+    wa, wb = (f16_bits(rng.normal(0, 0.1, (o, i, 3, 3))) for i, o in zip(c, c[1:]))
+    plan = fhconv.ConvPairPlan(a, wa, f16_bits(np.zeros(c[1])), None, b, wb, f16_bits(np.zeros(c[2])), None)
+    name = plan.describe()["name"]
+    say("pair views", n, h, w, c, name)
+    assert name.endswith(loop), name
+    # the earlier choice gives the same bits on a padded copy of the input
+    dev = torch.device("cuda", 0)
+    x = torch.from_numpy(rng.uniform(-1, 1, (n, h, w, c[0])).astype(np.float16)).to(dev)
+    outs = []
+    for xc, yc in ((xcs, ycs), ((c[0] + 7) // 8 * 8, (c[2] + 7) // 8 * 8)):
+        xp = torch.zeros((n, h, w, xc), dtype=torch.float16, device=dev)
+        xp[..., :c[0]] = x
+        y = torch.zeros((n, ho, wo, yc), dtype=torch.float16, device=dev)
+        a.x_cstride, b.y_cstride = xc, yc
+        fhconv.ConvPairPlan(a, wa, f16_bits(np.zeros(c[1])), None, b, wb, f16_bits(np.zeros(c[2])), None).run(xp, y)
+        torch.cuda.synchronize()
+        outs.append(y[..., :c[2]].contiguous().view(torch.int16).cpu().numpy())
+    assert np.array_equal(*outs)
