@@ -284,9 +284,10 @@ union FitTileLds {
 
 // one fit round of the repair (workgroups 0-127, gm_fit.h at 192 threads) and a conv plan's workgroups (the rest:
 // tile t, channel tile ct at 128 + t + tiles * ct) in one launch
-template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, bool VEC>
+template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, int VIEW>
 __global__ __launch_bounds__(192) void fit_conv_kernel(FitRoundArgs f, ConvKArgs a, uint32_t tiles) {
     static_assert(64 * WM * WN * WK == 192, "the conv's workgroup is 192 threads");
+    static_assert(CIN32 > 32, "no form for fewer than 8 channels");
     constexpr uint32_t NFIT = gmfit::kNwg * 4;
     __shared__ __align__(16) FitTileLds<KS, S, CIN32, FM, WM, WN, WK> lds;
     if (blockIdx.x < NFIT) {  // uniform over the workgroup
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(192) void fit_conv_kernel(FitRoundArgs f, ConvKArgs
                                blockIdx.x % gmfit::kNwg, blockIdx.x / gmfit::kNwg, lds.fit);
     } else {
         const uint32_t b = blockIdx.x - NFIT;
-        conv_tile_body<KS, S, CIN32, FM, WM, WN, WK, VEC>(a, (int)(b % tiles), (int)(b / tiles), lds.tile);
+        conv_tile_body<KS, S, CIN32, FM, WM, WN, WK, VIEW>(a, (int)(b % tiles), (int)(b / tiles), lds.tile);
     }
 }
 
@@ -302,9 +303,9 @@ template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK>
 hipError_t fit_conv_launch(const FitRoundArgs& f, const ConvKArgs& a, dim3 cg, hipStream_t s) {
     const dim3 grid(gmfit::kNwg * 4 + cg.x * cg.y);
     if (a.xvec)
-        hipLaunchKernelGGL((fit_conv_kernel<KS, S, CIN32, FM, WM, WN, WK, true>), grid, dim3(192), 0, s, f, a, cg.x);
+        hipLaunchKernelGGL((fit_conv_kernel<KS, S, CIN32, FM, WM, WN, WK, kWhole>), grid, dim3(192), 0, s, f, a, cg.x);
     else
-        hipLaunchKernelGGL((fit_conv_kernel<KS, S, CIN32, FM, WM, WN, WK, false>), grid, dim3(192), 0, s, f, a, cg.x);
+        hipLaunchKernelGGL((fit_conv_kernel<KS, S, CIN32, FM, WM, WN, WK, kAny>), grid, dim3(192), 0, s, f, a, cg.x);
     return hipGetLastError();
 }
 

@@ -85,18 +85,21 @@ __device__ __forceinline__ uint2 load_res4(const ConvKArgs& a, size_t pix, int c
 
 // 8 consecutive input channels ch..ch+7 of one pixel (p points at channel ch < cin), as one 16-byte load wherever the
 // pixel has 8 channels; settle_group then gives zeros at and past cin, where the value is next used (after the wait
-// for a whole tile's loads). VEC: the view is 16-byte aligned (cstride, c0 multiples of 8), so the stride holds every
+// for a whole tile's loads). kWhole: the view is 16-byte aligned (cstride, c0 multiples of 8), so the stride holds every
 // whole group and a partial group arrives with the channels next to it in the tensor. Other views take the load at
-// its 2-byte alignment (global loads need none), a partial last group as the pixel's last 8 channels. Pixels of
+// its 2-byte alignment (global loads need none), a partial last group as the pixel's last 8 channels. kFew, pixels of
 // fewer than 8 channels: independent 2-byte loads at clamped in-bounds addresses, selected without branches (as a
 // group's 8 loads in every unaligned view, 36 -> 48 at 2 x 200 x 320 took 36.0 us, with the 16-byte loads 29.0 (28.9 in
-// a padded stride); 279 -> 96 at 68 x 120 33.1 -> 24.1)
+// a padded stride); 279 -> 96 at 68 x 120 33.1 -> 24.1).
+// The launcher picks the kernel of the view's kind: both forms behind a branch on cin made the compiler wait at the join
+// (3 -> 36 -> 36 at 468 x 515 21.9 us, as kernels of their own 20.8). kEither: decided at run time.
+enum ViewKind : int { kAny = 0, kWhole = 1, kFew = 2, kEither = 3 };
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-template <bool VEC>
+template <int VIEW>
 __device__ __forceinline__ uint4 load_group(const uint16_t* p, int ch, int cin) {
     const int rem = cin - ch;
-    if constexpr (VEC) return *reinterpret_cast<const uint4*>(p);
-    if (cin >= 8) {
+    if constexpr (VIEW == kWhole) return *reinterpret_cast<const uint4*>(p);
+    if (VIEW == kAny || (VIEW == kEither && cin >= 8)) {
         const u32x4_a2 q = *reinterpret_cast<const u32x4_a2*>(p - max(0, 8 - rem));
         return uint4{q.x, q.y, q.z, q.w};
     }
@@ -125,10 +128,10 @@ __device__ __forceinline__ uint4 shift_group(uint4 v, int k) {
 }
 
 // load_group's value v with zeros past its rem valid channels (v is zero where rem <= 0: nothing was loaded)
-template <bool VEC>
+template <int VIEW>
 __device__ __forceinline__ uint4 settle_group(uint4 v, int rem, int cin) {
-    if constexpr (VEC) return mask_group(v, rem);
-    if (cin >= 8 && (cin & 7)) return shift_group(v, rem >= 8 ? 0 : min(8 - rem, 7));  // uniform
+    if constexpr (VIEW == kWhole) return mask_group(v, rem);
+    if ((VIEW == kAny || (VIEW == kEither && cin >= 8)) && (cin & 7)) return shift_group(v, rem >= 8 ? 0 : min(8 - rem, 7));  // uniform
     return v;
 }
 
@@ -179,7 +182,7 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
     ConvKArgs a) {
     static_assert(WK == 1 || (WK == 3 && KS == 3), "the K split runs one kernel row per wave");
     static_assert(!PERSIST || MODE >= 2, "the persistent configurations run the buffer loop");
-    constexpr bool VEC = MODE > 0;  // 16-byte aligned input
+    constexpr int VIEW = MODE > 0 ? kWhole : kEither;
     constexpr int TH = FM * WM, TW = 16, BN = 16 * NA * WN, NT = 64 * WM * WN * WK;
     constexpr int IH = (TH - 1) * S + KS, IW = (TW - 1) * S + KS;
     constexpr int GPT = CIN32 / 8, PSTR = CIN32 + 8, M = CIN32 / 32;
@@ -264,7 +267,7 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
                             (ch < a.cin);
             pre[i] = uint4{0u, 0u, 0u, 0u};
             if (ok)
-                pre[i] = load_group<VEC>(a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch,
+                pre[i] = load_group<VIEW>(a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch,
                                          a.cin);
         }
     };
@@ -273,7 +276,7 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
         for (int i = 0; i < NLD; i++) {
             const int e = tid + i * NT;
             const int pix = e / GPT, g = e - pix * GPT;
-            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
+            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VIEW>(pre[i], a.cin - g * 8, a.cin);
         }
     };
 
@@ -481,14 +484,14 @@ __attribute__((amdgpu_waves_per_eu(1, PERSIST ? persist_waves_per_simd(WM * WN *
                 for (int i = 0; i < NLD; i++) {
                     const int e = tid + i * NT;
                     const int pix = e / GPT, g = e - pix * GPT;
-                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<true>(pre[i], a.cin - g * 8, a.cin);
+                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<kWhole>(pre[i], a.cin - g * 8, a.cin);
                 }
             } else {
 #pragma unroll
                 for (int i = 0; i < NLD; i++) {
                     const int e = tid + i * NT;
                     const int pix = e / GPT, g = e - pix * GPT;
-                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<false>(pre[i], a.cin - g * 8, a.cin);
+                    *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<kAny>(pre[i], a.cin - g * 8, a.cin);
                 }
             }
         };
@@ -597,7 +600,7 @@ struct TileLds {
 
 // the body of one conv_tile workgroup: spatial tile t, channel tile ct (conv_tile's blockIdx.x, .y; a launch that
 // runs other work beside the conv passes its own numbering), in the workgroup's LDS L
-template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, bool VEC, bool SPLIT = false>
+template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, int VIEW, bool SPLIT = false>
 __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, const int ct,
                                                TileLds<KS, S, CIN32, FM, WM, WN, WK>& L) {
     static_assert(WK == 1 || (WK == 3 && KS == 3), "the K split runs one kernel row per wave");
@@ -635,7 +638,7 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
             pre[i] = uint4{0u, 0u, 0u, 0u};
             if ((i + 1) * NT <= HALO || e < HALO)
                 if (gy >= 0 && gy < a.h && gx >= 0 && gx < a.w && ch < a.cin)
-                    pre[i] = load_group<VEC>(
+                    pre[i] = load_group<VIEW>(
                         a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin);
         }
     }
@@ -670,7 +673,7 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
         const int e = tid + i * NT;
         if ((i + 1) * NT <= HALO || e < HALO) {
             const int pix = e / GPT, g = e - pix * GPT;
-            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
+            *reinterpret_cast<uint4*>(halo + pix * PSTR + g * 8) = settle_group<VIEW>(pre[i], a.cin - g * 8, a.cin);
         }
     }
     __syncthreads();
@@ -750,10 +753,10 @@ __device__ __forceinline__ void conv_tile_body(const ConvKArgs& a, const int t, 
     }
 }
 
-template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, bool VEC, bool SPLIT = false>
+template <int KS, int S, int CIN32, int FM, int WM, int WN, int WK, int VIEW, bool SPLIT = false>
 __global__ __launch_bounds__(64 * WM * WN * WK) void conv_tile(ConvKArgs a) {
     __shared__ __align__(16) TileLds<KS, S, CIN32, FM, WM, WN, WK> lds;
-    conv_tile_body<KS, S, CIN32, FM, WM, WN, WK, VEC, SPLIT>(a, blockIdx.x, blockIdx.y, lds);
+    conv_tile_body<KS, S, CIN32, FM, WM, WN, WK, VIEW, SPLIT>(a, blockIdx.x, blockIdx.y, lds);
 }
 
 // The sibling convs' launch of a one-tile configuration (one workgroup per tile, one channel tile)
@@ -762,9 +765,9 @@ hipError_t launch_tile_split(const ConvKArgs& a, dim3 grid, size_t lds, hipStrea
     (void)lds;
     const dim3 block(64 * WM * WN * WK);
     if (a.xvec)
-        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, true, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kWhole, true>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, false, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kAny, true>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
@@ -803,9 +806,11 @@ hipError_t launch_direct(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t 
     }
     if constexpr (NA == 1) {
         if (a.xvec)
-            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, true>), grid, block, 0, s, a);
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kWhole>), grid, block, 0, s, a);
+        else if (CIN32 > 32 || a.cin >= 8)
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kAny>), grid, block, 0, s, a);
         else
-            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, false>), grid, block, 0, s, a);
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, CIN32 == 32 ? kFew : kAny>), grid, block, 0, s, a);
     } else {
         if (a.xvec)
             hipLaunchKernelGGL((conv_direct<KS, S, CIN32, FM, WM, WN, NA, WK, false, 1>), grid, block, 0, s, a);
@@ -824,7 +829,7 @@ const void* direct_kernel(bool residual) {
     else if constexpr (NA > 1)
         return reinterpret_cast<const void*>(&conv_direct<KS, S, CIN32, FM, WM, WN, NA, WK, false, 1>);
     else
-        return reinterpret_cast<const void*>(&conv_tile<KS, S, CIN32, FM, WM, WN, WK, true>);
+        return reinterpret_cast<const void*>(&conv_tile<KS, S, CIN32, FM, WM, WN, WK, kWhole>);
 }
 
 }  // namespace fhc

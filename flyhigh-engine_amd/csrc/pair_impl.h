@@ -122,7 +122,7 @@ struct PairLds {
 // FILM: A's input goes through film_modulate as it is staged (a.film, the one-tile loop only). The body of one
 // tile t (conv_pair's workgroup t; a launch that runs other work beside the pair passes its own numbering) in the
 // workgroup's LDS L; the block is 64 * WN * WM threads.
-template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, bool VEC, bool FILM = false, int CPA = 32>
+template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, int VIEW, bool FILM = false, int CPA = 32>
 __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t, PairLds<SA, CA32, CB32, TH>& L) {
     constexpr int WN = NBA > NBB ? NBA : NBB, NT = 64 * WN * WM, TWB = kPairTileW;
     constexpr int FA = TH + 2;                                  // A's rows per tile
@@ -171,7 +171,7 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
             pre[i] = uint4{0u, 0u, 0u, 0u};
             if ((i + 1) * NT <= HALO || e < HALO)
                 if (gy >= 0 && gy < a.h && gx >= 0 && gx < a.w && ch < a.cin) {
-                    pre[i] = load_group<VEC>(
+                    pre[i] = load_group<VIEW>(
                         a.x + (((size_t)img * a.h + gy) * a.w + gx) * (size_t)a.xcs + a.xc0 + ch, ch, a.cin);
                     if constexpr (FILM) inside |= 1u << i;
                 }
@@ -223,7 +223,7 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
         const int e = tid + i * NT;
         if ((i + 1) * NT <= HALO || e < HALO) {
             const int pix = e / GPA, g = e - pix * GPA;
-            uint4 q = settle_group<VEC>(pre[i], a.cin - g * 8, a.cin);
+            uint4 q = settle_group<VIEW>(pre[i], a.cin - g * 8, a.cin);
             if constexpr (FILM)
                 if ((inside >> i) & 1u) q = film_group(q, fgm, fbt, a.cin - g * 8);
             *reinterpret_cast<uint4*>(hin + pix * PSA + g * 8) = q;
@@ -296,10 +296,10 @@ __device__ __forceinline__ void conv_pair_tile(const PairKArgs& pk, const int t,
     }
 }
 
-template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, bool VEC, bool FILM = false, int CPA = 32>
+template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, int VIEW, bool FILM = false, int CPA = 32>
 __global__ __launch_bounds__(64 * (NBA > NBB ? NBA : NBB) * WM) void conv_pair(PairKArgs pk) {
     __shared__ __align__(16) PairLds<SA, CA32, CB32, TH> lds;
-    conv_pair_tile<SA, CA32, CB32, NBA, NBB, TH, WM, VEC, FILM, CPA>(pk, blockIdx.x, lds);
+    conv_pair_tile<SA, CA32, CB32, NBA, NBB, TH, WM, VIEW, FILM, CPA>(pk, blockIdx.x, lds);
 }
 
 // The persistent pair: G = gridDim.x resident workgroups loop over B's output tiles t, t + G, ... with both layers'
@@ -700,6 +700,20 @@ inline bool pair_buffer_ok(const PairKArgs& pk) {
            (!ext || view_bytes(pout, b.rcs, b.rc0, b.cout) < lim);
 }
 
+// The one-tile kernel of the input view's kind
+template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, int CPA>
+hipError_t launch_pair_tile(const PairKArgs& pk, dim3 grid, hipStream_t s) {
+    const dim3 block(64 * (NBA > NBB ? NBA : NBB) * WM);
+    if (pk.a.xvec)
+        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, kWhole, false, CPA>), grid, block, 0, s, pk);
+    else if (CA32 > 32 || pk.a.cin >= 8)
+        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, kAny, false, CPA>), grid, block, 0, s, pk);
+    else
+        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, CA32 == 32 ? kFew : kAny, false, CPA>), grid, block, 0,
+                           s, pk);
+    return hipGetLastError();
+}
+
 template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int CPA = 32>
 hipError_t launch_pair_ws(const PairKArgs& pk, dim3 grid, hipStream_t s) {
     if (pair_buffer_ok(pk)) {
@@ -708,12 +722,7 @@ hipError_t launch_pair_ws(const PairKArgs& pk, dim3 grid, hipStream_t s) {
     }
     // views the buffer loop cannot serve: one workgroup per tile
     grid.x = (unsigned)(pk.b.n * pk.b.tiles_y * pk.b.tiles_x);
-    const dim3 block(64 * (NBA > NBB ? NBA : NBB));
-    if (pk.a.xvec)
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, 1, true, false, CPA>), grid, block, 0, s, pk);
-    else
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, 1, false, false, CPA>), grid, block, 0, s, pk);
-    return hipGetLastError();
+    return launch_pair_tile<SA, CA32, CB32, NBA, NBB, TH, 1, CPA>(pk, grid, s);
 }
 
 template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, int CPA = 32>
@@ -726,28 +735,19 @@ hipError_t launch_pair_p(const PairKArgs& pk, dim3 grid, hipStream_t s) {
     // one workgroup per tile, at stride 2 on one wave row: 3 -> 36 -> 36 at 523 x 967 off an aligned pointer 38 us
     // against 57 on two
     grid.x = (unsigned)(pk.b.n * pk.b.tiles_y * pk.b.tiles_x);
-    constexpr int FW = SA == 2 ? 1 : WM;
-    const dim3 fblock(64 * (NBA > NBB ? NBA : NBB) * FW);
-    if (pk.a.xvec)
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, FW, true, false, CPA>), grid, fblock, 0, s, pk);
-    else
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, FW, false, false, CPA>), grid, fblock, 0, s, pk);
-    return hipGetLastError();
+    return launch_pair_tile<SA, CA32, CB32, NBA, NBB, TH, SA == 2 ? 1 : WM, CPA>(pk, grid, s);
 }
 
 template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int WM, int CPA = 32>
 hipError_t launch_pair(const PairKArgs& pk, dim3 grid, hipStream_t s) {
+    if (!pk.a.film) return launch_pair_tile<SA, CA32, CB32, NBA, NBB, TH, WM, CPA>(pk, grid, s);
+    // FiLM on the input: its own instantiations, so the others stage as before
     const dim3 block(64 * (NBA > NBB ? NBA : NBB) * WM);
-    if (pk.a.film) {  // FiLM on the input: its own instantiations, so the others stage as before
-        if (pk.a.xvec)
-            hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, true, true, CPA>), grid, block, 0, s, pk);
-        else
-            hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, false, true, CPA>), grid, block, 0, s, pk);
-    } else if (pk.a.xvec) {
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, true, false, CPA>), grid, block, 0, s, pk);
-    } else {
-        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, false, false, CPA>), grid, block, 0, s, pk);
-    }
+    if (pk.a.xvec)
+        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, kWhole, true, CPA>), grid, block, 0, s, pk);
+    else
+        hipLaunchKernelGGL((conv_pair<SA, CA32, CB32, NBA, NBB, TH, WM, CA32 == 32 ? kEither : kAny, true, CPA>), grid, block,
+                           0, s, pk);
     return hipGetLastError();
 }
 

@@ -23,7 +23,7 @@ PairLaunchFn pair_entry(const void** kernel) {
     } else {
         if (kernel)
             *kernel = reinterpret_cast<const void*>(
-                &conv_pair<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, c.wm, true, false, cp>);
+                &conv_pair<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, c.wm, kWhole, false, cp>);
         return launch_pair<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, c.wm, cp>;
     }
 }
@@ -50,16 +50,17 @@ union FitPairLds {
     PairLds<SA, CA32, CB32, TH> pair;
 };
 
-template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, bool VEC>
+template <int SA, int CA32, int CB32, int NBA, int NBB, int TH, int VIEW>
 __global__ __launch_bounds__(192) void fit_film_pair_kernel(FitRoundArgs f, PairKArgs pk) {
     static_assert((NBA > NBB ? NBA : NBB) == 3, "the pair's workgroup is 192 threads");
+    static_assert(CA32 > 32, "no form for fewer than 8 channels");
     constexpr uint32_t NFIT = gmfit::kNwg * 4;
     __shared__ __align__(16) FitPairLds<SA, CA32, CB32, TH> lds;
     if (blockIdx.x < NFIT)  // uniform over the workgroup
         gmfit::round_body<192>(f.flow, f.cs, f.c0, f.h8, f.w8, f.delta, f.round, f.part_in, f.part_out,
                                blockIdx.x % gmfit::kNwg, blockIdx.x / gmfit::kNwg, lds.fit);
     else
-        conv_pair_tile<SA, CA32, CB32, NBA, NBB, TH, 1, VEC, true>(pk, (int)(blockIdx.x - NFIT), lds.pair);
+        conv_pair_tile<SA, CA32, CB32, NBA, NBB, TH, 1, VIEW, true>(pk, (int)(blockIdx.x - NFIT), lds.pair);
 }
 
 template <int I>
@@ -67,10 +68,10 @@ hipError_t fit_pair_launch(const FitRoundArgs& f, const PairKArgs& pk, uint32_t 
     constexpr PairCfg c = kPairCfgs[I];
     const dim3 grid(gmfit::kNwg * 4 + tiles);
     if (pk.a.xvec)
-        hipLaunchKernelGGL((fit_film_pair_kernel<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, true>), grid, dim3(192), 0, s,
+        hipLaunchKernelGGL((fit_film_pair_kernel<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, kWhole>), grid, dim3(192), 0, s,
                            f, pk);
     else
-        hipLaunchKernelGGL((fit_film_pair_kernel<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, false>), grid, dim3(192),
+        hipLaunchKernelGGL((fit_film_pair_kernel<c.sa, c.ca32, c.cb32, c.nba, c.nbb, c.th, kAny>), grid, dim3(192),
                            0, s, f, pk);
     return hipGetLastError();
 }

@@ -291,9 +291,9 @@ hipError_t launch_wave(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s)
     // the same tiles and channel tiles, one workgroup (NA waves of 16 channels) per tile
     grid.x = (unsigned)(a.n * a.tiles_y * a.tiles_x);
     if (a.xvec)
-        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, 1, NA, 1, true>), grid, dim3(64 * NA), 0, s, a);
+        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, 1, NA, 1, kWhole>), grid, dim3(64 * NA), 0, s, a);
     else
-        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, 1, NA, 1, false>), grid, dim3(64 * NA), 0, s, a);
+        hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, 1, NA, 1, kAny>), grid, dim3(64 * NA), 0, s, a);
     return hipGetLastError();
 }
 
