@@ -283,27 +283,37 @@ __global__ __launch_bounds__(kCvThreads) void convex_tile_kernel(View wt, View x
 
 // ---- film_modulate: shaders/film.wgsl:11-14 ---------------------------------------------------------------------
 // Grid y is the phase: its vectors (one per image of h) and its images of out, whose pixels begin at phase * pixels.
-// VEC: the views and vectors hold 8-byte groups of 4 channels. HBM-bound in its bytes, at 8 pairs x 3 phases of
-// 60 x 108 x 48 some 10 us: the vectors by 2-byte loads 13, a launch a phase 20.
+// VEC: the views hold 8-byte groups of 4 channels. QUAD (c a multiple of 4): the vectors by 8-byte loads, at any
+// alignment of theirs. HBM-bound in its bytes, at 8 pairs x 3 phases of 60 x 108 x 48 some 10 us: the vectors by 2-byte
+// loads 13, a launch a phase 20.
 struct FilmVectors {
     const uint16_t* g[kMaxPhases];
 };
-template <bool VEC>
+template <bool VEC, bool QUAD>
 __global__ __launch_bounds__(kThreads) void film_kernel(View hv, FilmVectors g, OView out, uint32_t hw, uint32_t c,
                                                         uint32_t groups, uint32_t items, uint32_t pixels) {
+    static_assert(QUAD || !VEC, "8-byte groups hold 4 channels each");
+    typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
     const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
     if (t >= items) return;
     const uint32_t pix = t / groups, ch = (t - pix * groups) * 4;
     const uint16_t* gi = g.g[blockIdx.y] + (size_t)(pix / hw) * 2 * c;
-    View gv = hv;
-    gv.p = gi, gv.cs = 0, gv.c0 = 0;
-    float v[4], scale[4], shift[4], o[4];
+    float v[4], o[4];
     ld4<VEC>(hv, pix, ch, c, v);
-    ld4<VEC>(gv, 0, ch, c, scale);
-    gv.c0 = c;
-    ld4<VEC>(gv, 0, ch, c, shift);
+    uint16_t scale[4], shift[4];
+    if constexpr (QUAD) {
+        const u32x2_a2 a = *reinterpret_cast<const u32x2_a2*>(gi + ch), b = *reinterpret_cast<const u32x2_a2*>(gi + c + ch);
+        scale[0] = (uint16_t)a.x, scale[1] = (uint16_t)(a.x >> 16), scale[2] = (uint16_t)a.y, scale[3] = (uint16_t)(a.y >> 16);
+        shift[0] = (uint16_t)b.x, shift[1] = (uint16_t)(b.x >> 16), shift[2] = (uint16_t)b.y, shift[3] = (uint16_t)(b.y >> 16);
+    } else {
 #pragma unroll
-    for (uint32_t i = 0; i < 4; i++) o[i] = v[i] * (1.0f + scale[i]) + shift[i];
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t cc = ch + i < c ? ch + i : 0;  // channels past c are not stored
+            scale[i] = gi[cc], shift[i] = gi[c + cc];
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) o[i] = v[i] * (1.0f + h2f(scale[i])) + h2f(shift[i]);
     st4<VEC>(out, blockIdx.y * pixels + pix, ch, c, o);
 }
 
@@ -2442,11 +2452,10 @@ int film_run(const char* op, const fhc_tensor* hv, const FilmVectors& gv, uint32
     FHC_TRY(check(hv, "film_modulate h", c, false));
     FHC_TRY(check(out, "film_modulate out", c, false, true));
     const uint32_t groups = (c + 3) / 4;
-    bool v = vec4(c, {hv, out});
-    for (uint32_t j = 0; j < phases; j++) v = v && reinterpret_cast<uintptr_t>(gv.g[j]) % 8 == 0;
+    const bool v = vec4(c, {hv, out});
     if ((uint64_t)n * h * w * groups * phases >= kMaxItems) return fail(-1, "%s: too many work items", op);
     return launch(op, (uint64_t)n * h * w * groups, [&](dim3 g, uint32_t items) {
-        auto k = v ? film_kernel<true> : film_kernel<false>;
+        auto k = v ? film_kernel<true, true> : c % 4 == 0 ? film_kernel<false, true> : film_kernel<false, false>;
         hipLaunchKernelGGL(k, dim3(g.x, phases), dim3(kThreads), 0, (hipStream_t)stream, in(hv), gv, outv(out), h * w, c,
                            groups, items, n * h * w);
     });

@@ -144,6 +144,18 @@ def test_film_modulate_matches_oracle(n, h, w, c, cs, c0):
     exact(got, want, "film")
 
 
+# vectors off 8-byte alignment, beside views of 8-byte groups, views off them, and channels that are no multiple of 4
+@pytest.mark.parametrize("n,h,w,c,cs,c0,off", [(2, 21, 33, 48, 48, 0, 1), (1, 17, 20, 48, 53, 1, 0), (3, 9, 11, 36, 37, 0, 2),
+                                               (2, 8, 9, 4, 4, 0, 3), (1, 10, 7, 7, 8, 0, 1)])
+def test_film_modulate_takes_vectors_at_any_alignment(n, h, w, c, cs, c0, off):
+    say("film off", n, h, w, c, cs, c0, off)
+    fh = fhops()
+    rng = np.random.default_rng(n * h * w + c)
+    hv, g = rand(rng, (n, h, w, cs), -3, 3), rand(rng, (n, 2 * c), -1, 1)
+    gd = dev(np.concatenate([np.full(off, 0x7c00, g.dtype), g.ravel()]))[off:]
+    exact(host(fh.film(fh.View(dev(hv), c0), gd, c)), oracle.film(hv, g, c, c0=c0), "film")
+
+
 @pytest.mark.parametrize("n,h,w,c,cs,c0,phases", [(1, 60, 108, 48, 48, 0, 2), (3, 13, 17, 48, 52, 4, 3),
                                                   (2, 5, 7, 7, 11, 3, 8), (1, 1, 1, 1, 1, 0, 2)])
 def test_film_phases_match_oracle(n, h, w, c, cs, c0, phases):
