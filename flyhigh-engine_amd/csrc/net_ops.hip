@@ -509,14 +509,27 @@ __device__ __forceinline__ void aa_row(const uint2 (&q)[KMX], const float (&wx)[
     }
 }
 
+// K neighbouring cells from LDS, each by a read of its own (the atomic keeps the compiler from pairing them): lanes four
+// cells apart meet in the banks twice as often in paired reads (8 x 8 taps at a 4x scale: 680,000 conflict cycles
+// against 334,000, two 480 x 864 pictures' pyramid 6.05 us against 5.7)
+template <int K>
+__device__ __forceinline__ void aa_cells(const uint2* p, uint2 (&q)[K]) {
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const uint64_t t = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p + j), __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_SINGLETHREAD);
+        q[j] = uint2{(uint32_t)t, (uint32_t)(t >> 32)};
+    }
+}
+
 // V4: the input view's pixels are 8-byte aligned 4-channel groups (cs and c0 multiples of 4): one load a pixel. NC: the
-// channels summed (at least c).
-// Bound by VALU issue, 8 instructions a tap: the KMX x KMY taps are those of the scale (5 x 5 where an 8 x 8 form served
-// everything above 4), each a fixed offset from the lane's first, and the LDS is what the taps reach: two 1088 x 1920
-// pictures to 480 x 864 30.4 -> 15.2 us, two of 480 x 864 to 120 x 216 with the pyramid 5.75 -> 6.2, sixteen 23.2 -> 22.4. A tap outside its window has weight +0 and
-// adds +0, as the reference's skipped tap leaves the sums, unless the pixel there is infinite or NaN: a lane whose
-// sums come out so sums again over its window's taps alone.
-template <int KMX, int KMY, int PX, int PY, bool PYR, bool V4, int NC = PYR ? 3 : 4>
+// channels c.
+// Bound by VALU issue, 8 instructions a tap of three channels: the KMX x KMY taps are those of the scale (5 x 5 where an
+// 8 x 8 form served everything above 4), each a fixed offset from the lane's first, and the LDS is what the taps reach: two
+// 1088 x 1920 pictures to 480 x 864 30 -> 12.5 us, two of 480 x 864 to 120 x 216 with the pyramid 5.77 -> 5.71, sixteen
+// 22.2 -> 18.7. A tap outside its window has weight +0 and adds +0, as the reference's skipped tap leaves the sums, unless
+// the pixel there is infinite or NaN: a lane whose sums come out so sums again over its window's taps alone.
+template <int KMX, int KMY, int PX, int PY, bool PYR, bool V4, int NC>
 __global__ __launch_bounds__(kThreads) void interp_aa_lds_kernel(View x, OView out, uint32_t ih, uint32_t iw,
                                                                  uint32_t oh, uint32_t ow, uint32_t c,
                                                                  uint32_t tiles_x, uint32_t tiles_y, PyrOut pyr) {
@@ -532,26 +545,30 @@ __global__ __launch_bounds__(kThreads) void interp_aa_lds_kernel(View x, OView o
     const float fsh = fmaxf(sh, 1.0f), fsw = fmaxf(sw, 1.0f);
     const int ylo = max(0, (int)floorf(((float)oy0 + 0.5f) * sh - fsh + 0.5f));
     const int xlo = max(0, (int)floorf(((float)ox0 + 0.5f) * sw - fsw + 0.5f));
+    // the last row and column of the tile's windows: cells past them hold the last pixel again (taps of weight +0, and no
+    // memory read that the windows do not need)
+    const int ylast = max(0, min((int)ih, (int)floorf(((float)min(oy0 + kAaT, oh) - 0.5f) * sh + fsh + 0.5f)) - 1 - ylo);
+    const int xlast = max(0, min((int)iw, (int)floorf(((float)min(ox0 + kAaT, ow) - 0.5f) * sw + fsw + 0.5f)) - 1 - xlo);
     // the window's first pixel (uniform), then 32-bit byte offsets of the lane's rows and columns (a few rows of the
     // picture at most, so row * iw * cs stays far below 2^32 for any frame)
     const char* wbase = reinterpret_cast<const char*>(x.p + (((size_t)img * ih + ylo) * iw + xlo) * x.cs + x.c0);
     uint32_t roff[RY], coff[RX];
 #pragma unroll
-    for (uint32_t i = 0; i < RY; i++) roff[i] = min(ty + kAaT * i, ih - 1 - ylo) * iw * x.cs * 2u;
+    for (uint32_t i = 0; i < RY; i++) roff[i] = min(ty + kAaT * i, (uint32_t)ylast) * iw * x.cs * 2u;
 #pragma unroll
-    for (uint32_t j = 0; j < RX; j++) coff[j] = min(tx + kAaT * j, iw - 1 - xlo) * x.cs * 2u;
+    for (uint32_t j = 0; j < RX; j++) coff[j] = min(tx + kAaT * j, (uint32_t)xlast) * x.cs * 2u;
     uint2 cell[RY][RX];
 #pragma unroll
     for (uint32_t i = 0; i < RY; i++)
 #pragma unroll
         for (uint32_t j = 0; j < RX; j++) {
             const uint16_t* src = reinterpret_cast<const uint16_t*>(wbase + (roff[i] + coff[j]));
-            if constexpr (V4) {  // channels past c reach sums that are not stored
+            if constexpr (V4) {
                 cell[i][j] = *reinterpret_cast<const uint2*>(src);
             } else {
-                uint16_t v[4];
+                uint16_t v[4] = {0, 0, 0, 0};
 #pragma unroll
-                for (uint32_t k = 0; k < 4; k++) v[k] = src[min(k, c - 1)];
+                for (int k = 0; k < NC; k++) v[k] = src[k];
                 cell[i][j] = uint2{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)};
             }
         }
@@ -594,14 +611,16 @@ __global__ __launch_bounds__(kThreads) void interp_aa_lds_kernel(View x, OView o
 #pragma unroll
         for (int jy = 0; jy < KMY; jy++) {
             uint2 q[KMX];
-#pragma unroll
-            for (int j = 0; j < KMX; j++) q[j] = first[jy * P + j];
+            aa_cells<KMX>(first + jy * P, q);
             aa_row<KMX, NC>(q, wx, wys[ty * KMY + jy], acc, norm);
         }
     }
+    // the weights' sum complete here: it is not needed before the division, and the compiler would move its chain of
+    // additions behind the branch below, where nothing fills the wait for each (two 480 x 864 pictures' pyramid 6.5 us)
+    asm volatile("" : "+v"(norm));
     bool finite = true;
 #pragma unroll
-    for (int i = 0; i < NC; i++) finite &= i >= (int)c || fabsf(acc[i]) < INFINITY;
+    for (int i = 0; i < NC; i++) finite &= fabsf(acc[i]) < INFINITY;
     if (!finite) {
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[i] = 0.0f;
@@ -1868,8 +1887,8 @@ __device__ __forceinline__ uint2 bgr_cell(uint32_t v) {
 // pixels, so a lane's KMX x KMY cells from its first tap on always hold values in [0, 1], and a tap outside its window
 // (weight +0) adds +0, leaving the sums as the reference's skipped tap leaves them. Bound by VALU issue: 8 instructions
 // a tap. Every tap is therefore a fixed offset from the lane's first (no address arithmetic), the taps of the axes are counted apart and a last row that no lane of the wave uses is skipped.
-// Sixteen 2160p frames (9 x 10 taps) 312 -> 245 us, eight 1440p frames (6 x 6) 78 -> 52, two 1080p frames (5 x 5,
-// bound by the latency of staging, then summing) 14.0 -> 13.7.
+// Sixteen 2160p frames (9 x 10 taps) to 864 x 480 316 -> 222 us, eight 1440p frames (6 x 6) 78 -> 46, two 1080p frames
+// (5 x 5, bound by the latency of staging, then summing) 12.4 -> 12.0.
 template <int KMX, int KMY, int TH, int PX, int PY>
 __global__ __launch_bounds__(16 * TH) void rgba_resize_kernel(const uint32_t* src, uint32_t w, uint32_t h,
                                                               uint32_t pitch, uint64_t fstride, uint32_t ih,
@@ -1885,16 +1904,19 @@ __global__ __launch_bounds__(16 * TH) void rgba_resize_kernel(const uint32_t* sr
     const float fsh = fmaxf(sh, 1.0f), fsw = fmaxf(sw, 1.0f);  // sh = ih / oh, sw = iw / ow from the host
     const int ylo = max(0, (int)floorf(((float)oy0 + 0.5f) * sh - fsh + 0.5f));
     const int xlo = max(0, (int)floorf(((float)ox0 + 0.5f) * sw - fsw + 0.5f));
-    // the frame through a buffer resource: a pixel's byte offset is one 24-bit multiply-add
+    // the frame through a buffer resource: a pixel's byte offset is one 24-bit multiply-add. Cells past the tile's windows
+    // hold their last pixel again
     const auto rf = buf_rsrc(src + img * fstride, ((h - 1) * pitch + w) * 4u);
     const uint32_t pitch4 = pitch * 4u;
+    const uint32_t ylast = min(h - 1, (uint32_t)max(0, (int)floorf(((float)min(oy0 + TH, oh) - 0.5f) * sh + fsh + 0.5f) - 1));
+    const uint32_t xlast = min(w - 1, (uint32_t)max(0, (int)floorf(((float)min(ox0 + 16, ow) - 0.5f) * sw + fsw + 0.5f) - 1));
     uint32_t v[RY][RX];
 #pragma unroll
     for (uint32_t i = 0; i < RY; i++)
 #pragma unroll
         for (uint32_t j = 0; j < RX; j++)
             v[i][j] = __builtin_amdgcn_raw_buffer_load_b32(
-                rf, __umul24(min((uint32_t)ylo + ty + TH * i, h - 1), pitch4) + min((uint32_t)xlo + tx + 16 * j, w - 1) * 4u,
+                rf, __umul24(min((uint32_t)ylo + ty + TH * i, ylast), pitch4) + min((uint32_t)xlo + tx + 16 * j, xlast) * 4u,
                 0, 0);
     // the tap weights and first taps of the block's 16 columns (entries 0 .. 16 KMX - 1) and TH rows (the rest):
     // interp_aa.wgsl's per-tap weight, which depends on the output column (row) alone, once per block
@@ -2538,6 +2560,20 @@ extern "C" int fhc_avgpool(const fhc_tensor* x, const fhc_tensor* out, uint32_t 
     });
 }
 
+namespace {
+using AaKernel = decltype(&interp_aa_lds_kernel<8, 8, 72, 72, true, true, 3>);
+// interp_aa_lds_kernel of K taps an axis that reach R pixels, for c channels (1 to 4)
+template <int K, int R>
+AaKernel aa_lds_form(bool v4, uint32_t c) {
+    static const AaKernel forms[2][4] = {
+        {interp_aa_lds_kernel<K, K, R, R, false, false, 1>, interp_aa_lds_kernel<K, K, R, R, false, false, 2>,
+         interp_aa_lds_kernel<K, K, R, R, false, false, 3>, interp_aa_lds_kernel<K, K, R, R, false, false, 4>},
+        {interp_aa_lds_kernel<K, K, R, R, false, true, 1>, interp_aa_lds_kernel<K, K, R, R, false, true, 2>,
+         interp_aa_lds_kernel<K, K, R, R, false, true, 3>, interp_aa_lds_kernel<K, K, R, R, false, true, 4>}};
+    return forms[v4 ? 1 : 0][c - 1];
+}
+}  // namespace
+
 extern "C" int fhc_interpolate(const fhc_tensor* x, const fhc_tensor* out, uint32_t n, uint32_t c, uint32_t ih,
                                uint32_t iw, uint32_t oh, uint32_t ow, int antialias, void* stream) {
     return guard(-3, [&]() -> int {
@@ -2554,23 +2590,15 @@ extern "C" int fhc_interpolate(const fhc_tensor* x, const fhc_tensor* out, uint3
                 const uint32_t tx = (ow + kAaT - 1) / kAaT, ty = (oh + kAaT - 1) / kAaT;
                 if ((uint64_t)n * tx * ty >= kMaxItems) return fail(-1, "interpolate: too many tiles");
                 const bool v4 = vec4(4, {x});
-                // the smallest form whose taps and reach serve the scale (8 taps reach at most 69 pixels); three channels
-                // or fewer of 8-byte pixels are summed apart from four
-                const int f = !v4 ? 0 : c == 4 ? 1 : 2;
-                using KL = decltype(&interp_aa_lds_kernel<8, 8, 72, 72, false, true>);
-                static const KL kls[4][3] = {
-                    {interp_aa_lds_kernel<4, 4, 36, 36, false, false>, interp_aa_lds_kernel<4, 4, 36, 36, false, true>,
-                     interp_aa_lds_kernel<4, 4, 36, 36, false, true, 3>},
-                    {interp_aa_lds_kernel<5, 5, 44, 44, false, false>, interp_aa_lds_kernel<5, 5, 44, 44, false, true>,
-                     interp_aa_lds_kernel<5, 5, 44, 44, false, true, 3>},
-                    {interp_aa_lds_kernel<6, 6, 56, 56, false, false>, interp_aa_lds_kernel<6, 6, 56, 56, false, true>,
-                     interp_aa_lds_kernel<6, 6, 56, 56, false, true, 3>},
-                    {interp_aa_lds_kernel<8, 8, 72, 72, false, false>, interp_aa_lds_kernel<8, 8, 72, 72, false, true>,
-                     interp_aa_lds_kernel<8, 8, 72, 72, false, true, 3>}};
+                // the smallest form whose taps and reach serve the scale (8 taps reach at most 69 pixels), for 8-byte
+                // pixels or any, by the channels
                 auto serves = [&](uint32_t k, uint32_t r) {
                     return taps <= k && aa_tile_reach(ih, oh, kAaT, k) <= r && aa_tile_reach(iw, ow, kAaT, k) <= r;
                 };
-                const KL kl = kls[serves(4, 36) ? 0 : serves(5, 44) ? 1 : serves(6, 56) ? 2 : 3][f];
+                const AaKernel kl = serves(4, 36)   ? aa_lds_form<4, 36>(v4, c)
+                                    : serves(5, 44) ? aa_lds_form<5, 44>(v4, c)
+                                    : serves(6, 56) ? aa_lds_form<6, 56>(v4, c)
+                                                    : aa_lds_form<8, 72>(v4, c);
                 hipLaunchKernelGGL(kl, dim3(n * tx * ty), dim3(kThreads), 0, (hipStream_t)stream, in(x), outv(out),
                                    ih, iw, oh, ow, c, tx, ty, PyrOut{});
                 const hipError_t e = hipGetLastError();
@@ -2775,8 +2803,8 @@ extern "C" int fhc_pair_input_n(const fhc_tensor* ab, const fhc_tensor* q, const
         const uint32_t tx = (ow + kAaT - 1) / kAaT, ty = (oh + kAaT - 1) / kAaT;
         const bool v4 = vec4(4, {ab});
         const bool small = taps <= 4 && std::max(aa_tile_reach(ih, oh, kAaT, 4), aa_tile_reach(iw, ow, kAaT, 4)) <= 36;
-        auto kl = small ? (v4 ? interp_aa_lds_kernel<4, 4, 36, 36, true, true> : interp_aa_lds_kernel<4, 4, 36, 36, true, false>)
-                        : (v4 ? interp_aa_lds_kernel<8, 8, 72, 72, true, true> : interp_aa_lds_kernel<8, 8, 72, 72, true, false>);
+        auto kl = small ? (v4 ? interp_aa_lds_kernel<4, 4, 36, 36, true, true, 3> : interp_aa_lds_kernel<4, 4, 36, 36, true, false, 3>)
+                        : (v4 ? interp_aa_lds_kernel<8, 8, 72, 72, true, true, 3> : interp_aa_lds_kernel<8, 8, 72, 72, true, false, 3>);
         if ((uint64_t)2 * pairs * tx * ty >= kMaxItems / kThreads) return fail(-1, "pair_input: too many tiles");
         hipLaunchKernelGGL(kl, dim3(2 * pairs * tx * ty), dim3(kThreads), 0, (hipStream_t)stream, in(ab), outv(q), ih,
                            iw, oh, ow, 3u, tx, ty, PyrOut{outv(i8), outv(i16), outv(l16)});
@@ -2917,13 +2945,15 @@ extern "C" int fhc_rgba_resize(const void* rgba, uint32_t n, uint32_t w, uint32_
             return fail(-1, "rgba_resize: frames of pitch %u and %u rows are too large", pitch, h);
         const uint32_t kx = aa_taps(wp, ow), ky = aa_taps(hp, oh);
         // by the taps an axis and the pixels a tile's lanes reach: 1080p to 864 x 480 5 x 5 taps and 48 x 48 pixels, 1440p
-        // 6 x 6 and 56 x 56, 2160p 9 x 10 and 80 x 80 (16 rows of outputs 245 us for sixteen frames, 8 rows 270)
+        // 6 x 6 and 56 x 56 (48 x 48 up to a scale of 2.7: nine loads a lane for sixteen, nine 2044 x 3557 frames to
+        // 1408 x 800 151 -> 131 us), 2160p 9 x 10 and 80 x 80 (16 rows of outputs 245 us for sixteen frames, 8 rows 270)
         using K = decltype(&rgba_resize_kernel<5, 5, 16, 48, 48>);
         struct Form {
             uint32_t kx, ky, th, px, py;
             K k;
         };
         static const Form forms[] = {{5, 5, 16, 48, 48, rgba_resize_kernel<5, 5, 16, 48, 48>},
+                                     {6, 6, 16, 48, 48, rgba_resize_kernel<6, 6, 16, 48, 48>},
                                      {6, 6, 16, 56, 56, rgba_resize_kernel<6, 6, 16, 56, 56>},
                                      {8, 8, 16, 72, 72, rgba_resize_kernel<8, 8, 16, 72, 72>},
                                      {9, 10, 16, 80, 80, rgba_resize_kernel<9, 10, 16, 80, 80>},

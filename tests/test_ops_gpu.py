@@ -346,10 +346,12 @@ def test_rgba_in_and_out_match_oracle(n, h, w, hp, wp, cs, c0):
     torch.cuda.synchronize()
 
 
-# (image, input and output size, channels, channel stride, first channel): the forms of 4, 5, 6 and 8 taps, 3 channels and
-# 4, 8-byte pixels and not, tiles past the output's edge
+# (image, input and output size, channels, channel stride, first channel): the forms of 4, 5, 6 and 8 taps, 1 to 4
+# channels, 8-byte pixels and not, tiles past the output's edge
 @pytest.mark.parametrize("case", [(2, 60, 90, 40, 64, 3, 4, 0), (1, 97, 130, 41, 52, 3, 4, 0), (1, 88, 91, 33, 37, 4, 4, 0),
-                                  (2, 70, 67, 25, 24, 3, 5, 1), (1, 130, 101, 36, 27, 4, 8, 4), (1, 120, 136, 30, 34, 2, 4, 0)])
+                                  (2, 70, 67, 25, 24, 3, 5, 1), (1, 130, 101, 36, 27, 4, 8, 4), (1, 120, 136, 30, 34, 2, 4, 0),
+                                  (3, 70, 67, 25, 24, 1, 5, 2), (2, 60, 90, 40, 64, 1, 4, 0), (1, 101, 90, 37, 33, 2, 3, 1),
+                                  (1, 88, 91, 33, 37, 4, 5, 1)])
 def test_antialiased_resize_skips_what_lies_outside_a_window(case):
     """The antialiased resize of pictures with infinities and NaNs strewn in: an output whose window holds none equals
     the oracle's bit for bit, however close they lie; one whose window does is the oracle's infinity or NaN."""
@@ -367,12 +369,12 @@ def test_antialiased_resize_skips_what_lies_outside_a_window(case):
     assert np.array_equal(np.where(np.isnan(got), 0, got), np.where(np.isnan(want), 0, want))
 
 
-# the shapes reach each kernel form (taps, pixels a tile reaches): 5 x 5 and 48 at 1080p, 6 x 6 and 64, 8 x 8 and 80,
-# 9 x 10 and 80 at 2160p, 10 x 10 and 96 at 4096 x 2160
+# the shapes reach each kernel form (taps, pixels a tile reaches): 5 x 5 and 48 at 1080p, 6 x 6 and 48, 6 x 6 and 56 at
+# 1440p, 8 x 8 and 72, 9 x 10 and 80 at 2160p, 10 x 10 and 86 x 48 (8 rows of outputs) at 4096 x 2160
 @pytest.mark.parametrize("h,w,oh,ow", [(1080, 1920, 480, 864), (150, 300, 64, 128), (61, 97, 30, 40),
                                        (60, 30, 40, 8), (60, 30, 40, 11), (60, 90, 40, 32), (2160, 3840, 480, 864),
                                        (2160, 4096, 480, 864), (1440, 2560, 480, 864),
-                                       (96, 128, 24, 32), (95, 161, 26, 60)])
+                                       (96, 128, 24, 32), (95, 161, 26, 60), (156, 188, 60, 72)])
 def test_rgba_resize_equals_rgba_in_then_the_antialiased_resize(h, w, oh, ow):
     """The fused frame input against the oracle's rgba_in at the padded size then its antialiased interpolate:
     bit-exact (the same f16 inputs, f32 operations in the same order, one rounding)."""
