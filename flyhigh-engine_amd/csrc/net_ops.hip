@@ -2129,27 +2129,35 @@ __device__ __forceinline__ void box_sum4(uint32_t r, float (&acc)[4], Get get) {
 }
 
 // box_h then box_v of radius r (gm_box.wgsl:8-25) on map channel blockIdx.z % 5 of src ([5][hc][wc]) into the same
-// channel of dst, for the block's 32 x 32 tile of cells, pair blockIdx.z / 5. The window of clamped rows and columns
-// the tile's taps reach ((32 + 2r) x (32 + 2r) cells, the width rounded up to 4) goes into LDS by DMA; box_h runs on
-// every window row (a window row is a clamped map row, so its sums are the map's own), box_v on the tile, each sum over
-// its taps in order. Bound by its adds and LDS reads: a lane forms four neighbouring sums from one pass over their
-// 2r + 4 values (a sum's taps were read one by one), and the tile's halo rows are shared by 32 output rows (by 16): at
-// 544 x 960 cells with r = 20 56 -> 30 us, 8 pairs of 240 x 432 with r = 5 22 -> 18.7 us.
-constexpr uint32_t kBoxW = 32, kBoxH = 32, kBoxPitch = 40;  // the tile's columns; hs's row pitch (a wave's two row groups differ
-                                                // by half the LDS banks)
-inline uint32_t box_lds_floats(uint32_t r) {
-    const uint32_t w = (kBoxW + 2 * r + 3) & ~3u, h = kBoxH + 2 * r;
-    return (w * h + kThreads - 1) / kThreads * kThreads + h * kBoxPitch;
-}
+// channel of dst, for the block's T x T tile of cells (32 or 16). The window of clamped rows and columns the tile's taps
+// reach ((T + 2r) x (T + 2r) cells, the width rounded up to 4) goes into LDS by DMA; box_h runs on every window row (a
+// window row is a clamped map row, so its sums are the map's own), box_v on the tile, each sum over its taps in order.
+// Bound by its adds and LDS reads: a lane forms four neighbouring sums from one pass over their 2r + 4 values (a sum's
+// taps were read one by one), and the tile's halo rows are shared by 32 output rows: at 544 x 960 cells with r = 20
+// 56 -> 30 us, 8 pairs of 240 x 432 with r = 5 22 -> 18.7 us. Below two tiles of 32 a CU the launch is one block's
+// latency, a third as much work in tiles of 16 (the whole repair at 64 x 88 cells 36.8 us in tiles of 32, 33.4 in tiles of
+// 16, at 192 x 320 40.5 and 39.6, at 240 x 432 38.1 and 38.5)
+constexpr uint32_t kBoxTiles = 512;
+template <uint32_t T>
+struct BoxGeom {
+    // hs's row pitch: the wave's groups of four rows (two at 32 columns, four at 16) part the LDS banks
+    static constexpr uint32_t kPitch = T == 32 ? 40 : 20;
+    static uint32_t lds_floats(uint32_t r) {
+        const uint32_t w = (T + 2 * r + 3) & ~3u, h = T + 2 * r;
+        return (w * h + kThreads - 1) / kThreads * kThreads + h * kPitch;
+    }
+};
+template <uint32_t T>
 __global__ __launch_bounds__(kThreads) void gm_box_kernel(const float* src, float* dst, uint32_t hc, uint32_t wc,
                                                           uint32_t r, size_t wsf) {
+    constexpr uint32_t PITCH = BoxGeom<T>::kPitch;
     extern __shared__ __align__(16) float glds[];
-    const uint32_t t = threadIdx.x, x0 = blockIdx.x * kBoxW, y0 = blockIdx.y * kBoxH, ch = blockIdx.z % 5;
+    const uint32_t t = threadIdx.x, x0 = blockIdx.x * T, y0 = blockIdx.y * T, ch = blockIdx.z % 5;
     src += (size_t)(blockIdx.z / 5) * wsf, dst += (size_t)(blockIdx.z / 5) * wsf;
-    const uint32_t w = (kBoxW + 2 * r + 3) & ~3u, h = kBoxH + 2 * r, cells = w * h;
+    const uint32_t w = (T + 2 * r + 3) & ~3u, h = T + 2 * r, cells = w * h;
     const uint32_t rounds = (cells + kThreads - 1) / kThreads;
     float* win = glds;                      // [h][w], whole rounds of a cell a lane
-    float* hs = glds + rounds * kThreads;   // [h][kBoxPitch]
+    float* hs = glds + rounds * kThreads;   // [h][PITCH]
     const size_t n = (size_t)hc * wc;
     const auto plane = buf_rsrc(src + ch * n, (uint32_t)(n * 4));
     {
@@ -2166,25 +2174,26 @@ __global__ __launch_bounds__(kThreads) void gm_box_kernel(const float* src, floa
     __builtin_amdgcn_s_waitcnt(0);  // this wave's DMA has landed
     __syncthreads();
     const float den = (float)(2 * r + 1);
-    for (uint32_t e = t; e < h * (kBoxW / 4); e += kThreads) {
-        const uint32_t row = e / (kBoxW / 4), q = e % (kBoxW / 4);
+    for (uint32_t e = t; e < h * (T / 4); e += kThreads) {
+        const uint32_t row = e / (T / 4), q = e % (T / 4);
         const float4* p = reinterpret_cast<const float4*>(win + row * w) + q;
         float acc[4];
         box_sum4(r, acc, [&](int b, float (&v)[4]) {
             const float4 u = p[b];
             v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
         });
-        *reinterpret_cast<float4*>(hs + row * kBoxPitch + 4 * q) =
+        *reinterpret_cast<float4*>(hs + row * PITCH + 4 * q) =
             float4{acc[0] / den, acc[1] / den, acc[2] / den, acc[3] / den};
     }
     __syncthreads();
-    const uint32_t col = t % kBoxW, q = t / kBoxW;  // kThreads / kBoxW = kBoxH / 4 groups of four rows
-    const float* p = hs + 4 * q * kBoxPitch + col;
+    const uint32_t col = t % T, q = t / T;  // T / 4 groups of four rows
+    if (T / 4 * T < kThreads && q >= T / 4) return;
+    const float* p = hs + 4 * q * PITCH + col;
     float acc[4];
     const uint32_t top = h - 1 - 4 * q;  // the last group may reach past the window: values no sum holds
     box_sum4(r, acc, [&](int b, float (&v)[4]) {
 #pragma unroll
-        for (uint32_t m = 0; m < 4; m++) v[m] = p[min(4u * (uint32_t)b + m, top) * kBoxPitch];
+        for (uint32_t m = 0; m < 4; m++) v[m] = p[min(4u * (uint32_t)b + m, top) * PITCH];
     });
     if (x0 + col < wc) {
 #pragma unroll
@@ -3131,8 +3140,13 @@ int fhc::gmhs_run(const fhc_tensor* a, const fhc_tensor* b, uint32_t h, uint32_t
                            h, w, in(flow), h8, w8, part[1], coef, raw, p.hc, p.wc, wsf);
         // the texture window over the 5 maps (raw -> maps), then the decision window at the cells the select reads
         // (its rows at their columns, its columns at their rows) and the select (maps -> dec, flow)
-        hipLaunchKernelGGL(gm_box_kernel, dim3((p.wc + kBoxW - 1) / kBoxW, (p.hc + kBoxH - 1) / kBoxH, 5 * pairs),
-                           dim3(kThreads), box_lds_floats(p.r_blk) * sizeof(float), st, raw, maps, p.hc, p.wc, p.r_blk, wsf);
+        const uint32_t bx = (p.wc + 31) / 32, by = (p.hc + 31) / 32;
+        if (bx * by * 5 * pairs < kBoxTiles)
+            hipLaunchKernelGGL(gm_box_kernel<16>, dim3((p.wc + 15) / 16, (p.hc + 15) / 16, 5 * pairs), dim3(kThreads),
+                               BoxGeom<16>::lds_floats(p.r_blk) * sizeof(float), st, raw, maps, p.hc, p.wc, p.r_blk, wsf);
+        else
+            hipLaunchKernelGGL(gm_box_kernel<32>, dim3(bx, by, 5 * pairs), dim3(kThreads),
+                               BoxGeom<32>::lds_floats(p.r_blk) * sizeof(float), st, raw, maps, p.hc, p.wc, p.r_blk, wsf);
         const bool wide = 2 * p.r_dwin + 1 > 33;
         const uint32_t nh = 3 * p.hc * w8, ne = h8 * w8;
         // the columns of 64 lanes lie at most floor(63 wc / w8) + 1 cells apart

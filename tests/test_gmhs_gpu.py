@@ -88,6 +88,8 @@ CASES = [  # network h, w, padded frame width, flow cstride, level
     (70, 90, 128, 6, 2),      # level 2 (no jump gate), odd grids
     (770, 1106, 2208, 8, 1),  # many texture-window tiles, ragged
     (64, 128, 2048, 8, 1),    # the smallest windows (radius 1)
+    (480, 864, 864, 4, 1),    # the largest windows in the larger texture-window tiles
+    (66, 70, 96, 6, 1),       # the smaller tiles, one cell past them
 ]
 
 
