@@ -263,6 +263,33 @@ def test_network_ops_reject_bad_views_before_any_launch():
         ("fhc_render_rgba_n", (0x1000, 2, 3, 64, 32, 64, 64 * 32, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8, 16,
                                ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 0, 0x3000, 64, 100, None),
          "frame stride"),
+        # the frame render with pictures: the exact order only, a view of three channels, the frame count and strides
+        ("fhc_render_rgba_pic_n", (0x1000, 1, 2, 64, 32, 64, 64 * 32, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8, 16,
+                                   ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 0, 0x3000, 64, 64 * 32, _tv(), None),
+         "exact f32 order"),
+        ("fhc_render_rgba_pic_n", (0x1000, 1, 2, 64, 32, 64, 64 * 32, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8, 16,
+                                   ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 4, 0x3000, 64, 64 * 32, _tv(cs=2), None),
+         "render_rgba pic"),
+        ("fhc_render_rgba_pic_n", (0x1000, 1, 2, 64, 32, 64, 64 * 32, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8, 16,
+                                   ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 4, 0x3000, 64, 64 * 32, _tv(p=0), None),
+         "null pointer"),
+        ("fhc_render_rgba_pic_n", (0x1000, 300, 300, 64, 32, 64, 64 * 32, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8,
+                                   16, ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 4, 0x3000, 64, 64 * 32, _tv(), None),
+         "launch limit"),
+        ("fhc_render_rgba_pic_n", (0x1000, 1, 2, 64, 32, 64, 100, 32, 64, _tv(cs=8), _tv(cs=8, c0=4), _tv(), 8, 16,
+                                   ctypes.c_float(1.0), ctypes.c_float(1.0), 1, 4, 0x3000, 64, 64 * 32, _tv(), None),
+         "frame stride"),
+        # several phases' FiLM modulation: at most 8, every phase's vectors present, the views and the item count
+        ("fhc_film_modulate_n", (_tv(), (ctypes.c_void_p * 9)(*[0x1000] * 9), 9, _tv(), 1, 4, 4, 4, None), "9 phases"),
+        ("fhc_film_modulate_n", (_tv(), None, 2, _tv(), 1, 4, 4, 4, None), "null g"),
+        ("fhc_film_modulate_n", (_tv(), (ctypes.c_void_p * 2)(0x1000, None), 2, _tv(), 1, 4, 4, 4, None),
+         "null g of phase 1"),
+        ("fhc_film_modulate_n", (_tv(scale=0.5), (ctypes.c_void_p * 2)(0x1000, 0x1000), 2, _tv(), 1, 4, 4, 4, None),
+         "unscaled"),
+        ("fhc_film_modulate_n", (_tv(), (ctypes.c_void_p * 2)(0x1000, 0x1000), 2, _tv(cs=3), 1, 4, 4, 4, None),
+         "film_modulate out"),
+        ("fhc_film_modulate_n", (_tv(), (ctypes.c_void_p * 8)(*[0x1000] * 8), 8, _tv(), 64, 4096, 1024, 4, None),
+         "too many work items"),
         # the convex upsample with the refine input: its phases, image count and every view before any launch
         ("fhc_mid_input_n", (_tv(cs=40), _tv(cs=8), _tv(cs=8), (ctypes.c_float * 9)(*[0.5] * 9), 9, _tv(cs=8),
                              _tv(cs=8), _tv(cs=16), 1, 4, 4, ctypes.c_float(0.25), ctypes.c_float(0.05), None),
