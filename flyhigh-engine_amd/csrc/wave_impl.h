@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void conv_wave(ConvKArgs a) {
 // Whether a launch can take the wave kernel: whole 16-byte input groups at 16-byte aligned addresses, 8-byte output
 // stores, no residual, and 32-bit buffer offsets.
 inline bool wave_path_ok(const ConvKArgs& a) {
-    return !a.residual && a.cin % 8 == 0 && buffer_path_ok(a);
+    return !a.residual && a.xvec && a.cin % 8 == 0 && buffer_path_ok(a);
 }
 
 template <int KS, int S, int CIN32, int FM, int NA>
