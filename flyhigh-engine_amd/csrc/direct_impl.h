@@ -793,7 +793,11 @@ inline bool buffer_path_ok(const ConvKArgs& a) {
 template <int KS, int S, int CIN32, int FM, int WM, int WN, int NA, int WK, bool PERSIST>
 hipError_t launch_direct(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s) {
     (void)lds;
-    const dim3 block(64 * WM * WN * WK);
+    // one tile a workgroup: the persistent 8-row wave tiles on two wave rows of 4 (the same tiles and bits; 14 -> 52 at 7 x
+    // 309 x 507 off an aligned pointer 163 us on one wave row of 8, the weights' wait and the staging of four waves)
+    constexpr bool TALL = PERSIST && S == 1 && FM == 8 && WM == 1;
+    constexpr int F1 = TALL ? 4 : FM, W1 = TALL ? 2 : WM;
+    dim3 block(64 * WM * WN * WK);
     if constexpr (PERSIST) {
         if (buffer_path_ok(a)) {
             if (a.residual)
@@ -803,14 +807,15 @@ hipError_t launch_direct(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t 
             return hipGetLastError();
         }
         grid.x = (unsigned)(a.n * a.tiles_y * a.tiles_x);
+        block.x = 64 * W1 * WN * WK;
     }
     if constexpr (NA == 1) {
         if (a.xvec)
-            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kWhole>), grid, block, 0, s, a);
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, F1, W1, WN, WK, kWhole>), grid, block, 0, s, a);
         else if (CIN32 > 32 || a.cin >= 8)
-            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, kAny>), grid, block, 0, s, a);
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, F1, W1, WN, WK, kAny>), grid, block, 0, s, a);
         else
-            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, FM, WM, WN, WK, CIN32 == 32 ? kFew : kAny>), grid, block, 0, s, a);
+            hipLaunchKernelGGL((conv_tile<KS, S, CIN32, F1, W1, WN, WK, CIN32 == 32 ? kFew : kAny>), grid, block, 0, s, a);
     } else {
         if (a.xvec)
             hipLaunchKernelGGL((conv_direct<KS, S, CIN32, FM, WM, WN, NA, WK, false, 1>), grid, block, 0, s, a);

@@ -248,9 +248,10 @@ inline bool gemm_path_ok(const ConvKArgs& a) {
     return (a.xvec || pairs_ok(a)) && (uint64_t)a.n * a.h * a.w * a.xcs * 2 < (1ull << 31);
 }
 
-// The chunked kernel's configuration that stands in on views the DMA path cannot read: 8 rows x 16 channels, which
-// divides every np; same packed weights (chunks of cc = CK channels), same split.
-constexpr int kGemmFallbackCfg = 3;
+// The chunked kernel's configuration that stands in on views the DMA path cannot read: 8 rows by the widest channel tile
+// that divides the kernel's own (each tile reads the input again: 256 -> 60 at 86 x 125, a pointer at 2 bytes, 35 us in
+// tiles of 16); same packed weights (chunks of cc = CK channels), same split, the same bits in every width.
+constexpr int gemm_fallback_cfg(int bn) { return bn % 64 == 0 ? 1 : bn % 48 == 0 ? 9 : bn % 32 == 0 ? 2 : 3; }
 
 template <int S, int CK, int FM, int NA, int WM, int WN, int ST>
 hipError_t launch_gemm(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s) {
@@ -259,7 +260,9 @@ hipError_t launch_gemm(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s)
         hipLaunchKernelGGL((conv_gemm<S, CK, FM, NA, WM, WN, ST>), grid, dim3(64 * WM * WN), 0, s, a);
         return hipGetLastError();
     }
-    constexpr TileCfg t = kTileCfgs[kGemmFallbackCfg];
+    constexpr int fallback = gemm_fallback_cfg(16 * NA * WN);
+    constexpr TileCfg t = kTileCfgs[fallback];
+    static_assert(t.wk == 1 && (16 * NA * WN) % (t.fn * 16 * t.wn) == 0, "whole tiles of the packed weights");
     constexpr int TH = t.fm * t.wm, BN = t.fn * 16 * t.wn;
     ConvKArgs b = a;
     b.tiles_y = (a.hout + TH - 1) / TH;
@@ -267,7 +270,7 @@ hipError_t launch_gemm(const ConvKArgs& a, dim3 grid, size_t lds, hipStream_t s)
     const size_t ih = (size_t)(TH - 1) * S + 3, iw = (size_t)15 * S + 3;
     const size_t flds = (((size_t)b.tapgroups * 4 + 15) & ~(size_t)15) + ih * iw * (size_t)(b.cc + 8) * 2;
     const dim3 fgrid((unsigned)((size_t)b.n * b.tiles_y * b.tiles_x * b.ntn), grid.z, 1);
-    return conv_launcher(3, S, kGemmFallbackCfg)(b, fgrid, flds, s);
+    return conv_launcher(3, S, fallback)(b, fgrid, flds, s);
 }
 
 template <int S, int CK, int FM, int NA, int WM, int WN, int ST>

@@ -1475,7 +1475,8 @@ __device__ __forceinline__ uint32_t byte_of(uint16_t hv) {
     return (uint32_t)(fminf(fmaxf(h2f(hv), 0.0f), 1.0f) * 255.0f + 0.5f);
 }
 
-// byte_of for a value already clamped to [0, 1]: the product and the sum are exact, so one FMA forms them
+// byte_of for a value already clamped to [0, 1]: the product (11 bits by 8) is exact in f32, so one FMA rounds the sum as
+// the product and the sum by themselves do
 __device__ __forceinline__ uint32_t byte_in01(uint16_t hv) {
     return (uint32_t)__builtin_fmaf(h2f(hv), 255.0f, 0.5f);
 }

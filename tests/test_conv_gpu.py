@@ -689,3 +689,33 @@ def test_fused_pairs_take_the_grid_that_their_views_allow(n, h, w, c, stride, xc
         torch.cuda.synchronize()
         outs.append(y[..., :c[2]].contiguous().view(torch.int16).cpu().numpy())
     assert np.array_equal(*outs)
+
+
+# tensors whose pointers are off the alignment that a plan's own loop needs: every resident-grid and deep-layer variant's
+# stand-in (ragged tiles, several channel tiles with a partial last one, a residual), input or output at 2 bytes
+@pytest.mark.parametrize("cin,cout,stride", [(24, 84, 1), (48, 68, 1), (96, 100, 1), (128, 52, 1), (30, 68, 2), (64, 36, 2)])
+@pytest.mark.parametrize("xoff,yoff", [(1, 0), (0, 1)])
+def test_pointers_off_alignment_run_the_stand_in(cin, cout, stride, xoff, yoff):
+    import torch
+    c = Case(1, 27, 37, cin, cout, stride=stride, act=1, residual=True, xv=((cin + 7) // 8 * 8, 0), seed=cin)
+    want = c.run_oracle(threads=8)
+    dev = torch.device("cuda", 0)
+    codes = [k for k in fhconv.variant_list(c.fhc_desc())
+             if fhconv.variant_name(k).startswith("gemm") or fhconv.variant_name(k).endswith("/p")]
+    assert codes
+
+    def at(a, off):
+        b = torch.zeros(a.size + 8, dtype=torch.int16, device=dev)
+        b[off:off + a.size] = torch.from_numpy(a.ravel().view(np.int16)).to(dev)
+        return b[off:off + a.size]
+
+    r = at(c.res, 0)
+    for code in codes:
+        say("off", cin, cout, stride, xoff, yoff, fhconv.variant_name(code))
+        plan = fhconv.ConvPlan(c.fhc_desc(code), c.wt, c.bias, c.slope)
+        ws = torch.empty(plan.workspace_bytes // 4 + 4, dtype=torch.float32, device=dev) if plan.workspace_bytes else None
+        x, y = at(c.x, xoff), at(c.y0, yoff)
+        plan.run(x, y, r, ws)
+        torch.cuda.synchronize()
+        ok, md, mref = parity(y.cpu().numpy().view(np.uint16).reshape(c.y0.shape), want)
+        assert ok, (fhconv.variant_name(code), md, mref)
