@@ -1171,15 +1171,17 @@ extern "C" int fhc_conv_pair_plan_create(const fhc_conv_desc* desc_a, const uint
         auto select = [&](int cp) {
             auto serves = [&](const PairCfg& c) { return serves_cp(c, cp); };
             // the resident grids measured fastest over batches 1-24 of the network's pairs (the same bits in every
-            // loop), from the tiles where they pass the one-tile kernel. Other views run one tile a workgroup, in the
-            // split of the choice below: dense 3 -> 36 -> 36 at 3 x 520 x 637 on the two wave rows 103 us against 68
-            if (buffers && !loop_req && !th_req && !wm_req) {
+            // loop), from the tiles where they pass the one-tile kernel. Views off the loop run its one-tile form: over 32
+            // channels that is the faster one too (24 -> 24 -> 3 at 24 x 120 x 216, whose 3 channels no loop stores,
+            // 42.7 us against 45.5; dense 14 -> 24 -> 24 43.9 against 59.2), on the two others not (dense 3 -> 36 -> 36 at
+            // 3 x 520 x 637 103 us against 68)
+            if (!loop_req && !th_req && !wm_req) {
                 int th = 0, wm = 0, persist = 0;
                 if (A.stride == 1 && ca32 == 32 && cb32 == 32 && tiles_at(8) >= 1024)
                     th = 8, wm = 2, persist = 1;  // 14 -> 24 -> 24 at 622,080 px: 37.9 us against 45.5 on separate waves
-                else if (A.stride == 1 && ca32 == 64 && cb32 == 64 && nba == 3 && nbb == 3 && tiles_at(4) >= 600)
+                else if (buffers && A.stride == 1 && ca32 == 64 && cb32 == 64 && nba == 3 && nbb == 3 && tiles_at(4) >= 600)
                     th = 4, wm = 1, persist = 2;  // 48 -> 48 -> 48 at 51,840 px: 15.4 against 17.5 on one tile
-                else if (A.stride == 2 && ca32 == 32 && cb32 == 64 && tiles_at(4) >= 1200)
+                else if (buffers && A.stride == 2 && ca32 == 32 && cb32 == 64 && tiles_at(4) >= 1200)
                     th = 4, wm = 2, persist = 1;  // 3 -> 36 -> 36, 103,680 px out: 23.4 against 26.1 on one tile
                 for (int i = 0; i < kNumPair && th; i++)
                     if (serves(kPairCfgs[i]) && kPairCfgs[i].th == th && kPairCfgs[i].wm == wm &&

@@ -657,14 +657,14 @@ def test_sibling_convs_equal_the_two_convs_at_one_split(h, w, ca, cb):
         assert np.array_equal(y.cpu().numpy().view(np.uint16), c.run_gpu(ksplit=1)), c.cout
 
 
-# fused pairs over their resident grids' lines: the grid's loop where its buffer loop reads and writes the views, else
-# the earlier choice's (whose one-tile form such views run)
+# fused pairs over their resident grids' lines: the grid's loop where its buffer loop reads and writes the views, and for
+# pairs over 32 channels in any view, else the earlier choice's (whose one-tile form such views run)
 @pytest.mark.parametrize("n,h,w,c,stride,xcs,ycs,loop", [
     (4, 322, 454, (3, 36, 36), 2, 8, 40, "w2.k8/p"), (4, 322, 454, (3, 36, 36), 2, 3, 36, "w1.k8/ws"),
     (4, 322, 454, (3, 36, 36), 2, 8, 37, "w1.k8/ws"), (13, 146, 215, (3, 36, 36), 2, 6, 36, "w1.k8"),
     (8, 120, 216, (48, 48, 48), 1, 48, 48, "w1/ws"), (8, 120, 216, (48, 48, 48), 1, 48, 49, "t4x14.w1/ws"),
     (4, 60, 216, (48, 48, 48), 1, 52, 48, "t4x14.w1"), (9, 184, 320, (14, 24, 24), 1, 16, 24, "t8x14.w2.k16/p"),
-    (2, 184, 320, (14, 24, 24), 1, 14, 24, "w1.k16/ws")])
+    (2, 184, 320, (14, 24, 24), 1, 14, 24, "t8x14.w2.k16/p"), (9, 120, 216, (24, 24, 3), 1, 24, 8, "t8x14.w2/p")])
 def test_fused_pairs_take_the_grid_that_their_views_allow(n, h, w, c, stride, xcs, ycs, loop):
     import torch
     ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
