@@ -1217,9 +1217,10 @@ def main():
                     per_launch_bytes=dom["bytes"], per_launch_flops=dom["flops"], traffic_source=traffic_note,
                     sustained_mfma_tflops=round(mfma_rate, 1))
     if dom["label"].startswith("frame_render"):
-        # 1920 x 1088 lanes of bicubic sampling in the reference's f32 order: the SQ counters put it at ~900 VALU
-        # instructions per wave over 32,400 waves, the VALU issue rate of the chip, far below the HBM roofline
-        roofline["note"] = "VALU issue and vector memory returns: ~427 VALU instructions per wave, 32,400 waves (SQ counter pass)"
+        # 1920 x 1088 lanes of bicubic sampling in the default (fused) order: the SQ counters put it at ~427 VALU
+        # instructions per wave over 32,400 waves. Its tap rows, 16 bytes a lane at the lane's own address, keep the
+        # texture-data units about as busy; both are far from the HBM roofline
+        roofline["note"] = "texture data and VALU issue: ~427 VALU instructions per wave, 32,400 waves (SQ counter pass)"
     log("bench: dominant launch", json.dumps(roofline))
 
     cpu = None

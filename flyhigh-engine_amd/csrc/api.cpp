@@ -547,7 +547,7 @@ uint32_t measured_code(const fhc_conv_desc& d, const Geometry& g) {
 // configurations that launch one workgroup per tile, the narrowest channel tile that covers cout in one tile (else
 // the widest there is), and among the tile heights the tallest that still gives about two workgroups per CU (the
 // small layers of a frame take short tiles: more, shorter-running workgroups). Up to 128 input channels the
-// kernel-row K split is left to the autotuner.
+// kernel-row K split is left to measured_code's lines and the autotuner.
 int direct_default(const fhc_conv_desc& d, const Geometry& g) {
     const int need = (int)div_ceil(d.cout, 16);
     auto eligible = [&](int i) {
@@ -605,8 +605,8 @@ bool pairs_faster(const fhc_conv_desc& d, const Geometry& g) {
 // The planner's general choice: the deep-layer kernel for stride-1 3x3 convs over more than 64 input channels whose
 // input view has 16-byte channel groups and at least 4096 output pixels (on smaller ones its fixed cost per launch, the
 // first chunk's load and the epilogue, outweighs the direct kernel's longer chains), with `pairs` also in views of
-// channel pairs where pairs_faster. Then the direct kernel whenever a configuration serves the input channels, then the deep-layer kernel from 64
-// input channels, else the chunked kernel.
+// channel pairs where pairs_faster. Then the direct kernel whenever a configuration serves the input channels, then the
+// deep-layer kernel from 64 input channels, else the chunked kernel.
 uint32_t general_code(const fhc_conv_desc& d, const Geometry& g, bool pairs) {
     const bool deep = d.kh == 3 && d.stride == 1 && d.cin >= 64 && input_in_reach(d);
     const bool gemm_ok = deep && d.x_cstride % 8 == 0 && d.x_c0 % 8 == 0;

@@ -526,7 +526,7 @@ __device__ __forceinline__ void aa_cells(const uint2* p, uint2 (&q)[K]) {
 // channels c.
 // Bound by VALU issue, 8 instructions a tap of three channels: the KMX x KMY taps are those of the scale (5 x 5 where an
 // 8 x 8 form served everything above 4), each a fixed offset from the lane's first, and the LDS is what the taps reach: two
-// 1088 x 1920 pictures to 480 x 864 30 -> 12.5 us, two of 480 x 864 to 120 x 216 with the pyramid 5.77 -> 5.71, sixteen
+// 1088 x 1920 pictures to 480 x 864 28.4 -> 11.3 us, two of 480 x 864 to 120 x 216 with the pyramid 5.77 -> 5.71, sixteen
 // 22.2 -> 18.7. A tap outside its window has weight +0 and adds +0, as the reference's skipped tap leaves the sums, unless
 // the pixel there is infinite or NaN: a lane whose sums come out so sums again over its window's taps alone.
 template <int KMX, int KMY, int PX, int PY, bool PYR, bool V4, int NC>
@@ -1773,6 +1773,8 @@ __device__ __forceinline__ void render_rgba_px(uint32_t x, uint32_t y, const flo
 // and rk = 1, so r * rk is r and mixed * (1 - stillw) + own * stillw is mixed (or +0 for a mixed of -0, which the
 // clamp and the byte conversion turn into the same byte 0): that variant leaves those terms out.
 // PIC: also the f16 picture (hp x wp, its padding included) into pic, image j * per + p.
+// Bound by the texture-data units: a tap row, 16 bytes a lane at the lane's own address, is 34 cache accesses a wave (24
+// frames of 3840 x 2160: the units busy 98% of 2,350 us, VALU issue 82%, LDS 78%; one of 1920 x 1080 31 us).
 template <bool CUBIC, bool QV, bool FL, bool FMA, bool PIC = false>
 // blockIdx.z: generated frame z of `phases` per pair, pair-major (pair p = z / phases, phase j): its frames at
 // p * pstride words past fa and fb, its maps image j * per + p of fl, vis and rt, its output frame j * per + p,
@@ -1887,7 +1889,8 @@ __device__ __forceinline__ uint2 bgr_cell(uint32_t v) {
 // outputs' windows, each converted once, as f16 cells of 8 bytes; past the windows' union lie further (clamped) frame
 // pixels, so a lane's KMX x KMY cells from its first tap on always hold values in [0, 1], and a tap outside its window
 // (weight +0) adds +0, leaving the sums as the reference's skipped tap leaves them. Bound by VALU issue: 8 instructions
-// a tap. Every tap is therefore a fixed offset from the lane's first (no address arithmetic), the taps of the axes are counted apart and a last row that no lane of the wave uses is skipped.
+// a tap. Every tap is therefore a fixed offset from the lane's first (no address arithmetic), the taps of the axes are
+// counted apart and a last row that no lane of the wave uses is skipped.
 // Sixteen 2160p frames (9 x 10 taps) to 864 x 480 316 -> 222 us, eight 1440p frames (6 x 6) 78 -> 46, two 1080p frames
 // (5 x 5, bound by the latency of staging, then summing) 12.4 -> 12.0.
 template <int KMX, int KMY, int TH, int PX, int PY>
