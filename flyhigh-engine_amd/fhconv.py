@@ -282,8 +282,8 @@ class ConvPairPlan(ConvPlan):
 
 class ConvSiblingPlan(ConvPlan):
     """Two convs A and B of one input view in one launch (fhc_conv_sibling_plan_create): A's output channels, then
-    B's, each computed as its own plan at ksplit 1 computes it. run(x, y_a, res_a, y_b) takes the shared input, A's output and
-    residual and B's output."""
+    B's, each computed as its own plan at ksplit 1 computes it. run(x, y_a, res_a, y_b) takes the shared input, A's
+    output and residual and B's output."""
 
     def __init__(self, desc_a: ConvDesc, w_a, bias_a, slope_a, desc_b: ConvDesc, w_b, bias_b, slope_b):
         L = load()
